@@ -15,9 +15,13 @@
 // Work decomposition: X sweeps group problems by line length into the
 // register-blocking classes of the single-array X kernel (K cells per lane,
 // one launch per class, one wave per group of whole lines); Y sweeps use the
-// column march with a per-problem segment count S (columns split in S
-// segments held by lanes of one wave). The autotuner picks S per size class
-// by timing the candidates on the ensemble itself.
+// column march with columns cut into segments. Each fluid step has one X and
+// one Y sweep: the first goes from the pool to a second pool and the other
+// back, so neither has to leave cells for its neighbours and a problem's
+// segments fill waves of their own. Where the second pool does not fit the
+// device, the sweeps work in place (a column's segments in one wave).
+// The autotuner picks the segment counts per size class by timing the
+// candidates on the ensemble itself.
 #include <algorithm>
 #include <cstring>
 #include <vector>
@@ -33,6 +37,7 @@ namespace imogen {
 // problems' gas; dusty problems add an entry for their dust.
 struct EnsProblem {
     double *q;
+    double *q2;     // the array's image in the second pool (q when there is none)
     int64_t pitch;  // doubles between slabs
     int nx, ny;
     double hx, hy;
@@ -45,10 +50,20 @@ struct EnsProblem {
 
 struct EnsItem {
     int p;   // problem
-    int a;   // X: first line; Y: first column
+    int a;   // X: first line; Y: first column (in place) or first (segment, column) pair
     int b;   // Y: segments S
     int pad;
 };
+
+// which pool a sweep reads and writes (nothing to choose in place, q2 == q)
+struct EnsSweep {
+    const double *src;
+    double *dst;
+};
+__device__ __forceinline__ EnsSweep ens_arrays(const EnsProblem &P, int fromSecond)
+{
+    return fromSecond ? EnsSweep{P.q2, P.q} : EnsSweep{P.q, P.q2};
+}
 
 constexpr int kEnsCflBlocks = 32;  // CFL partial minima per problem
 constexpr int kEnsGhost = 4;       // ghost cells per face set by the boundary kernel
@@ -232,7 +247,7 @@ __device__ __forceinline__ HydroConsts ens_consts(double gamma)
 // output cells into fold[problem] (entries with P.fold set).
 template <int K, int LIM, bool CFL>
 __global__ __launch_bounds__(256, 2) void ens_sweep_x(const EnsProblem *__restrict__ probs,
-                                                   const EnsItem *__restrict__ work, int nwork,
+                                                   const EnsItem *__restrict__ work, int nwork, int fromSecond,
                                                    const double *__restrict__ lam, int rt,
                                                    double *__restrict__ dummy, unsigned long long *__restrict__ fold,
                                                    unsigned long long *__restrict__ err)
@@ -260,7 +275,8 @@ __global__ __launch_bounds__(256, 2) void ens_sweep_x(const EnsProblem *__restri
     cnt = cnt < K ? cnt : K;
     if (!laneUsed) cnt = 0;
     const int lc = line < P.ny ? line : P.ny - 1;
-    double *b = P.q + (int64_t)lc * N + x0;
+    const EnsSweep A = ens_arrays(P, fromSecond);
+    const double *b = A.src + (int64_t)lc * N + x0;
     V5 Q[K];
 #pragma unroll
     for (int k = 0; k < K; k++) Q[k] = (k < cnt) ? load_cell<Hllc, 1>(b + k, P.pitch) : V5{1.0, 1.0, 0.0, 0.0, 0.0};
@@ -272,7 +288,7 @@ __global__ __launch_bounds__(256, 2) void ens_sweep_x(const EnsProblem *__restri
     x_fluxes<Hllc, K, LIM>(hc, rt, U1, cnt, srcL, srcR, F, Fm);
     const int64_t gtid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t nthr = (int64_t)gridDim.x * blockDim.x;
-    double *dst = own ? b : dummy + gtid;
+    double *dst = own ? A.dst + (int64_t)lc * N + x0 : dummy + gtid;
     const int64_t st = own ? P.pitch : nthr;
     const bool fl = CFL && own && P.fold;
     const CflArgs ca = ens_cfl_args(P);
@@ -293,82 +309,31 @@ __global__ __launch_bounds__(256, 2) void ens_sweep_x(const EnsProblem *__restri
     if (CFL) ens_fold_wave(cmin, nan, fold + P.owner, err);
 }
 
-// X sweep of lines split into two halves, one wave per half. A wave holds its
-// half and the 4 cells beyond each end (the two stages' stencil, periodic
-// within the line, as the whole-line sweep reads them), so it forms its half's
-// outputs alone; the window's outer cells only feed discarded values. The two
-// waves of a line are in one workgroup (4 waves: 2 lines), and every load of
-// the workgroup precedes the barrier while every store follows it, so no wave
-// overwrites a cell its partner has still to read. One work item (problem,
-// line) per wave pair; lines of at most 2 (64 K - 8) cells.
+// X sweep of lines split into two halves, one wave per half (xp_body). The two
+// waves of a line are in one workgroup (4 waves: 2 lines), as the in-place form
+// needs. One work item (problem, line) per wave pair; lines of at most
+// 2 (64 K - 8) cells.
 template <int K, int LIM, bool CFL>
 __global__ __launch_bounds__(256, 2) void ens_sweep_xh(const EnsProblem *__restrict__ probs,
-                                                    const EnsItem *__restrict__ work, int nwork,
+                                                    const EnsItem *__restrict__ work, int nwork, int fromSecond,
                                                     const double *__restrict__ lam, int rt,
-                                                    double *__restrict__ dummy,
                                                     unsigned long long *__restrict__ fold,
                                                     unsigned long long *__restrict__ err)
 {
-    const int lane = threadIdx.x & 63;
     const int wib = threadIdx.x >> 6;
     int item = (int)blockIdx.x * 2 + (wib >> 1);
     const bool itemValid = item < nwork;
     item = itemValid ? item : nwork - 1;  // waves past the list still meet the barrier
-    const int part = wib & 1;
     const EnsItem it = work[item];
     const EnsProblem P = probs[it.p];
-    const HydroConsts hc = ens_consts(P.gamma);
-    const double lambda = lam[2 * it.p];
-    const int N = P.nx;
-    const int h = (N + 1) >> 1;
-    const int s0 = part ? h : 0;          // first output cell of this half
-    const int Wn = (part ? N - h : h) + 8;  // window: the half and 4 cells beyond each end
-    const int nl = (Wn + K - 1) / K;
-    const bool laneUsed = lane < nl;
-    const int srcL = laneUsed ? (lane == 0 ? nl - 1 : lane - 1) : lane;
-    const int srcR = laneUsed ? (lane == nl - 1 ? 0 : lane + 1) : lane;
-    const int w0 = lane * K;
-    int cnt = Wn - w0;
-    cnt = cnt < K ? cnt : K;
-    if (!laneUsed) cnt = 0;
-    double *row = P.q + (int64_t)it.a * N;
-    V5 Q[K];
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        int g = s0 - 4 + w0 + k;  // window cell -> line cell, periodic
-        g = (g < 0) ? g + N : g;
-        g = (g >= N) ? g - N : g;
-        g = (g < N) ? g : N - 1;
-        Q[k] = (k < cnt) ? load_cell<Hllc, 1>(row + g, P.pitch) : V5{1.0, 1.0, 0.0, 0.0, 0.0};
-    }
-    __syncthreads();
-    V5 F[K], Fm;
-    x_fluxes<Hllc, K, LIM>(hc, rt, Q, cnt, srcL, srcR, F, Fm);
-    V5 U1[K];
-#pragma unroll
-    for (int k = 0; k < K; k++) U1[k] = axpy_update(Q[k], lambda, F[k], k == 0 ? Fm : F[k > 0 ? k - 1 : 0]);
-    x_fluxes<Hllc, K, LIM>(hc, rt, U1, cnt, srcL, srcR, F, Fm);
-    const int64_t gtid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t nthr = (int64_t)gridDim.x * blockDim.x;
+    const EnsSweep A = ens_arrays(P, fromSecond);
+    const int64_t row = (int64_t)it.a * P.nx;
     const bool fl = CFL && P.fold;
-    const CflArgs ca = ens_cfl_args(P);
+    const CflFuse cf{nullptr, ens_cfl_args(P), fl ? kEnsGhost : 0, fl ? P.nx - kEnsGhost : 0, 0};
     double cmin = kEnsCflNone;
     unsigned nan = 0;
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        if (k < cnt) {
-            const int w = w0 + k;
-            const bool own = itemValid && w >= 4 && w < Wn - 4;
-            const int x = s0 + w - 4;
-            const V5 o = avg_update(add5(U1[k], Q[k]), lambda, F[k], k == 0 ? Fm : F[k > 0 ? k - 1 : 0]);
-            store_cell<Hllc, 1>(own ? row + x : dummy + gtid, own ? P.pitch : nthr, o);
-            if (fl && own && x >= kEnsGhost && x < N - kEnsGhost) {
-                const double u = cfl_of_cell<Hllc, 1>(ca, o);
-                cmin = (u < cmin) ? u : cmin;
-                nan += (u != u);
-            }
-        }
-    }
+    xp_body<Hllc, K, LIM, CFL>(A.src + row, A.dst + row, P.pitch, P.nx, wib & 1, 2, itemValid, A.src == A.dst,
+                               lam[2 * it.p], ens_consts(P.gamma), rt, cf, cmin, nan);
     if (CFL) ens_fold_wave(cmin, nan, fold + P.owner, err);
 }
 
@@ -378,10 +343,14 @@ static int64_t x_blocks(int cls, int64_t n)
     return kXClassSplit[cls] ? (n + 1) / 2 : (n + 3) / 4;
 }
 
-// Y sweep: column march, one work item (problem, first column, S) per wave
+// Y sweep: column march, one work item per wave. In place (problem, first
+// column, S): 64/S columns, their S segments side by side in the lanes.
+// Otherwise (problem, first pair, S): 64 of the problem's (segment, column)
+// pairs, numbered segment * nx + column, so all lanes but the last wave's
+// carry one (short problems leave none idle past their last column).
 template <int LIM, bool CFL>
 __global__ __launch_bounds__(256) void ens_sweep_y(const EnsProblem *__restrict__ probs,
-                                                   const EnsItem *__restrict__ work, int nwork,
+                                                   const EnsItem *__restrict__ work, int nwork, int fromSecond,
                                                    const double *__restrict__ lam, int rt,
                                                    double *__restrict__ defer, unsigned long long *__restrict__ fold,
                                                    unsigned long long *__restrict__ err)
@@ -393,21 +362,23 @@ __global__ __launch_bounds__(256) void ens_sweep_y(const EnsProblem *__restrict_
     const int lane = threadIdx.x & 63;
     const EnsItem it = work[wave];
     const EnsProblem P = probs[it.p];
+    const EnsSweep A = ens_arrays(P, fromSecond);
+    const bool inplace = A.src == A.dst;
     const HydroConsts hc = ens_consts(P.gamma);
     const double lambda = lam[2 * it.p + 1];
     const int S = it.b;
-    const int W = 64 / S;
-    const int s = lane / W;
-    const int c = lane - s * W;
-    const int x = it.a + c;
+    const int W = inplace ? 64 / S : P.nx;
+    const int id = (inplace ? 0 : it.a) + lane;
+    const int s = id / W;
+    const int x = (inplace ? it.a : 0) + id % W;
     const bool colValid = (x < P.nx) && (s < S);
     const int N = P.ny;
     const int seglen = (N + S - 1) / S;
     const int j0 = colValid ? s * seglen : 0;  // lanes of no column: zero-length segment at row 0
     int L = N - j0;
     L = L < seglen ? L : seglen;
-    if (!colValid) L = 0;
-    double *col = P.q + (colValid ? x : 0);
+    if (!colValid || L < 0) L = 0;
+    const int off = colValid ? x : 0;
     const int64_t gtid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t nthr = (int64_t)gridDim.x * blockDim.x;
     // cells [kEnsGhost, N - kEnsGhost) of the column fold their CFL limits
@@ -415,8 +386,9 @@ __global__ __launch_bounds__(256) void ens_sweep_y(const EnsProblem *__restrict_
     const CflFuse cf{nullptr, ens_cfl_args(P), fl ? kEnsGhost : 0, fl ? N - kEnsGhost : 0, 0};
     double cmin = kEnsCflNone;
     unsigned nan = 0;
-    march_body<Hllc, 2, LIM, CFL>(col, P.pitch, (int64_t)P.nx, N, seglen, j0, L, lambda, hc, rt, defer, gtid,
-                                  nthr, sring[wib], lane, cf, cmin, nan);
+    march_body<Hllc, 2, LIM, CFL>(A.src + off, A.dst + off, P.pitch, (int64_t)P.nx, N, seglen, j0, L,
+                                  inplace ? 4 : 0, lambda, hc, rt, defer, gtid, nthr, sring[wib], lane, cf, cmin,
+                                  nan);
     if (CFL) ens_fold_wave(cmin, nan, fold + P.owner, err);
 }
 
@@ -429,9 +401,11 @@ __global__ __launch_bounds__(256) void ens_sweep_y(const EnsProblem *__restrict_
 // its boundaries (flux.cu:99-107, the swept direction rotated into memory x);
 // 0: the y kernel's innermost-ghost copy (cudaStatics.cu:1461-1466), as
 // src0001.m's boundary calls on unrotated arrays
-__global__ __launch_bounds__(256) void ens_bc_const(const EnsProblem *__restrict__ probs, int dir, int d, int xrules)
+__global__ __launch_bounds__(256) void ens_bc_const(const EnsProblem *__restrict__ probs, int second, int dir, int d,
+                                                    int xrules)
 {
     const EnsProblem P = probs[blockIdx.x];
+    double *q = second ? P.q2 : P.q;
     const int nx = P.nx, ny = P.ny;
     const int N = (dir == 1) ? nx : ny;
     if (N < d + 2) return;
@@ -459,7 +433,7 @@ __global__ __launch_bounds__(256) void ens_bc_const(const EnsProblem *__restrict
                 r = together ? (r >> 1) : r;
                 const int slab = r % 5;
                 const int row = r / 5;
-                double *a = P.q + slab * P.pitch + (int64_t)row * nx;
+                double *a = q + slab * P.pitch + (int64_t)row * nx;
                 if (side == 0) a[g] = a[d];
                 else a[nx - d + g] = a[nx - d - 1];
             }
@@ -471,7 +445,7 @@ __global__ __launch_bounds__(256) void ens_bc_const(const EnsProblem *__restrict
                 const int r = t / nx;
                 const int side = together ? (r & 1) : pass;
                 const int slab = together ? (r >> 1) : r;
-                double *a = P.q + slab * P.pitch + x;
+                double *a = q + slab * P.pitch + x;
                 if (side == 0) {
                     const double f = a[(int64_t)d * nx];
                     for (int g = 0; g < d; g++) a[(int64_t)g * nx] = f;
@@ -493,9 +467,10 @@ struct EnsembleImpl {
     double gamma = 1.4, cfl = 0.4;
     int limiter = 0;
     std::vector<EnsProblem> host;
-    std::vector<int> segS;  // chosen Y segments per problem
+    std::vector<int> segS;  // Y segments per problem: the count (in place) or a factor on the base count
     std::vector<int> xcls;  // X line class per problem (x_class_of unless tuned)
-    double *pool = nullptr;
+    double *pool = nullptr, *pool2 = nullptr;  // pool2: the sweeps' second arrays (null: in place)
+    int segLen = 64;  // cells per Y segment the base counts aim at (second pool)
     EnsProblem *dprobs = nullptr;
     double *lam = nullptr, *clock = nullptr, *cflPart = nullptr;
     // folded CFL minima (one key per problem) and the entries the reduction
@@ -518,7 +493,7 @@ struct EnsembleImpl {
     int64_t cells = 0;
     // dust (imogen_ensemble_set_dust)
     int Pd = 0;
-    double *dpool = nullptr, *dtp = nullptr;
+    double *dpool = nullptr, *dpool2 = nullptr, *dtp = nullptr;
     EnsDragTable *dragTab = nullptr;
     EnsDragItem *dragItems = nullptr;
     int nDragItems = 0;
@@ -537,6 +512,40 @@ static void free_graphs(EnsembleImpl *e)
             if (e->graph[f][k]) (void)hipGraphExecDestroy(e->graph[f][k]);
             e->graph[f][k] = nullptr;
         }
+}
+
+// segments of entry k's columns: the chosen count in place, or the chosen
+// factor times the count that cuts them into about segLen cells
+static int y_segments(const EnsembleImpl *e, int k)
+{
+    const EnsProblem &P = e->host[k];
+    int S = e->segS[P.owner];
+    if (!e->pool2) return S;
+    S *= (P.ny + e->segLen - 1) / e->segLen;
+    S = std::min(S, std::max(1, P.ny / 4));
+    const int len = (P.ny + S - 1) / S;
+    return (P.ny + len - 1) / len;  // no empty segment
+}
+
+// Cells per segment of the out-of-place Y march: with w waves of L cells the
+// launch takes about (w / 1024 + 1/2) (L + 9) steps (the waves go to the SIMDs
+// longest first; the last one's steps are half hidden), a wave's steps taking
+// their issue time however many share a SIMD. 60 problems of 64..512 cells
+// (3.7 M): 339 us per launch with up to 2 segments per column in place.
+static int ens_segment_cells(const EnsembleImpl *e)
+{
+    int best = 8;
+    double bestCost = 0.0;
+    for (int L = 8; L <= 512; L += (L < 64 ? 4 : 16)) {
+        int64_t waves = 0;
+        for (const EnsProblem &P : e->host) waves += ((int64_t)P.nx * ((P.ny + L - 1) / L) + 63) / 64;
+        const double cost = std::max(1.0, waves / 1024.0 + 0.5) * (L + 9);
+        if (L == 8 || cost < bestCost) {
+            best = L;
+            bestCost = cost;
+        }
+    }
+    return best;
 }
 
 static int build_work(EnsembleImpl *e)
@@ -563,6 +572,7 @@ static int build_work(EnsembleImpl *e)
     if (IM_HIP(hipMemcpy(e->cflList, cl.data(), cl.size() * sizeof(int), hipMemcpyHostToDevice)))
         return ERROR_CUDA_BLEW_UP;
     std::vector<EnsItem> xw[kXClasses], yw;
+    e->segLen = ens_segment_cells(e);
     for (int c = 0; c < kXClasses; c++) e->xcells[c] = 0;
     for (int p = 0; p < e->NE; p++) {
         const EnsProblem &P = e->host[p];
@@ -572,9 +582,11 @@ static int build_work(EnsembleImpl *e)
         const int lpw = kXClassSplit[cls] ? 1 : 64 / nl;  // split classes: one item per line
         for (int l = 0; l < P.ny; l += lpw) xw[cls].push_back(EnsItem{p, l, 0, 0});
         e->xcells[cls] += (int64_t)P.nx * P.ny;
-        const int S = e->segS[e->host[p].owner];
-        const int W = 64 / S;
-        for (int x = 0; x < P.nx; x += W) yw.push_back(EnsItem{p, x, S, 0});
+        const int S = y_segments(e, p);
+        if (e->pool2)
+            for (int id = 0; id < P.nx * S; id += 64) yw.push_back(EnsItem{p, id, S, 0});
+        else
+            for (int x = 0; x < P.nx; x += 64 / S) yw.push_back(EnsItem{p, x, S, 0});
     }
     for (int c = 0; c < kXClasses; c++) {
         std::stable_sort(xw[c].begin(), xw[c].end(),
@@ -614,9 +626,9 @@ static int build_work(EnsembleImpl *e)
     return SUCCESSFUL;
 }
 
-static int ens_bc(EnsembleImpl *e, int dir, hipStream_t s, int xrules)
+static int ens_bc(EnsembleImpl *e, int second, int dir, hipStream_t s, int xrules)
 {
-    hipLaunchKernelGGL(ens_bc_const, dim3((unsigned)e->NE, 16), dim3(256), 0, s, e->dprobs, dir, 4, xrules);
+    hipLaunchKernelGGL(ens_bc_const, dim3((unsigned)e->NE, 16), dim3(256), 0, s, e->dprobs, second, dir, 4, xrules);
     return IM_LAUNCHED("ens_bc_const");
 }
 
@@ -630,16 +642,17 @@ static int ens_source(EnsembleImpl *e, double fraction, hipStream_t s)
                              e->dragMethod, e->queue, e->qcount, s, 2);
     if (rc) return rc;
     for (int d = 1; d <= 2; d++) {
-        rc = ens_bc(e, d, s, 0);
+        rc = ens_bc(e, 0, d, s, 0);
         if (rc) return rc;
     }
     return SUCCESSFUL;
 }
 
-// one sweep of every entry in direction dir, then that direction's boundaries;
-// CFL: the sweep folds the CFL minima of the entries that fold
+// one sweep of every entry in direction dir, from the pool to the second one
+// or (fromSecond) back, then that direction's boundaries; CFL: the sweep folds
+// the CFL minima of the entries that fold
 template <int LIM, bool CFL>
-static int ens_sweep(EnsembleImpl *e, int dir, int rt, hipStream_t s)
+static int ens_sweep(EnsembleImpl *e, int dir, int fromSecond, int rt, hipStream_t s)
 {
     unsigned long long *err = state()->err;
     if (dir == 1) {
@@ -660,10 +673,10 @@ static int ens_sweep(EnsembleImpl *e, int dir, int rt, hipStream_t s)
             const unsigned blocks = (unsigned)x_blocks(c, e->nx_work[c]);
 #define IM_EX(KK)                                                                                              \
     hipLaunchKernelGGL((ens_sweep_x<KK, LIM, CFL>), dim3(blocks), dim3(256), 0, sx, e->dprobs, e->xwork[c],     \
-                       e->nx_work[c], e->lam, rt, e->xdummy, e->fold, err)
+                       e->nx_work[c], fromSecond, e->lam, rt, e->xdummy, e->fold, err)
 #define IM_EXH(KK)                                                                                             \
     hipLaunchKernelGGL((ens_sweep_xh<KK, LIM, CFL>), dim3(blocks), dim3(256), 0, sx, e->dprobs, e->xwork[c],    \
-                       e->nx_work[c], e->lam, rt, e->xdummy, e->fold, err)
+                       e->nx_work[c], fromSecond, e->lam, rt, e->fold, err)
             if (kXClassSplit[c]) {
                 switch (kXClassK[c]) {
                 case 3: IM_EXH(3); break;
@@ -690,20 +703,20 @@ static int ens_sweep(EnsembleImpl *e, int dir, int rt, hipStream_t s)
     } else {
         const unsigned blocks = (unsigned)((e->ny_work + 3) / 4);
         hipLaunchKernelGGL((ens_sweep_y<LIM, CFL>), dim3(blocks), dim3(256), 0, s, e->dprobs, e->ywork,
-                           e->ny_work, e->lam, rt, e->ydefer, e->fold, err);
+                           e->ny_work, fromSecond, e->lam, rt, e->ydefer, e->fold, err);
         int rc = IM_LAUNCHED("ens_sweep_y");
         if (rc) return rc;
     }
-    return ens_bc(e, dir, s, 1);
+    return ens_bc(e, !fromSecond, dir, s, 1);
 }
 
 template <bool CFL>
-static int ens_sweep_lim(EnsembleImpl *e, int dir, hipStream_t s)
+static int ens_sweep_lim(EnsembleImpl *e, int dir, int fromSecond, hipStream_t s)
 {
     switch (e->limiter) {
-    case LIMITER_OSPRE: return ens_sweep<0, CFL>(e, dir, 0, s);
-    case LIMITER_VANLEER: return ens_sweep<1, CFL>(e, dir, 1, s);
-    default: return ens_sweep<-1, CFL>(e, dir, e->limiter, s);
+    case LIMITER_OSPRE: return ens_sweep<0, CFL>(e, dir, fromSecond, 0, s);
+    case LIMITER_VANLEER: return ens_sweep<1, CFL>(e, dir, fromSecond, 1, s);
+    default: return ens_sweep<-1, CFL>(e, dir, fromSecond, e->limiter, s);
     }
 }
 
@@ -734,11 +747,14 @@ static int ens_iteration(EnsembleImpl *e, int it, hipStream_t s, bool useFold)
         int last = 0;
         for (int n = 0; n < 3; n++)
             if (kFluxcall[n][sweep] != 3) last = n;
+        int fromSecond = 0;  // the step's first sweep leaves the pool, its other one returns
         for (int n = 0; n < 3; n++) {
             const int d = kFluxcall[n][sweep];
             if (d == 3) continue;  // 2D problems
-            rc = (dirn < 0 && n == last) ? ens_sweep_lim<true>(e, d, s) : ens_sweep_lim<false>(e, d, s);
+            rc = (dirn < 0 && n == last) ? ens_sweep_lim<true>(e, d, fromSecond, s)
+                                         : ens_sweep_lim<false>(e, d, fromSecond, s);
             if (rc) return rc;
+            fromSecond = !fromSecond;
         }
         if ((rc = ens_source(e, dirn > 0 ? 1.0 : 0.5, s))) return rc;
     }
@@ -754,6 +770,20 @@ struct ImogenEnsemble {
 };
 
 extern "C" {
+
+// A second pool of n doubles, or null when it would not leave half of the
+// device's free memory (the sweeps then work in place).
+static double *second_pool(int64_t n)
+{
+    size_t freeB = 0, totalB = 0;
+    double *p = nullptr;
+    if (hipMemGetInfo(&freeB, &totalB) != hipSuccess || (size_t)n * sizeof(double) > freeB / 2 ||
+        hipMalloc(&p, (size_t)n * sizeof(double)) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return p;
+}
 
 int imogen_ensemble_create(int nprob, const int *nx, const int *ny, const double *hx, const double *hy, double gamma,
                            int limiter, double cfl, ImogenEnsemble **out)
@@ -783,14 +813,18 @@ int imogen_ensemble_create(int nprob, const int *nx, const int *ny, const double
         const int64_t pitch = (n + 31) / 32 * 32;  // 256-byte slabs
         off[p] = total;
         total += 5 * pitch;
-        e->host.push_back(EnsProblem{nullptr, pitch, nx[p], ny[p], hx[p], hy[p], gamma, p, -1, 0, 0});
+        e->host.push_back(EnsProblem{nullptr, nullptr, pitch, nx[p], ny[p], hx[p], hy[p], gamma, p, -1, 0, 0});
         e->cells += n;
-        e->segS.push_back(ny[p] >= 256 ? 2 : 1);
         e->xcls.push_back(x_class_of(nx[p]));
     }
     int rc = SUCCESSFUL;
     if (IM_HIP(hipMalloc(&e->pool, (size_t)total * sizeof(double)))) rc = ERROR_CUDA_BLEW_UP;
-    for (int p = 0; p < nprob && !rc; p++) e->host[p].q = e->pool + off[p];
+    if (!rc) e->pool2 = second_pool(total);
+    for (int p = 0; p < nprob && !rc; p++) {
+        e->host[p].q = e->pool + off[p];
+        e->host[p].q2 = (e->pool2 ? e->pool2 : e->pool) + off[p];
+        e->segS.push_back(!e->pool2 && ny[p] >= 256 ? 2 : 1);
+    }
     if (!rc && IM_HIP(hipMalloc(&e->dprobs, nprob * sizeof(EnsProblem)))) rc = ERROR_CUDA_BLEW_UP;
     if (!rc && IM_HIP(hipMemcpy(e->dprobs, e->host.data(), nprob * sizeof(EnsProblem), hipMemcpyHostToDevice)))
         rc = ERROR_CUDA_BLEW_UP;
@@ -873,7 +907,7 @@ int imogen_ensemble_set_dust(ImogenEnsemble *E, const int *hasDust, double dustG
         }
     if (dusty.empty()) return SUCCESSFUL;
     const int NE = e->P + (int)dusty.size();
-    double *dpool = nullptr, *lam = nullptr, *part = nullptr;
+    double *dpool = nullptr, *dpool2 = nullptr, *lam = nullptr, *part = nullptr;
     EnsProblem *dprobs = nullptr;
     EnsDragTable *tab = nullptr;
     EnsDragItem *items = nullptr;
@@ -884,10 +918,12 @@ int imogen_ensemble_set_dust(ImogenEnsemble *E, const int *hasDust, double dustG
     std::vector<EnsDragItem> hitems;
     int64_t off = 0;
     int rc = IM_HIP(hipMalloc(&dpool, (size_t)total * sizeof(double)));
+    if (!rc && e->pool2) dpool2 = second_pool(total);
     for (size_t k = 0; k < dusty.size() && !rc; k++) {
         const int p = dusty[k];
         EnsProblem D = host[p];
         D.q = dpool + off;
+        D.q2 = (dpool2 ? dpool2 : dpool) + off;
         D.gamma = dustGamma;
         D.owner = p;
         D.dust = -1;
@@ -909,7 +945,7 @@ int imogen_ensemble_set_dust(ImogenEnsemble *E, const int *hasDust, double dustG
     if (!rc) rc = IM_HIP(hipMalloc(&queue, (size_t)cells * 2 * sizeof(int64_t)));  // queue + second-call list
     if (!rc) rc = IM_HIP(hipMalloc(&qcount, 3 * sizeof(unsigned long long)));
     if (rc) {
-        void *bufs[] = {dpool, dprobs, lam, part, tab, items, queue, qcount};
+        void *bufs[] = {dpool, dpool2, dprobs, lam, part, tab, items, queue, qcount};
         for (void *b : bufs)
             if (b) (void)hipFree(b);
         return ERROR_CUDA_BLEW_UP;
@@ -921,6 +957,13 @@ int imogen_ensemble_set_dust(ImogenEnsemble *E, const int *hasDust, double dustG
     e->NE = NE;
     e->Pd = (int)dusty.size();
     e->dpool = dpool;
+    e->dpool2 = dpool2;
+    if (e->pool2 && !dpool2) {  // one mode for all: in place
+        (void)hipFree(e->pool2);
+        e->pool2 = nullptr;
+        for (EnsProblem &P : e->host) P.q2 = P.q;
+        for (int p = 0; p < e->P; p++) e->segS[p] = e->host[p].ny >= 256 ? 2 : 1;
+    }
     e->dprobs = dprobs;
     e->lam = lam;
     e->cflPart = part;
@@ -1044,12 +1087,13 @@ int imogen_ensemble_autotune(ImogenEnsemble *E, int trials, int *chosen)
         return rc;
     };
     int rc = SUCCESSFUL;
-    // Y-march segments per size class (ny <= 128, <= 256, <= 512) among {1, 2, 4}:
+    // Y-march segments (factors on the base counts when there is a second pool)
+    // per size class (ny <= 128, <= 256, <= 512) among {1, 2, 4}:
     // the class's default first, another count only when it is 1 % faster (two
     // trial iterations differ by about that)
-    static const int cand[3][3] = {{1, 2, 4}, {1, 2, 4}, {2, 1, 4}};
+    const int cand[3][3] = {{1, 2, 4}, {1, 2, 4}, {e->pool2 ? 1 : 2, e->pool2 ? 2 : 1, 4}};
     auto cls_of = [](int ny) { return ny <= 128 ? 0 : (ny <= 256 ? 1 : 2); };
-    int best[3] = {1, 1, 2};
+    int best[3] = {1, 1, cand[2][0]};
     for (int cls = 0; cls < 3 && !rc; cls++) {
         bool any = false;
         for (int p = 0; p < e->P; p++) any = any || cls_of(e->host[p].ny) == cls;
@@ -1133,7 +1177,7 @@ int imogen_ensemble_destroy(ImogenEnsemble *E)
     free_graphs(e);
     for (int c = 0; c < kXClasses; c++)
         if (e->xwork[c]) (void)hipFree(e->xwork[c]);
-    void *bufs[] = {e->pool,   e->dprobs,   e->lam,       e->clock, e->cflPart, e->fold, e->cflList, e->ywork, e->xdummy,
+    void *bufs[] = {e->pool,   e->pool2,    e->dpool2,    e->dprobs,   e->lam,       e->clock, e->cflPart, e->fold, e->cflList, e->ywork, e->xdummy,
                     e->ydefer, e->dpool,    e->dtp,       e->dragTab, e->dragItems, e->queue, e->qcount};
     for (void *p : bufs)
         if (p) (void)hipFree(p);

@@ -11,16 +11,18 @@
 // wrap along the swept line (cudaFluidStep.cu:1159-1162).
 //
 // Two data-movement schemes, both free of transposes:
-//  * X (contiguous) lines: a wave owns whole lines. Each lane holds K
-//    consecutive cells in registers; the one-cell neighbours it needs from the
-//    adjacent lanes (primitives, left face, flux) come by cross-lane shuffle.
-//    No LDS, no barrier, no halo re-read.
+//  * X (contiguous) lines: a wave owns whole lines or, for long or few lines,
+//    a part of one. Each lane holds K consecutive cells in registers; the
+//    one-cell neighbours it needs from the adjacent lanes (primitives, left
+//    face, flux) come by cross-lane shuffle. No LDS.
 //  * Y/Z (strided) lines: each lane marches along one column (coalesced over
 //    x across the wave) keeping a register window of the two-stage stencil.
-//    Columns may be split into S segments held by lanes of the same wave, for
-//    occupancy; a segment reads its 4-cell halos directly, and keeps its first
-//    4 outputs in a scratch buffer until the whole wave has finished reading,
-//    so the in-place update (and the periodic wrap) is race-free.
+//    Columns are split into segments for occupancy. A sweep whose output goes
+//    to a second state array (update_3d pairs such sweeps) may cut them
+//    anywhere; one that works in place keeps a column's segments in one wave,
+//    and each segment its first 4 outputs in a scratch buffer until the whole
+//    wave has finished reading, so the update (and the periodic wrap) is
+//    race-free.
 #include "sweep_kernels.h"
 #include "imogen_internal.h"
 
@@ -31,9 +33,9 @@ namespace imogen {
 // host launchers
 // ---------------------------------------------------------------------------
 
-// Segments per column for the Y/Z march, S in {1, 2, 4} (W = 64/S columns per
-// wave, so every lane has a column slot). The kernel's time follows the
-// busiest SIMD: with w waves over 1024 SIMDs (256 CUs x 4, up to 2 resident
+// Segments per column of an in-place Y/Z march, S in {1, 2, 4} (W = 64/S
+// columns per wave, so every lane has a column slot). The kernel's time follows
+// the busiest SIMD: with w waves over 1024 SIMDs (256 CUs x 4, up to 2 resident
 // waves each) it runs ceil(w / 1024) waves of seglen + 9 steps, and a launch
 // with fewer waves than SIMDs runs about 1.8x slower per step (idle SIMDs,
 // no latency hiding). Segments shorter than 16 cells are not used. Measured
@@ -45,7 +47,7 @@ namespace imogen {
 // lines: S = 3, 6 (21, 10 columns) ran 1.5-2x slower than S = 2 or 4 (smooth
 // state, 160^3-384^3; 192^3: S=3 0.374, S=6 0.395 against S=4 0.197), and
 // S = 8 (8 columns, 64 bytes) 1.3-1.5x slower.
-static int march_segments(int64_t columns, int N)
+static int segments_in_place(int64_t columns, int N)
 {
     int best = 1;
     double bestCost = 0.0;
@@ -62,38 +64,74 @@ static int march_segments(int64_t columns, int N)
     return best;
 }
 
-// Launch shape of an X sweep over nlines lines of N cells: K cells per lane,
-// nl lanes per line, 256-thread blocks. K = 0 when N is above 1024.
+// Segments per column of an out-of-place march, any count: a wave holds one
+// segment of 64 columns, a segment of L cells takes L + 9 steps, and a step
+// of one wave is bound by its issue (about 1.0 us alone on a SIMD, 1.15 us
+// per wave with two), so the time is about ceil(waves / 1024) (L + 9); a lone
+// wave per SIMD also waits for memory (the 5 %). Measured (HLLC, van Leer,
+// smooth states, us; in place in brackets):
+//   1024^2 L=8 61  L=16 46  L=32 57 (305)      64^3  L=4 22.5  L=8 26  L=16 34 (35)
+//   600^2  L=4 37  L=6 26   L=16 35 (193)      128^3 L=16 72   L=32 60 L=64 94 (65)
+//   160^3  L=16 133 L=32 105 L=80 136 (124)    192^3 L=32 195  L=64 174 L=192 268 (212)
+//   256^3  Y: L=64 363  L=128 341  L=256 355 (409-480)  Z: 353, 329, 345 (336-353)
+static int segments_out_of_place(int64_t columns, int N)
+{
+    const int64_t colWaves = (columns + 63) / 64;
+    int best = 1;
+    double bestCost = 0.0;
+    for (int S = 1; S == 1 || S * 4 <= N; S++) {
+        const int64_t rounds = (colWaves * S + 1023) / 1024;
+        const double cost = (double)rounds * ((N + S - 1) / S + 9) * (rounds == 1 ? 1.05 : 1.0);
+        if (S == 1 || cost < bestCost) {
+            best = S;
+            bestCost = cost;
+        }
+        if (rounds > 16) break;
+    }
+    return best;
+}
+
+// Launch shape of an X sweep over nlines lines of N cells: K cells per lane;
+// parts = 0: whole lines (sweep_x, nl lanes per line, 256-thread blocks),
+// otherwise one line per block, split over `parts` waves (sweep_xp).
+// K = 0 when N is above 1024.
 struct XGeom {
-    int K = 0, nl = 0;
+    int K = 0, nl = 0, parts = 0;
     int64_t blocks = 0;
-    bool split = false;  // sweep_xh: halves of the line, one wave each, 2 lines per 256-thread block
+    int threads = 256;
 };
 
+// A part's window is its cells and 8 more, so K cells per lane take parts of
+// at most 64 K - 8 cells. Measured (HLLC, van Leer, smooth states, us):
+//  * Lines of up to 256 cells fill most lanes whole and a wave prefetches its
+//    next lines (65536 lines of 256: whole K=4 365, K=3 in 2 parts 534), as do
+//    lines of exactly 384 (36864 lines: whole K=6 363, K=4 in 2 parts 414,
+//    K=3 in 3 453).
+//  * Longer ones: K=3 (321: K=3 253, K=2 271, K=4 298; 512 x 32768: K=3 459,
+//    K=5 476, whole K=8 471; 1024 x 1024: K=3 39.5, K=5 44.1, K=4 55.6, and
+//    whole lines of 16 cells per lane, whose arrays left the registers, 130),
+//    but K=4 where two parts of it replace three (369..496).
+//  * Too few lines to fill the 1024 SIMDs: smaller K for a shorter chain per
+//    wave (17 lines of 300: K=1 5.3, K=2 5.7, K=3 6.6; 400 x 400: K=1 8.8,
+//    K=2 8.9, K=3 10.8), as far as 8 waves reach.
 static XGeom x_geom(int N, int64_t nlines)
 {
     XGeom g;
-    if (N > 256 && N <= 512 && N != 384 && N != 512) {
-        // halves of <= 184 / 248 / 256 cells plus 8 window cells in 3 / 4 / 5-cell lanes.
-        // Lines of exactly 384 or 512 cells fill every lane of a whole-line wave
-        // (6 or 8 cells each) and stay whole: 384^3 X sweep 1.13 ms whole,
-        // 1.43 split; 512^3 3.33 whole, 3.29 split; 320^3 1.29 whole (partly
-        // filled lanes), 0.78 split.
-        g.split = true;
-        g.K = (N <= 3 * 64 * 2 - 16) ? 3 : (N <= 4 * 64 * 2 - 16 ? 4 : 5);
-        g.nl = 64;
-        g.blocks = (nlines + 1) / 2;
+    if (N > 1024) return g;
+    const auto parts = [N](int K) { return (N + 64 * K - 9) / (64 * K - 8); };
+    if (N > 64 && N <= 256 && nlines * parts(1) <= 1024) {
+        g.K = 1;
+    } else if (N > 256 && N != 384) {
+        if (nlines * parts(3) >= 1536) g.K = (N > 368 && N <= 496) ? 4 : 3;
+        else g.K = parts(1) <= 8 ? 1 : (parts(2) <= 8 ? 2 : 3);
+    }
+    if (g.K) {
+        g.parts = parts(g.K);
+        g.threads = 64 * g.parts;
+        g.blocks = nlines;
         return g;
     }
-    if (N <= 64) g.K = 1;
-    else if (N <= 128) g.K = 2;
-    else if (N <= 192) g.K = 3;
-    else if (N <= 256) g.K = 4;
-    else if (N == 384) g.K = 6;
-    else if (N == 512) g.K = 8;
-    else if (N <= 768) g.K = 12;
-    else if (N <= 1024) g.K = 16;
-    else return g;
+    g.K = (N == 384) ? 6 : (N + 63) / 64;
     g.nl = (N + g.K - 1) / g.K;
     const int lpw = 64 / g.nl;
     int64_t waves = (nlines + lpw - 1) / lpw;
@@ -104,121 +142,123 @@ static XGeom x_geom(int N, int64_t nlines)
     return g;
 }
 
-// Launch shape of a Y (dir 2) or Z (dir 3) march: S segments per column, a
-// grid of blocksPerRow x nother blocks of 256 threads (nthr in all).
+// Launch shape of a Y (dir 2) or Z (dir 3) march: S segments per column,
+// blocks of 256 threads (nthr in all).
 struct MarchGeom {
-    int N = 0, nother = 0, S = 1, seglen = 0, wavesPerRow = 0, blocksPerRow = 0;
-    int64_t nthr = 0;
+    int N = 0, S = 1, seglen = 0;
+    int64_t columns = 0, blocks = 0, nthr = 0;
 };
 
-static MarchGeom march_geom(int nx, int ny, int nz, int dir)
+static MarchGeom march_geom(int nx, int ny, int nz, int dir, bool inplace)
 {
     MarchGeom g;
     g.N = (dir == 2) ? ny : nz;
-    g.nother = (dir == 2) ? nz : ny;
-    g.S = march_segments((int64_t)nx * g.nother, g.N);
+    g.columns = (int64_t)nx * ((dir == 2) ? nz : ny);
+    g.S = inplace ? segments_in_place(g.columns, g.N) : segments_out_of_place(g.columns, g.N);
     g.seglen = (g.N + g.S - 1) / g.S;
-    const int W = 64 / g.S;
-    g.wavesPerRow = (nx + W - 1) / W;
-    g.blocksPerRow = (g.wavesPerRow + 3) / 4;
-    g.nthr = (int64_t)g.blocksPerRow * g.nother * 256;
+    if (!inplace) g.S = (g.N + g.seglen - 1) / g.seglen;  // no empty segment
+    const int W = inplace ? 64 / g.S : 64;
+    const int64_t colWaves = (g.columns + W - 1) / W;
+    g.blocks = ((inplace ? colWaves : colWaves * g.S) + 3) / 4;
+    g.nthr = g.blocks * 256;
     return g;
 }
 
+// Scratch doubles per marching lane: a dummy slot of 5 and, in place, 4
+// deferred outputs.
+static int march_slots(bool inplace)
+{
+    return inplace ? 25 : 5;
+}
+
+// Scratch of one launch: past the first `off` bytes of the library's block,
+// which update_3d keeps a second state array in.
+static void *sweep_scratch(size_t off, size_t bytes)
+{
+    char *p = (char *)scratch_block(off + bytes);
+    return p ? p + off : nullptr;
+}
+
 template <class M, int LIM>
-static int launch_x(double *q, int64_t pitch, int N, int64_t nlines, double lambda, const double *lamp,
-                    const HydroConsts &hc, int rt, const CflFuse &cf, hipStream_t s)
+static int launch_x(const double *src, double *dst, size_t scratchOff, int64_t pitch, int N, int64_t nlines,
+                    double lambda, const double *lamp, const HydroConsts &hc, int rt, const CflFuse &cf, hipStream_t s)
 {
     const XGeom g = x_geom(N, nlines);
     if (g.K == 0) return IM_FAIL(ERROR_NOIMPLEMENT, "X sweep supports lines of at most 1024 cells (got %d)", N);
     const int K = g.K, nl = g.nl;
-    const int64_t blocks = g.blocks;
-    if (cf.part && blocks * 4 > cf.cap) return IM_FAIL(ERROR_INVALID_ARGS, "CFL partial buffer too small");
-    if (blocks > INT32_MAX) return IM_FAIL(ERROR_INVALID_ARGS, "too many lines for one X launch");
-    dim3 grid((unsigned)blocks), block(256);
-    const bool full = (nl * K == N) && (64 % nl == 0);
-    double *dummy = (double *)scratch_block((size_t)blocks * 256 * 5 * sizeof(double));
-    if (!dummy) return IM_FAIL(ERROR_NOMEM, "no scratch for the X sweep");
-    if (g.split) {
-#define IM_XH(KK)                                                                                        \
-    case KK:                                                                                             \
-        if (cf.part)                                                                                     \
-            hipLaunchKernelGGL((sweep_xh<M, KK, LIM, true>), grid, block, 0, s, q, pitch, N, nlines, lambda, \
-                               lamp, hc, rt, dummy, cf);                                                 \
-        else                                                                                             \
-            hipLaunchKernelGGL((sweep_xh<M, KK, LIM, false>), grid, block, 0, s, q, pitch, N, nlines,     \
-                               lambda, lamp, hc, rt, dummy, cf);                                         \
+    if (cf.part && g.blocks * (g.threads / 64) > cf.cap)
+        return IM_FAIL(ERROR_INVALID_ARGS, "CFL partial buffer too small");
+    if (g.blocks > INT32_MAX) return IM_FAIL(ERROR_INVALID_ARGS, "too many lines for one X launch");
+    dim3 grid((unsigned)g.blocks), block((unsigned)g.threads);
+    if (g.parts) {
+#define IM_XP(KK, C)                                                                                          \
+    hipLaunchKernelGGL((sweep_xp<M, KK, LIM, C>), grid, block, 0, s, src, dst, pitch, N, g.parts, lambda, \
+                       lamp, hc, rt, cf)
+#define IM_XP_CASE(KK)                  \
+    case KK:                            \
+        if (cf.part) IM_XP(KK, true);   \
+        else IM_XP(KK, false);          \
         break;
         switch (K) {
-            IM_XH(3)
-            IM_XH(4)
-            IM_XH(5)
+            IM_XP_CASE(1)
+            IM_XP_CASE(2)
+            IM_XP_CASE(3)
+            IM_XP_CASE(4)
         }
-#undef IM_XH
-        return IM_LAUNCHED("sweep_xh");
+#undef IM_XP_CASE
+#undef IM_XP
+        return IM_LAUNCHED("sweep_xp");
     }
-#define IM_XK(KK)                                                                                       \
-    case KK:                                                                                            \
-        if (cf.part) {                                                                                  \
-            if (full)                                                                                   \
-                hipLaunchKernelGGL((sweep_x<M, KK, LIM, true, true>), grid, block, 0, s, q, pitch, N,    \
-                                   nlines, nl, lambda, lamp, hc, rt, dummy, cf);                        \
-            else                                                                                        \
-                hipLaunchKernelGGL((sweep_x<M, KK, LIM, false, true>), grid, block, 0, s, q, pitch, N,   \
-                                   nlines, nl, lambda, lamp, hc, rt, dummy, cf);                        \
-        } else if (full) {                                                                              \
-            hipLaunchKernelGGL((sweep_x<M, KK, LIM, true, false>), grid, block, 0, s, q, pitch, N,       \
-                               nlines, nl, lambda, lamp, hc, rt, dummy, cf);                            \
-        } else {                                                                                        \
-            hipLaunchKernelGGL((sweep_x<M, KK, LIM, false, false>), grid, block, 0, s, q, pitch, N,      \
-                               nlines, nl, lambda, lamp, hc, rt, dummy, cf);                            \
-        }                                                                                               \
-        break;
-#define IM_XK_FULL(KK)                                                                                  \
-    case KK:                                                                                            \
-        if (!full) return IM_FAIL(ERROR_INVALID_ARGS, "X lines of %d cells in %d-cell lanes", N, KK);     \
-        if (cf.part)                                                                                    \
-            hipLaunchKernelGGL((sweep_x<M, KK, LIM, true, true>), grid, block, 0, s, q, pitch, N, nlines, \
-                               nl, lambda, lamp, hc, rt, dummy, cf);                                    \
-        else                                                                                            \
-            hipLaunchKernelGGL((sweep_x<M, KK, LIM, true, false>), grid, block, 0, s, q, pitch, N, nlines, \
-                               nl, lambda, lamp, hc, rt, dummy, cf);                                    \
+    const bool full = (nl * K == N) && (64 % nl == 0);
+    double *dummy = (double *)sweep_scratch(scratchOff, (size_t)g.blocks * 256 * 5 * sizeof(double));
+    if (!dummy) return IM_FAIL(ERROR_NOMEM, "no scratch for the X sweep");
+#define IM_X(KK, F, C)                                                                                        \
+    hipLaunchKernelGGL((sweep_x<M, KK, LIM, F, C>), grid, block, 0, s, src, dst, pitch, N, nlines, nl, lambda, lamp, \
+                       hc, rt, dummy, cf)
+#define IM_X_CASE(KK)                              \
+    case KK:                                       \
+        if (full && cf.part) IM_X(KK, true, true); \
+        else if (full) IM_X(KK, true, false);      \
+        else if (cf.part) IM_X(KK, false, true);   \
+        else IM_X(KK, false, false);               \
         break;
     switch (K) {
-        IM_XK(1)
-        IM_XK(2)
-        IM_XK(3)
-        IM_XK(4)
-        IM_XK_FULL(6)
-        IM_XK_FULL(8)
-        IM_XK(12)
-        IM_XK(16)
+        IM_X_CASE(1)
+        IM_X_CASE(2)
+        IM_X_CASE(3)
+        IM_X_CASE(4)
+    case 6:  // 384 cells: every lane full
+        if (cf.part) IM_X(6, true, true);
+        else IM_X(6, true, false);
+        break;
     }
-#undef IM_XK
-#undef IM_XK_FULL
+#undef IM_X_CASE
+#undef IM_X
     return IM_LAUNCHED("sweep_x");
 }
 
 template <class M, int LIM>
-static int launch_march(double *q, int64_t pitch, int nx, int ny, int nz, int dir, double lambda,
-                        const double *lamp, const HydroConsts &hc, int rt, const CflFuse &cf, hipStream_t s)
+static int launch_march(const double *src, double *dst, size_t scratchOff, int64_t pitch, int nx, int ny, int nz,
+                        int dir, double lambda, const double *lamp, const HydroConsts &hc, int rt, const CflFuse &cf,
+                        hipStream_t s)
 {
     const int64_t sstride = (dir == 2) ? (int64_t)nx : (int64_t)nx * ny;
     const int64_t ostride = (dir == 2) ? (int64_t)nx * ny : (int64_t)nx;
-    const MarchGeom g = march_geom(nx, ny, nz, dir);
-    const int N = g.N, S = g.S, seglen = g.seglen, wavesPerRow = g.wavesPerRow;
-    dim3 grid((unsigned)g.blocksPerRow, (unsigned)g.nother), block(256);
-    const int64_t nthr = g.nthr;
-    if (cf.part && nthr / 64 > cf.cap) return IM_FAIL(ERROR_INVALID_ARGS, "CFL partial buffer too small");
-    // 4 deferred output slots + 1 dummy slot of 5 doubles per lane
-    double *defer = (double *)scratch_block((size_t)nthr * 25 * sizeof(double));
+    const MarchGeom g = march_geom(nx, ny, nz, dir, src == dst);
+    if (g.blocks > INT32_MAX) return IM_FAIL(ERROR_INVALID_ARGS, "too many columns for one march launch");
+    dim3 grid((unsigned)g.blocks), block(256);
+    if (cf.part && g.nthr / 64 > cf.cap) return IM_FAIL(ERROR_INVALID_ARGS, "CFL partial buffer too small");
+    double *defer = (double *)sweep_scratch(scratchOff, (size_t)g.nthr * march_slots(src == dst) * sizeof(double));
     if (!defer) return IM_FAIL(ERROR_NOMEM, "no scratch for deferred outputs");
     // rows of a multiple of 16 cells in a 256-byte-aligned slab: every segment
-    // row (16, 32 or 64 columns) is whole 128-byte lines -> nontemporal hint
-    const bool lines = (nx % 16) == 0 && (pitch % 32) == 0 && ((uintptr_t)q % 256) == 0;
-#define IM_MARCH(D, C, T)                                                                                  \
-    hipLaunchKernelGGL((sweep_march<M, D, LIM, C, T>), grid, block, 0, s, q, pitch, nx, sstride, ostride, N, S, \
-                       seglen, wavesPerRow, lambda, lamp, hc, rt, defer, cf)
+    // row (16, 32 or 64 columns) is whole 128-byte lines -> nontemporal hint,
+    // for states beyond the 256 MB last-level cache (256^3: 341 us with it,
+    // 347 without; 192^3: 174 and 170, 1024^2: 46 and 43)
+    const bool lines = (nx % 16) == 0 && (pitch % 32) == 0 && (((uintptr_t)src | (uintptr_t)dst) % 256) == 0 &&
+                       pitch * 5 * (int64_t)sizeof(double) > (int64_t)256 << 20;
+#define IM_MARCH(D, C, T)                                                                                      \
+    hipLaunchKernelGGL((sweep_march<M, D, LIM, C, T>), grid, block, 0, s, src, dst, pitch, nx, sstride, ostride, \
+                       g.columns, g.N, g.S, g.seglen, lambda, lamp, hc, rt, defer, cf)
 #define IM_MARCH_NT(D, C)             \
     do {                              \
         if (lines) IM_MARCH(D, C, true);  \
@@ -237,52 +277,60 @@ static int launch_march(double *q, int64_t pitch, int nx, int ny, int nz, int di
 }
 
 template <class M, int LIM>
-static int launch_dir(double *q, int64_t pitch, int nx, int ny, int nz, int dir, double lambda,
-                      const double *lamp, const HydroConsts &hc, int rt, const CflFuse &cf, hipStream_t s)
+static int launch_dir(const double *src, double *dst, size_t off, int64_t pitch, int nx, int ny, int nz, int dir,
+                      double lambda, const double *lamp, const HydroConsts &hc, int rt, const CflFuse &cf,
+                      hipStream_t s)
 {
     const int slot = prof_begin(PROF_SWEEP_X + dir - 1, s);
     int rc;
-    if (dir == 1) rc = launch_x<M, LIM>(q, pitch, nx, (int64_t)ny * nz, lambda, lamp, hc, rt, cf, s);
-    else rc = launch_march<M, LIM>(q, pitch, nx, ny, nz, dir, lambda, lamp, hc, rt, cf, s);
+    if (dir == 1) rc = launch_x<M, LIM>(src, dst, off, pitch, nx, (int64_t)ny * nz, lambda, lamp, hc, rt, cf, s);
+    else rc = launch_march<M, LIM>(src, dst, off, pitch, nx, ny, nz, dir, lambda, lamp, hc, rt, cf, s);
     prof_end(slot, s);
     return rc;
 }
 
 template <class M>
-static int launch_method(double *base, int64_t pitch, int nx, int ny, int nz, int dir, double lambda,
-                         const double *lamp, const HydroConsts &hc, int limiter, const CflFuse &cf, hipStream_t s)
+static int launch_method(const double *src, double *dst, size_t off, int64_t pitch, int nx, int ny, int nz, int dir,
+                         double lambda, const double *lamp, const HydroConsts &hc, int limiter, const CflFuse &cf,
+                         hipStream_t s)
 {
     switch (limiter) {
-    case LIMITER_OSPRE: return launch_dir<M, 0>(base, pitch, nx, ny, nz, dir, lambda, lamp, hc, 0, cf, s);
-    case LIMITER_VANLEER: return launch_dir<M, 1>(base, pitch, nx, ny, nz, dir, lambda, lamp, hc, 1, cf, s);
+    case LIMITER_OSPRE: return launch_dir<M, 0>(src, dst, off, pitch, nx, ny, nz, dir, lambda, lamp, hc, 0, cf, s);
+    case LIMITER_VANLEER: return launch_dir<M, 1>(src, dst, off, pitch, nx, ny, nz, dir, lambda, lamp, hc, 1, cf, s);
     case LIMITER_MINMOD:
     case LIMITER_SUPERBEE:
     case LIMITER_VANALBADA:
     case LIMITER_MC:
-    case LIMITER_ZERO: return launch_dir<M, -1>(base, pitch, nx, ny, nz, dir, lambda, lamp, hc, limiter, cf, s);
+    case LIMITER_ZERO:
+        return launch_dir<M, -1>(src, dst, off, pitch, nx, ny, nz, dir, lambda, lamp, hc, limiter, cf, s);
     default: return IM_FAIL(ERROR_INVALID_ARGS, "unknown slope limiter %d", limiter);
     }
 }
 
 // The grid arithmetic of launch_x / launch_march, for sizing fused-CFL buffers.
-int64_t sweep_waves(int nx, int ny, int nz, int dir)
+int64_t sweep_waves(int nx, int ny, int nz, int dir, bool inplace)
 {
-    if (dir == 1) return x_geom(nx, (int64_t)ny * nz).blocks * 4;
-    const MarchGeom g = march_geom(nx, ny, nz, dir);
-    return (int64_t)g.blocksPerRow * g.nother * 4;
+    if (dir == 1) {
+        const XGeom g = x_geom(nx, (int64_t)ny * nz);
+        return g.blocks * (g.threads / 64);
+    }
+    return march_geom(nx, ny, nz, dir, inplace).nthr / 64;
 }
 
-int64_t sweep_scratch_bytes(int nx, int ny, int nz, int dir)
+int64_t sweep_scratch_bytes(int nx, int ny, int nz, int dir, bool inplace)
 {
     const int N = (dir == 1) ? nx : (dir == 2 ? ny : nz);
     if (dir < 1 || dir > 3 || N < 3) return 0;
-    if (dir == 1) return x_geom(nx, (int64_t)ny * nz).blocks * 256 * 5 * (int64_t)sizeof(double);
-    return march_geom(nx, ny, nz, dir).nthr * 25 * (int64_t)sizeof(double);
+    if (dir == 1) {
+        const XGeom g = x_geom(nx, (int64_t)ny * nz);
+        return g.parts ? 0 : g.blocks * 256 * 5 * (int64_t)sizeof(double);
+    }
+    return march_geom(nx, ny, nz, dir, inplace).nthr * march_slots(inplace) * (int64_t)sizeof(double);
 }
 
-int launch_fluid_sweep(double *base, int64_t pitch, int nx, int ny, int nz, int dir, int method, double lambda,
-                       double gamma, double rhomin, double ciso, int limiter, hipStream_t s, const double *lamp,
-                       const CflFuse *cfl)
+int launch_fluid_sweep(const double *src, double *dst, size_t scratchOff, int64_t pitch, int nx, int ny, int nz,
+                       int dir, int method, double lambda, double gamma, double rhomin, double ciso, int limiter,
+                       hipStream_t s, const double *lamp, const CflFuse *cfl)
 {
     if (dir < 1 || dir > 3) return IM_FAIL(ERROR_INVALID_ARGS, "sweep direction %d", dir);
     const int N = (dir == 1) ? nx : (dir == 2 ? ny : nz);
@@ -297,8 +345,9 @@ int launch_fluid_sweep(double *base, int64_t pitch, int nx, int ny, int nz, int 
     hc.cisosq = ciso * ciso;
     const CflFuse cf = cfl ? *cfl : CflFuse{};
     if (method == METHOD_HLLC)
-        return launch_method<Hllc>(base, pitch, nx, ny, nz, dir, lambda, lamp, hc, limiter, cf, s);
-    if (method == METHOD_HLL) return launch_method<Hll>(base, pitch, nx, ny, nz, dir, lambda, lamp, hc, limiter, cf, s);
+        return launch_method<Hllc>(src, dst, scratchOff, pitch, nx, ny, nz, dir, lambda, lamp, hc, limiter, cf, s);
+    if (method == METHOD_HLL)
+        return launch_method<Hll>(src, dst, scratchOff, pitch, nx, ny, nz, dir, lambda, lamp, hc, limiter, cf, s);
     return IM_FAIL(ERROR_INVALID_ARGS, "sweep kernel for method %d", method);
 }
 

@@ -281,7 +281,10 @@ int fluid_boundary(MGArray *fluid, int direction, int xrules, const GeometryPara
     return rc;
 }
 
-int update_1d(MGArray *fluid, const FluidStepParams &params, const double *lampBase, const CflFuse *cfl)
+// One directional update; to: where the swept state goes (null: in place;
+// HLLC and HLL only), scratchOff: as launch_fluid_sweep.
+static int sweep_1d(MGArray *fluid, double *to, size_t scratchOff, const FluidStepParams &params,
+                    const double *lampBase, const CflFuse *cfl)
 {
     double *base;
     int64_t pitch;
@@ -303,8 +306,8 @@ int update_1d(MGArray *fluid, const FluidStepParams &params, const double *lampB
     switch (params.stepMethod) {
     case METHOD_HLLC:
     case METHOD_HLL:
-        return launch_fluid_sweep(base, pitch, fluid->dim[0], fluid->dim[1], fluid->dim[2], dir,
-                                  (int)params.stepMethod, lambda, params.thermoGamma, params.minimumRho,
+        return launch_fluid_sweep(base, to ? to : base, scratchOff, pitch, fluid->dim[0], fluid->dim[1],
+                                  fluid->dim[2], dir, (int)params.stepMethod, lambda, params.thermoGamma, params.minimumRho,
                                   params.Cisothermal, params.slopeLimiter, st->stream, lamp, cfl);
     case METHOD_XINJIN:
         if (cfl) return IM_FAIL(ERROR_NOIMPLEMENT, "the CFL is not folded into Xin-Jin sweeps");
@@ -312,6 +315,51 @@ int update_1d(MGArray *fluid, const FluidStepParams &params, const double *lampB
                                    params.thermoGamma, params.minimumRho, st->stream, lamp);
     default: return IM_FAIL(ERROR_INVALID_ARGS, "unknown fluid method %d", (int)params.stepMethod);
     }
+}
+
+int update_1d(MGArray *fluid, const FluidStepParams &params, const double *lampBase, const CflFuse *cfl)
+{
+    return sweep_1d(fluid, nullptr, 0, params, lampBase, cfl);
+}
+
+// Sweeps through a second state array. A sweep that need not leave its input
+// alone can cut its lines anywhere, so it fills the chip also where the lines
+// are few (segments_out_of_place in fluid_sweep.hip has both modes' times). A
+// step's state must end in its canister, so such sweeps come in pairs: Y and
+// Z where both are swept, otherwise the march and X. The second array is the
+// start of the scratch block, up to kPairBytes of it (beyond that the columns
+// fill the chip); an allocation-free call pairs only what its fixed scratch
+// holds.
+constexpr size_t kPairBytes = (size_t)2 << 30;
+
+static size_t pair_bytes(const MGArray *fluid)
+{
+    return (size_t)fluid->slabPitch[0] * 5;
+}
+
+// bit d - 1: direction d is swept out of place
+static unsigned paired_dirs(const MGArray *fluid, int method)
+{
+    const int *d3 = fluid->dim;
+    if (method != METHOD_HLLC && method != METHOD_HLL) return 0;
+    if (d3[1] == 1 && d3[2] == 1) return 0;
+    const bool x = d3[0] > 3, y = d3[1] > 3, z = d3[2] > 3;
+    const unsigned dirs = (y && z) ? 6u : (x && y) ? 3u : (x && z) ? 5u : 0u;
+    const size_t bytes = pair_bytes(fluid);
+    if (!dirs || bytes > kPairBytes) return 0;
+    int64_t need = 0;
+    for (int d = 1; d <= 3; d++)
+        if (d3[d - 1] > 3) {
+            const int64_t b = sweep_scratch_bytes(d3[0], d3[1], d3[2], d, !(dirs >> (d - 1) & 1));
+            need = (b > need) ? b : need;
+        }
+    // sized here, before the sweeps, so that no launch moves the block
+    return scratch_available(bytes + (size_t)need) ? dirs : 0;
+}
+
+bool sweep_out_of_place(const MGArray *fluid, int method, int dir)
+{
+    return paired_dirs(fluid, method) >> (dir - 1) & 1;
 }
 
 // flux.cu:27-155 on one rank: the sweep order of (stepNumber, stepDirection),
@@ -389,15 +437,38 @@ int update_3d(MGArray *fluid, const FluidStepParams &fsp, const double *lampBase
     }
     int sweep = (fsp.stepNumber + 3 * (fsp.stepDirection > 0)) % 6;
     if (sweep < 0) sweep += 6;
+    const unsigned paired = paired_dirs(fluid, (int)fsp.stepMethod);
+    // the fluid and its image in the second array, where the sweeps between
+    // the two paired ones find the state
+    MGArray other[5];
+    double *base = fluid->devicePtr[0], *second = nullptr;
+    size_t off = 0;
+    if (paired) {
+        off = pair_bytes(fluid);
+        second = (double *)scratch_block(off);
+        if (!second) return ERROR_NOMEM;
+        for (int k = 0; k < 5; k++) {
+            other[k] = fluid[k];
+            other[k].devicePtr[0] = second + (fluid[k].devicePtr[0] - base);
+        }
+    }
+    MGArray *at = fluid;
     for (int n = 0; n < 3; n++) {
         const int d = kFluxcall[n][sweep];
         if (fluid->dim[d - 1] > 3) {  // flux.cu:102
             p.stepDirection = d;
-            rc = update_1d(fluid, p, lampBase, (lastCfl && d == last) ? &cf : nullptr);
+            double *to = nullptr;
+            MGArray *next = at;
+            if (paired >> (d - 1) & 1) {
+                to = (at == fluid) ? second : base;
+                next = (at == fluid) ? other : fluid;
+            }
+            rc = sweep_1d(at, to, off, p, lampBase, (lastCfl && d == last) ? &cf : nullptr);
             if (rc) return rc;
+            at = next;
             // the reference sets these boundaries with direction d rotated into
             // memory x (flux.cu:99-107): the x kernels' conventions along d
-            rc = fluid_boundary(fluid, d, 1, &fsp.geometry);
+            rc = fluid_boundary(at, d, 1, &fsp.geometry);
             if (rc) return rc;
         }
     }
@@ -504,7 +575,7 @@ int performFluidUpdate_3D_noalloc(MGArray *fluid, ParallelTopology *parallelTopo
     for (int d = 1; d <= 3; d++) {
         if (line ? d != 1 : d3[d - 1] <= 3) continue;
         const int64_t b = (method == METHOD_XINJIN) ? xinjin_scratch_bytes(pitch, d3[0], d3[1], d3[2], d)
-                                                    : sweep_scratch_bytes(d3[0], d3[1], d3[2], d);
+                                                    : sweep_scratch_bytes(d3[0], d3[1], d3[2], d, true);
         if (b > need) need = b;
     }
     if (need > (int64_t)kFixedScratchBytes)

@@ -76,9 +76,13 @@ void prof_suspend(int on);
 // ERROR_NOMEM message when bytes is above kFixedScratchBytes) and never
 // allocates.
 void *scratch_block(size_t bytes);
+// Whether scratch_block(bytes) will succeed, for callers that can do with
+// less: the block is grown to that size unless it would take more than half of
+// the free device memory.
+bool scratch_available(size_t bytes);
 // Scratch bytes launch_fluid_sweep / launch_xinjin_sweep take for one sweep
 // (the launch shapes of fluid_sweep.hip and xinjin.hip).
-int64_t sweep_scratch_bytes(int nx, int ny, int nz, int dir);
+int64_t sweep_scratch_bytes(int nx, int ny, int nz, int dir, bool inplace);
 int64_t xinjin_scratch_bytes(int64_t pitch, int nx, int ny, int nz, int dir);
 
 // Validates a 5-array fluid canister (slab views of one 5-slab owner, XYZ
@@ -107,6 +111,9 @@ int update_3d(MGArray *fluid, const FluidStepParams &fsp, const double *lampBase
 int fluid_boundary(MGArray *fluid, int direction, int xrules, const GeometryParams *geo);
 // Direction swept last by update_3d for (stepNumber, stepDirection), 0 if none.
 int last_sweep_dir(const MGArray *fluid, int stepNumber, int stepDirection);
+// Whether update_3d runs direction dir of a step of this fluid and method out
+// of place, as one of a pair of sweeps through a second state array.
+bool sweep_out_of_place(const MGArray *fluid, int method, int dir);
 // Cells [lo, hi) of direction dir whose swept values survive the boundary
 // conditions update_3d sets after the sweep, when every other ghost they write
 // is a copy or mirror image of one of them (modes circular, mirror, const).
@@ -120,9 +127,12 @@ int cfl_keep_range(MGArray *fluid, int dir, int *lo, int *hi);
 // = dt/h from this device address instead of the `lambda` argument.
 // cfl: when not null, the sweep also writes the per-wave CFL minima of the
 // cells it stores (cfl_device.h).
-int launch_fluid_sweep(double *base, int64_t pitch, int nx, int ny, int nz, int dir, int method, double lambda,
-                       double gamma, double rhomin, double ciso, int limiter, hipStream_t s,
-                       const double *lamp = nullptr, const CflFuse *cfl = nullptr);
+// src == dst: in place; otherwise the swept state goes to dst, another array
+// of the same pitch, and src stays as it was. scratchOff: bytes at the start of
+// the scratch block the launch leaves alone.
+int launch_fluid_sweep(const double *src, double *dst, size_t scratchOff, int64_t pitch, int nx, int ny, int nz,
+                       int dir, int method, double lambda, double gamma, double rhomin, double ciso, int limiter,
+                       hipStream_t s, const double *lamp = nullptr, const CflFuse *cfl = nullptr);
 int launch_xinjin_sweep(double *base, int64_t pitch, int nx, int ny, int nz, int dir, double lambda,
                         double gamma, double rhomin, hipStream_t s, const double *lamp = nullptr);
 // xrules: apply the memory-x kernels' conventions along direction dir (the
@@ -159,6 +169,6 @@ int launch_cfl(const double *base, int64_t pitch, int64_t n, const double *cs, d
 int launch_cfl_final(const double *part, int64_t n, int halve, double *devOut, hipStream_t s);
 // Wave count of a sweep launch over an nx x ny x nz HLLC/HLL array in
 // direction dir (the entries a fused CFL needs).
-int64_t sweep_waves(int nx, int ny, int nz, int dir);
+int64_t sweep_waves(int nx, int ny, int nz, int dir, bool inplace);
 
 }  // namespace imogen

@@ -97,6 +97,25 @@ int take_device_errors(DeviceState *st)
                    c0, c1, c2, c3);
 }
 
+bool scratch_available(size_t bytes)
+{
+    DeviceState *st = state();
+    if (!st) return false;
+    if (st->fixedScratchOn) return bytes <= kFixedScratchBytes;
+    if (bytes <= st->scratchBytes) return true;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return false;  // the block cannot grow while the stream is captured
+    }
+    size_t freeB = 0, totalB = 0;
+    if (hipMemGetInfo(&freeB, &totalB) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return bytes + bytes / 4 <= freeB / 2 && scratch_block(bytes);
+}
+
 void *scratch_block(size_t bytes)
 {
     DeviceState *st = state();

@@ -151,9 +151,10 @@ __device__ __forceinline__ void x_fluxes(const HydroConsts &hc, int rt, V5 (&U)[
 // wait only for the loads it needs); lanes past the last line read a clamped
 // valid line and write into a private dummy slot.
 template <class M, int K, int LIM, bool FULL, bool CFL>
-__global__ __launch_bounds__(256, (K <= 4) ? 2 : 1) void sweep_x(double *__restrict__ q, int64_t pitch, int N, int64_t nlines,
-                                               int nl, double lambda, const double *__restrict__ lamp,
-                                               HydroConsts hc, int rt, double *__restrict__ dummy, CflFuse cf)
+__global__ __launch_bounds__(256, (K <= 4) ? 2 : 1) void sweep_x(const double *src, double *dst, int64_t pitch, int N,
+                                               int64_t nlines, int nl, double lambda,
+                                               const double *__restrict__ lamp, HydroConsts hc, int rt,
+                                               double *__restrict__ dummy, CflFuse cf)
 {
     if (lamp) lambda = lamp[0];  // time step kept on the device
     const int lane = threadIdx.x & 63;
@@ -176,12 +177,12 @@ __global__ __launch_bounds__(256, (K <= 4) ? 2 : 1) void sweep_x(double *__restr
     double *mydummy = dummy + gtid;
     const int64_t groupStride = nwaves * lpw;
 
-    auto line_ptr = [&](int64_t ln) {
+    auto line_off = [&](int64_t ln) {
         const int64_t c = ln < nlines ? ln : nlines - 1;
-        return q + c * (int64_t)N + x0;
+        return c * (int64_t)N + x0;
     };
     auto load_group = [&](int64_t ln, V5 (&Qd)[K]) {
-        double *b = line_ptr(ln);
+        const double *b = src + line_off(ln);
 #pragma unroll
         for (int k = 0; k < K; k++) {
             if (k < cnt) Qd[k] = load_cell<M, 1>(b + k, pitch);
@@ -213,13 +214,13 @@ __global__ __launch_bounds__(256, (K <= 4) ? 2 : 1) void sweep_x(double *__restr
         // stage B: Q = .5((U1 + Q) - lambda dF(U1))
         x_fluxes<M, K, LIM>(hc, rt, U1, cnt, srcL, srcR, F, Fm);
         const bool own = laneUsed && line < nlines;
-        double *dst = own ? line_ptr(line) : mydummy;
+        double *to = own ? dst + line_off(line) : mydummy;
         const int64_t st = own ? pitch : nthr;
 #pragma unroll
         for (int k = 0; k < K; k++) {
             if (k < cnt) {
                 const V5 o = avg_update(add5(U1[k], Q[k]), lambda, F[k], k == 0 ? Fm : F[k > 0 ? k - 1 : 0]);
-                store_cell<M, 1>(own ? dst + k : dst, st, o);
+                store_cell<M, 1>(own ? to + k : to, st, o);
                 if (CFL && own && x0 + k >= cf.lo && x0 + k < cf.hi) {
                     const double u = cfl_of_cell<M, 1>(cf.a, o);
                     cmin = (u < cmin) ? u : cmin;
@@ -238,31 +239,22 @@ __global__ __launch_bounds__(256, (K <= 4) ? 2 : 1) void sweep_x(double *__restr
     }
 }
 
-// X sweep of lines of 257-512 cells split into halves, one wave per half. A
-// wave holds its half and the 4 cells beyond each end (the two stages'
-// stencil, periodic within the line, as the whole-line sweep reads them), so
-// it forms its half's outputs alone; the window's outer cells only feed
-// discarded values. The two waves of a line are in one workgroup (4 waves: 2
-// lines), and every load of the workgroup precedes the barrier while every
-// store follows it, so no wave overwrites a cell its partner has still to
-// read. K = 3, 4 or 5 cells per lane keeps two waves per SIMD where a whole
-// line needs 6 or 8 at one.
+// One wave's part of an X line: part `part` of `parts` (near-equal runs of
+// cells), K consecutive cells per lane. The wave's window is its part and the
+// 4 cells beyond each end (the two stages' stencil, periodic within the line),
+// so it forms its outputs alone; the window's outer cells only feed discarded
+// values. inplace: the waves of a line share a workgroup and every load of the
+// workgroup precedes the barrier while every store follows it, so no wave
+// overwrites a cell another has still to read. valid false: nothing is stored. CFL: cmin takes the minimum CFL
+// limit of the outputs at cells [cf.lo, cf.hi), nanc counts the NaN limits.
 template <class M, int K, int LIM, bool CFL>
-__global__ __launch_bounds__(256, 2) void sweep_xh(double *__restrict__ q, int64_t pitch, int N, int64_t nlines,
-                                                  double lambda, const double *__restrict__ lamp, HydroConsts hc,
-                                                  int rt, double *__restrict__ dummy, CflFuse cf)
+__device__ __forceinline__ void xp_body(const double *src, double *dst, int64_t pitch, int N, int part, int parts,
+                                        bool valid, bool inplace, double lambda, const HydroConsts &hc, int rt,
+                                        const CflFuse &cf, double &cmin, unsigned &nanc)
 {
-    if (lamp) lambda = lamp[0];  // time step kept on the device
     const int lane = threadIdx.x & 63;
-    const int wib = threadIdx.x >> 6;
-    const int64_t wave = (int64_t)blockIdx.x * 4 + wib;
-    int64_t line = (int64_t)blockIdx.x * 2 + (wib >> 1);
-    const bool lineValid = line < nlines;
-    line = lineValid ? line : nlines - 1;  // waves past the last line still meet the barrier
-    const int part = wib & 1;
-    const int h = (N + 1) >> 1;
-    const int s0 = part ? h : 0;             // first output cell of this half
-    const int Wn = (part ? N - h : h) + 8;   // window: the half and 4 cells beyond each end
+    const int s0 = (int)((int64_t)N * part / parts);  // first output cell of this part
+    const int Wn = (int)((int64_t)N * (part + 1) / parts) - s0 + 8;
     const int nl = (Wn + K - 1) / K;
     const bool laneUsed = lane < nl;
     const int srcL = laneUsed ? (lane == 0 ? nl - 1 : lane - 1) : lane;
@@ -271,7 +263,6 @@ __global__ __launch_bounds__(256, 2) void sweep_xh(double *__restrict__ q, int64
     int cnt = Wn - w0;
     cnt = cnt < K ? cnt : K;
     if (!laneUsed) cnt = 0;
-    double *row = q + line * (int64_t)N;
     V5 Q[K];
 #pragma unroll
     for (int k = 0; k < K; k++) {
@@ -279,58 +270,75 @@ __global__ __launch_bounds__(256, 2) void sweep_xh(double *__restrict__ q, int64
         g = (g < 0) ? g + N : g;
         g = (g >= N) ? g - N : g;
         g = (g < N) ? g : N - 1;
-        Q[k] = (k < cnt) ? load_cell<M, 1>(row + g, pitch) : V5{1.0, 1.0, 0.0, 0.0, 0.0};
+        Q[k] = (k < cnt) ? load_cell<M, 1>(src + g, pitch) : V5{1.0, 1.0, 0.0, 0.0, 0.0};
     }
-    __syncthreads();
+    if (inplace) __syncthreads();
     V5 F[K], Fm;
     x_fluxes<M, K, LIM>(hc, rt, Q, cnt, srcL, srcR, F, Fm);
     V5 U1[K];
 #pragma unroll
     for (int k = 0; k < K; k++) U1[k] = axpy_update(Q[k], lambda, F[k], k == 0 ? Fm : F[k > 0 ? k - 1 : 0]);
     x_fluxes<M, K, LIM>(hc, rt, U1, cnt, srcL, srcR, F, Fm);
-    const int64_t gtid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t nthr = (int64_t)gridDim.x * blockDim.x;
-    double cmin = 1e38;
 #pragma unroll
     for (int k = 0; k < K; k++) {
-        if (k < cnt) {
-            const int w = w0 + k;
-            const bool own = lineValid && w >= 4 && w < Wn - 4;
+        const int w = w0 + k;
+        if (k < cnt && valid && w >= 4 && w < Wn - 4) {
             const int x = s0 + w - 4;
             const V5 o = avg_update(add5(U1[k], Q[k]), lambda, F[k], k == 0 ? Fm : F[k > 0 ? k - 1 : 0]);
-            store_cell<M, 1>(own ? row + x : dummy + gtid, own ? pitch : nthr, o);
-            if (CFL && own && x >= cf.lo && x < cf.hi) {
+            store_cell<M, 1>(dst + x, pitch, o);
+            if (CFL && x >= cf.lo && x < cf.hi) {
                 const double u = cfl_of_cell<M, 1>(cf.a, o);
                 cmin = (u < cmin) ? u : cmin;
+                nanc += (u != u);
             }
         }
     }
+}
+
+// X sweep of lines split into parts: one wave per part, one line per
+// workgroup of 64 parts threads (two lines per workgroup measured 1-20 %
+// slower: the barrier then waits for both).
+template <class M, int K, int LIM, bool CFL>
+__global__ __launch_bounds__(512, 2) void sweep_xp(const double *src, double *dst, int64_t pitch, int N, int parts,
+                                                  double lambda, const double *__restrict__ lamp, HydroConsts hc,
+                                                  int rt, CflFuse cf)
+{
+    if (lamp) lambda = lamp[0];  // time step kept on the device
+    const int wib = threadIdx.x >> 6;
+    const int64_t line = blockIdx.x;
+    double cmin = 1e38;
+    unsigned nanc = 0;  // not reported by the single-array fold
+    xp_body<M, K, LIM, CFL>(src + line * (int64_t)N, dst + line * (int64_t)N, pitch, N, wib, parts, true, src == dst,
+                            lambda, hc, rt, cf, cmin, nanc);
     if (CFL) {
         cmin = wave_min(cmin);
-        if (lane == 0) cf.part[wave] = cmin;
+        if ((threadIdx.x & 63) == 0) cf.part[(int64_t)blockIdx.x * (blockDim.x >> 6) + wib] = cmin;
     }
 }
 
 // ---------------------------------------------------------------------------
 // Y/Z sweep: register-window march along strided columns
 // ---------------------------------------------------------------------------
-// One wave-uniform march over the segments of W = 64/S columns: lane `lane`
-// walks cells [j0, j0+L) of the column starting at `col` (stride sstride, N
-// cells, periodic), the wave's stencil ring in LDS at `ring`. defer/gtid/nthr
-// address this lane's deferred-output slots. seglen is uniform over the wave.
-// CFL: cmin takes the minimum CFL limit of the outputs at column cells
-// [cf.lo, cf.hi), nanc counts the NaN limits among them.
+// One wave-uniform march: lane `lane` walks cells [j0, j0+L) of the column
+// starting at `col` (stride sstride, N cells, periodic), the wave's stencil
+// ring in LDS at `ring`, and writes to the column starting at `out`. In place
+// (out == col) the segments of a column belong to one wave and first = 4: a
+// segment's first 4 outputs, which its neighbours' halo reads and the periodic
+// wrap still need, wait in this lane's deferred slots (defer/gtid/nthr) until
+// the wave has finished reading. Out of place first = 0. seglen is uniform
+// over the wave. CFL: cmin takes the minimum CFL limit of the outputs at
+// column cells [cf.lo, cf.hi), nanc counts the NaN limits among them.
 template <class M, int DIR, int LIM, bool CFL = false, bool NT = false>
-__device__ __forceinline__ void march_body(double *__restrict__ col, int64_t pitch, int64_t sstride, int N,
-                                           int seglen, int j0, int L, double lambda, const HydroConsts &hc,
-                                           int rt, double *__restrict__ defer, int64_t gtid, int64_t nthr,
-                                           double (*ring)[5][64], int lane, const CflFuse &cf, double &cmin,
-                                           unsigned &nanc)
+__device__ __forceinline__ void march_body(const double *col, double *out, int64_t pitch, int64_t sstride, int N,
+                                           int seglen, int j0, int L, int first, double lambda,
+                                           const HydroConsts &hc, int rt, double *__restrict__ defer, int64_t gtid,
+                                           int64_t nthr, double (*ring)[5][64], int lane, const CflFuse &cf,
+                                           double &cmin, unsigned &nanc)
 {
     // wrapped sweep index of the first load (m = j0 - 4), in [0, N)
     int mw = (j0 - 4) % N;
     if (mw < 0) mw += N;
-    double *outp = col + (int64_t)(j0 - 9) * sstride;  // address of output t - 9
+    double *outp = out + (int64_t)(j0 - 9) * sstride;  // address of output t - 9
     double *const dfr = defer + gtid;
     const int64_t dstride = 5 * nthr;
 
@@ -385,8 +393,8 @@ __device__ __forceinline__ void march_body(double *__restrict__ col, int64_t pit
         const V5 S5{r[0], r[64], r[128], r[192], r[256]};
         const V5 o = avg_update(S5, lambda, FBn, FBp);  // cell m-5
 
-        // Every step stores exactly 5 doubles: to the cell (outputs 4..L-1), to
-        // a deferred slot (outputs 0..3) or to this lane's dummy slot (no
+        // Every step stores exactly 5 doubles: to the cell (outputs first..L-1),
+        // to a deferred slot (earlier ones) or to this lane's dummy slot (no
         // output yet / past the segment). With a fixed store count per step the
         // compiler can wait for a prefetched load without waiting for stores
         // (stores share the vector-memory counter on gfx9).
@@ -398,8 +406,8 @@ __device__ __forceinline__ void march_body(double *__restrict__ col, int64_t pit
             cmin = (u < cmin) ? u : cmin;
             nanc += (u != u);
         }
-        const bool direct = (oi >= 4) & (oi < L);
-        const int slot = ((oi >= 0) & (oi < 4) & (oi < L)) ? oi : 4;
+        const bool direct = (oi >= first) & (oi < L);
+        const int slot = ((oi >= 0) & (oi < first) & (oi < L)) ? oi : first;
         double *dq = dfr + (int64_t)slot * dstride;
         double *dst = direct ? outp : dq;
         const int64_t st = direct ? pitch : nthr;
@@ -419,7 +427,7 @@ __device__ __forceinline__ void march_body(double *__restrict__ col, int64_t pit
     // back-edge (load group, then 5 stores) so the wait at the loop head can
     // leave stores outstanding: the stores write the loaded cell into this
     // lane's dummy slot, which also pins them after the load.
-    store_cell<M, DIR, NT>(defer + gtid + (int64_t)4 * 5 * nthr, nthr, N0);
+    store_cell<M, DIR, NT>(dfr + (int64_t)first * dstride, nthr, N0);
 
     // Steps go in pairs. When maxsteps is odd the last pair's second step is
     // one past the segment: it loads a valid (wrapped) cell and stores to the
@@ -437,52 +445,59 @@ __device__ __forceinline__ void march_body(double *__restrict__ col, int64_t pit
     }
 
     // every lane of the wave has finished reading: release the deferred outputs
-    const int nd = L < 4 ? L : 4;
+    const int nd = L < first ? L : first;
     for (int oi = 0; oi < nd; oi++) {
         const V5 o = load_cell<M, DIR, NT>(defer + gtid + (int64_t)oi * 5 * nthr, nthr);
-        store_cell<M, DIR, NT>(col + (int64_t)(j0 + oi) * sstride, pitch, o);
+        store_cell<M, DIR, NT>(out + (int64_t)(j0 + oi) * sstride, pitch, o);
     }
 }
 
+// Columns are numbered x + nx * o (o: the other direction), so a wave's
+// columns run on across rows and every lane but the last wave's has one.
+// In place: a wave holds W = 64/S columns, their S segments side by side in
+// its lanes. Out of place (dst != src): a wave holds one segment of 64 columns
+// and the segments of a column are waves of their own, segment-major.
 template <class M, int DIR, int LIM, bool CFL, bool NT>
-__global__ __launch_bounds__(256) void sweep_march(double *__restrict__ q, int64_t pitch, int nx, int64_t sstride,
-                                                   int64_t ostride, int N, int S, int seglen, int wavesPerRow,
-                                                   double lambda, const double *__restrict__ lamp,
+__global__ __launch_bounds__(256) void sweep_march(const double *src, double *dst, int64_t pitch, int nx,
+                                                   int64_t sstride, int64_t ostride, int64_t columns, int N, int S,
+                                                   int seglen, double lambda, const double *__restrict__ lamp,
                                                    HydroConsts hc, int rt, double *__restrict__ defer, CflFuse cf)
 {
     if (lamp) lambda = lamp[0];  // time step kept on the device
     const int lane = threadIdx.x & 63;
     const int wib = threadIdx.x >> 6;
-    const int64_t waveId = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * (blockDim.x >> 6) + wib;
-    const int W = 64 / S;
-    const int s = lane / W;
-    const int c = lane - s * W;
-    const int64_t wrow = (int64_t)blockIdx.x * (blockDim.x >> 6) + wib;  // wave index within this row
-    if (wrow >= wavesPerRow) {
-        if (CFL && lane == 0) cf.part[waveId] = 1e38;
+    const int64_t wave = (int64_t)blockIdx.x * (blockDim.x >> 6) + wib;
+    const bool inplace = src == dst;
+    const int W = inplace ? 64 / S : 64;
+    const int64_t colWaves = (columns + W - 1) / W;
+    if (wave >= (inplace ? colWaves : colWaves * S)) {
+        if (CFL && lane == 0) cf.part[wave] = 1e38;
         return;
     }
-    const int64_t x = wrow * W + c;
-    const bool colValid = (x < nx) && (s < S);
-    // lanes of no column (x past the grid, or s >= S when S does not divide
+    const int64_t cw = inplace ? wave : wave % colWaves;
+    const int s = inplace ? lane / W : (int)(wave / colWaves);
+    const int64_t cid = cw * W + lane % W;
+    const bool colValid = (cid < columns) && (s < S);
+    // lanes of no column (past the last, or s >= S when S does not divide
     // 64) march a zero-length segment from row 0: their unconditional loads
     // then stay inside the column
     const int j0 = colValid ? s * seglen : 0;
     int L = N - j0;
     L = L < seglen ? L : seglen;
-    if (!colValid) L = 0;
+    if (!colValid || L < 0) L = 0;
 
-    double *col = q + (colValid ? x + (int64_t)blockIdx.y * ostride : 0);
-    const int64_t gtid = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;
-    const int64_t nthr = (int64_t)gridDim.x * gridDim.y * blockDim.x;
+    const int64_t other = cid / nx;
+    const int64_t off = colValid ? (cid - other * nx) + other * ostride : 0;
+    const int64_t gtid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t nthr = (int64_t)gridDim.x * blockDim.x;
     __shared__ double sring[4][4][5][64];  // [wave in block][slot][variable][lane]
     double cmin = 1e38;
     unsigned nanc = 0;  // not reported by the single-array fold
-    march_body<M, DIR, LIM, CFL, NT>(col, pitch, sstride, N, seglen, j0, L, lambda, hc, rt, defer, gtid, nthr,
-                                     sring[wib], lane, cf, cmin, nanc);
+    march_body<M, DIR, LIM, CFL, NT>(src + off, dst + off, pitch, sstride, N, seglen, j0, L, inplace ? 4 : 0, lambda,
+                                     hc, rt, defer, gtid, nthr, sring[wib], lane, cf, cmin, nanc);
     if (CFL) {
         cmin = wave_min(cmin);
-        if (lane == 0) cf.part[waveId] = cmin;
+        if (lane == 0) cf.part[wave] = cmin;
     }
 }
 

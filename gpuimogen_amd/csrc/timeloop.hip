@@ -173,7 +173,9 @@ static int iteration(TimeloopImpl *L, int it, bool fusedCfl, hipStream_t s)
     for (int f = 0; f < L->nf; f++) {
         if (fusedCfl && L->fuse[f]) {
             const MGArray *a = L->fluid[f];
-            const int64_t n = sweep_waves(a->dim[0], a->dim[1], a->dim[2], last_sweep_dir(a, it - 1, -1));
+            const int last = last_sweep_dir(a, it - 1, -1);
+            const int64_t n = sweep_waves(a->dim[0], a->dim[1], a->dim[2], last,
+                                          !sweep_out_of_place(a, (int)L->p[f].stepMethod, last));
             rc = launch_cfl_final(L->cf[f].part, n, 1, L->dbuf + kClockDoubles + (int64_t)f * kCflSlot, s);
         } else {
             rc = cfl_of(L, f, s);
@@ -249,8 +251,10 @@ int imogen_timeloop_create(MGArray *fluids, int nfluids, const GeometryParams *g
             if (!swept) continue;
             int lo, hi;
             if (a->dim[d - 1] <= 3 || cfl_keep_range(a, d, &lo, &hi)) ok = false;
-            const int64_t w = sweep_waves(a->dim[0], a->dim[1], a->dim[2], d);
-            cap = (w > cap) ? w : cap;
+            for (int in = 0; in < 2; in++) {
+                const int64_t w = sweep_waves(a->dim[0], a->dim[1], a->dim[2], d, in);
+                cap = (w > cap) ? w : cap;
+            }
         }
         if (!ok || cap == 0) continue;
         CflFuse &c = L->cf[f];
