@@ -816,165 +816,222 @@ __global__ __launch_bounds__(256) void drag_samples_kernel(int64_t n, const doub
 }
 
 // ---------------------------------------------------------------------------
-// FP32 training kernels: 64 rows per block of 256 threads
+// FP32 training kernels: groups of 16 rows per block of 256 threads
 // ---------------------------------------------------------------------------
-constexpr int kRows = 64;
+// The 64 x 64 products run on the FP32 MFMA (16x16x4, FP32 operands and
+// accumulation): wave w of a block owns hidden units 16 w .. 16 w + 15, and 16
+// rows are one tile, so a batch of 2048 makes 128 blocks (64 rows per block on
+// VALU loops: 32 blocks, forward 20 us and backward 126 us at that batch; the
+// launches are bound by their latency, not by the 0.06 GFLOP). The MFMA's
+// contraction index is free as long as both operands use the same one, so
+// lane group q = lane / 16 takes k = 16 q + i at step i: 16 consecutive
+// values, read as four 16-byte words.
+constexpr int kRows = 16;
+constexpr int kPadH = kHid + 4;      // LDS row of hidden units, 16-byte aligned
+constexpr int kBwdBlocks = 256;      // backward blocks at most (each leaves one partial gradient)
 
+__device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // a caller's buffer
+
+// 16 consecutive floats of a 16-byte aligned row
+__device__ __forceinline__ void load16(const float *p, float (&v)[16])
+{
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const float4 x = *reinterpret_cast<const float4 *>(p + 4 * i);
+        v[4 * i] = x.x;
+        v[4 * i + 1] = x.y;
+        v[4 * i + 2] = x.z;
+        v[4 * i + 3] = x.w;
+    }
+}
+
+// D = A B with A's row lane % 16 at k = 16 q + i in a[i] and B's column
+// lane % 16 there in b[i]; four accumulators, so no MFMA waits for the last
+__device__ __forceinline__ f32x4 mfma_k64(const float (&a)[16], const float (&b)[16])
+{
+    f32x4 c[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+    for (int i = 0; i < 16; i++) c[i & 3] = mfma_f32(a[i], b[i], c[i & 3]);
+    return (c[0] + c[1]) + (c[2] + c[3]);
+}
+
+// The forward pass adds its terms in the order of the units (k = 4 i + q at
+// step i, one accumulator that starts as the bias), the order of a plain loop.
 __global__ __launch_bounds__(256) void mlp_fwd_kernel(const float *__restrict__ P, int64_t batch,
                                                       const float *__restrict__ x, float *__restrict__ act,
                                                       float *__restrict__ y)
 {
-    __shared__ float W2[kHid][kHid];
-    __shared__ float H[kRows][kHid + 1];
+    __shared__ float H[kRows][kPadH];
+    __shared__ float H2[kRows][kPadH];
+    __shared__ float W3[kHid * kOut];
     const int t = threadIdx.x;
     const int64_t r0 = (int64_t)blockIdx.x * kRows;
-    for (int k = t; k < kHid * kHid; k += 256) W2[k / kHid][k % kHid] = P[kOffW2 + k];
-    const int r = t >> 2;          // row within the block
-    const int j0 = (t & 3) * 16;   // 16 hidden units per thread
+    const int lane = t & 63, w = t >> 6, q = lane >> 4, n = lane & 15;
+    // W2's column 16 w + n at rows 4 i + q
+    float b[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) b[i] = P[kOffW2 + (4 * i + q) * kHid + 16 * w + n];
+    const float b2 = P[kOffB2 + 16 * w + n];
+    if (t < kHid * kOut) W3[t] = P[kOffW3 + t];
+    const int r = t >> 4;         // row of layer 1
+    const int j0 = (t & 15) * 4;  // its 4 hidden units
     const int64_t row = r0 + r;
-    const bool live = row < batch;
     float xv[kIn];
 #pragma unroll
-    for (int k = 0; k < kIn; k++) xv[k] = live ? x[row * kIn + k] : 0.0f;
-    float *a = act + (live ? row : 0) * 256;
+    for (int k = 0; k < kIn; k++) xv[k] = row < batch ? x[row * kIn + k] : 0.0f;
+    float z[4], h[4];
 #pragma unroll
-    for (int jj = 0; jj < 16; jj++) {
-        const int j = j0 + jj;
-        float z = P[kOffB1 + j];
+    for (int jj = 0; jj < 4; jj++) {
+        z[jj] = P[kOffB1 + j0 + jj];
 #pragma unroll
-        for (int k = 0; k < kIn; k++) z += xv[k] * P[kOffW1 + k * kHid + j];
-        const float h = gelu_f(z);
-        H[r][j] = h;
-        if (live) {
-            a[j] = z;
-            a[64 + j] = h;
+        for (int k = 0; k < kIn; k++) z[jj] += xv[k] * P[kOffW1 + k * kHid + j0 + jj];
+        h[jj] = gelu_f(z[jj]);
+        H[r][j0 + jj] = h[jj];
+    }
+    if (row < batch) {
+#pragma unroll
+        for (int jj = 0; jj < 4; jj++) {
+            act[row * 256 + j0 + jj] = z[jj];
+            act[row * 256 + 64 + j0 + jj] = h[jj];
         }
     }
     __syncthreads();
-    float z2[16];
+    f32x4 d = {b2, b2, b2, b2};
 #pragma unroll
-    for (int jj = 0; jj < 16; jj++) z2[jj] = P[kOffB2 + j0 + jj];
-    for (int k = 0; k < kHid; k++) {
-        const float h = H[r][k];
+    for (int i = 0; i < 16; i++) d = mfma_f32(H[n][4 * i + q], b[i], d);
 #pragma unroll
-        for (int jj = 0; jj < 16; jj++) z2[jj] += h * W2[k][j0 + jj];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int jj = 0; jj < 16; jj++) {
-        const float h = gelu_f(z2[jj]);
-        H[r][j0 + jj] = h;
-        if (live) {
-            a[128 + j0 + jj] = z2[jj];
-            a[192 + j0 + jj] = h;
+    for (int i = 0; i < 4; i++) {  // D: row 4 q + i, column n
+        const int rr = 4 * q + i;
+        const float h2 = gelu_f(d[i]);
+        H2[rr][16 * w + n] = h2;
+        if (r0 + rr < batch) {
+            act[(r0 + rr) * 256 + 128 + 16 * w + n] = d[i];
+            act[(r0 + rr) * 256 + 192 + 16 * w + n] = h2;
         }
     }
     __syncthreads();
     if (t < kRows * kOut) {
         const int rr = t / kOut, o = t % kOut;
-        const int64_t rw = r0 + rr;
         float v = P[kOffB3 + o];
-        for (int k = 0; k < kHid; k++) v += H[rr][k] * P[kOffW3 + k * kOut + o];
-        if (rw < batch) y[rw * kOut + o] = v;
+#pragma unroll 16
+        for (int k = 0; k < kHid; k++) v += H2[rr][k] * W3[k * kOut + o];
+        if (r0 + rr < batch) y[(r0 + rr) * kOut + o] = v;
     }
 }
 
-// Per-block gradient partials (deterministic); reduced by mlp_grad_reduce.
+// Per-block gradient partials (deterministic), summed over the block's row
+// groups in registers; added up by mlp_grad_reduce.
 __global__ __launch_bounds__(256) void mlp_bwd_kernel(const float *__restrict__ P, int64_t batch,
                                                       const float *__restrict__ x, const float *__restrict__ act,
                                                       const float *__restrict__ dy, float *__restrict__ part)
 {
-    __shared__ float W2[kHid][kHid];
-    __shared__ float DZ2[kRows][kHid + 1];
-    __shared__ float DZ1[kRows][kHid + 1];
+    __shared__ alignas(16) float DZ2[kRows][kPadH];
+    __shared__ alignas(16) float DZ1[kRows][kPadH];
+    __shared__ alignas(16) float H1[kRows][kPadH];
+    __shared__ alignas(16) float H2[kRows][kPadH];
     __shared__ float DY[kRows][kOut];
+    __shared__ float X[kRows][kIn];
     const int t = threadIdx.x;
-    const int64_t r0 = (int64_t)blockIdx.x * kRows;
-    for (int k = t; k < kHid * kHid; k += 256) W2[k / kHid][k % kHid] = P[kOffW2 + k];
-    if (t < kRows * kOut) {
-        const int rr = t / kOut, o = t % kOut;
-        DY[rr][o] = (r0 + rr < batch) ? dy[(r0 + rr) * kOut + o] : 0.0f;
-    }
-    __syncthreads();
-    const int r = t >> 2;
-    const int j0 = (t & 3) * 16;
-    const int64_t row = r0 + r;
-    const bool live = row < batch;
-    const float *a = act + (live ? row : 0) * 256;
-    // dz2 = (dy W3^T) * gelu'(z2)
+    const int lane = t & 63, w = t >> 6, q = lane >> 4, n = lane & 15;
+    float b[16];  // W2^T's column 16 w + n: W2's row, at its columns 16 q + i
 #pragma unroll
-    for (int jj = 0; jj < 16; jj++) {
-        const int j = j0 + jj;
-        float dh = 0.0f;
+    for (int i = 0; i < 16; i++) b[i] = P[kOffW2 + (16 * w + n) * kHid + 16 * q + i];
+    const int r = t >> 4;
+    const int j0 = (t & 15) * 4;
+    float w3[4][kOut];
 #pragma unroll
-        for (int o = 0; o < kOut; o++) dh += DY[r][o] * P[kOffW3 + j * kOut + o];
-        DZ2[r][j] = live ? dh * gelu_grad(a[128 + j]) : 0.0f;
-    }
-    __syncthreads();
-    // dz1 = (dz2 W2^T) * gelu'(z1)
+    for (int jj = 0; jj < 4; jj++)
 #pragma unroll
-    for (int jj = 0; jj < 16; jj++) {
-        const int k = j0 + jj;
-        float dh = 0.0f;
-        for (int j = 0; j < kHid; j++) dh += DZ2[r][j] * W2[k][j];
-        DZ1[r][k] = live ? dh * gelu_grad(a[k]) : 0.0f;
+        for (int o = 0; o < kOut; o++) w3[jj][o] = P[kOffW3 + (j0 + jj) * kOut + o];
+    f32x4 dw2[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};  // rows 16 w + 4 q + i, columns 16 jt + n
+    // the other gradients: unit u = t & 63 and a quarter of the sums each
+    const int u = t & 63;
+    float g1[2] = {0.0f, 0.0f}, g3[2] = {0.0f, 0.0f};
+    for (int64_t r0 = (int64_t)blockIdx.x * kRows; r0 < batch; r0 += (int64_t)gridDim.x * kRows) {
+        const int64_t row = r0 + r;
+        const bool live = row < batch;
+        __syncthreads();  // the previous group's readers are done
+        if (t < kRows * kOut) (&DY[0][0])[t] = (r0 * kOut + t < batch * kOut) ? dy[r0 * kOut + t] : 0.0f;
+        else if (t >= 64 && t < 64 + kRows * kIn)
+            (&X[0][0])[t - 64] = (r0 * kIn + t - 64 < batch * kIn) ? x[r0 * kIn + t - 64] : 0.0f;
+        // rows past the batch: zero activations and zero gradients
+        const f32x4u *ar = reinterpret_cast<const f32x4u *>(act + (live ? row : 0) * 256 + j0);
+        f32x4 z1 = ar[0], h1 = ar[16], z2 = ar[32], h2 = ar[48];
+        if (!live) z1 = h1 = z2 = h2 = f32x4{0, 0, 0, 0};
+        *reinterpret_cast<f32x4 *>(&H1[r][j0]) = h1;
+        *reinterpret_cast<f32x4 *>(&H2[r][j0]) = h2;
+        __syncthreads();
+        // dz2 = (dy W3^T) * gelu'(z2)
+#pragma unroll
+        for (int jj = 0; jj < 4; jj++) {
+            float dh = 0.0f;
+#pragma unroll
+            for (int o = 0; o < kOut; o++) dh += DY[r][o] * w3[jj][o];
+            DZ2[r][j0 + jj] = dh * gelu_grad(z2[jj]);
+            DZ1[r][j0 + jj] = gelu_grad(z1[jj]);
+        }
+        __syncthreads();
+        // dz1 = (dz2 W2^T) * gelu'(z1)
+        float a[16];
+        load16(&DZ2[n][16 * q], a);
+        const f32x4 d = mfma_k64(a, b);
+#pragma unroll
+        for (int i = 0; i < 4; i++) DZ1[4 * q + i][16 * w + n] *= d[i];
+        // dW2 = h1^T dz2 over the 16 rows (row 4 q + i at step i)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float ha = H1[4 * q + i][16 * w + n];
+#pragma unroll
+            for (int jt = 0; jt < 4; jt++) dw2[jt] = mfma_f32(ha, DZ2[4 * q + i][16 * jt + n], dw2[jt]);
+        }
+        __syncthreads();
+        // dW1 (wave w: input w; wave 0 also input 4), db1, db2 (waves 1, 2),
+        // dW3 (wave w < 3: output w), db3 (wave 3, first lanes)
+        for (int rr = 0; rr < kRows; rr++) {
+            const float d1 = DZ1[rr][u];
+            g1[0] += X[rr][w] * d1;
+            if (w == 0) g1[1] += X[rr][4] * d1;
+            else if (w == 1) g1[1] += d1;
+            else if (w == 2) g1[1] += DZ2[rr][u];
+            if (w < kOut) g3[0] += H2[rr][u] * DY[rr][w];
+            else if (u < kOut) g3[0] += DY[rr][u];
+        }
     }
-    __syncthreads();
     float *pp = part + (int64_t)blockIdx.x * kNParams;
-    // dW2[k][j] = sum_r h1[r][k] dz2[r][j]: thread owns 16 (k, j) pairs
-    for (int e = t; e < kHid * kHid; e += 256) {
-        const int k = e / kHid, j = e % kHid;
-        float s = 0.0f;
-        for (int rr = 0; rr < kRows; rr++) {
-            const int64_t rw = r0 + rr;
-            if (rw < batch) s += act[rw * 256 + 64 + k] * DZ2[rr][j];
-        }
-        pp[kOffW2 + e] = s;
-    }
-    // dW1[k][j] = sum_r x[r][k] dz1[r][j]; db1, db2
-    for (int e = t; e < kIn * kHid; e += 256) {
-        const int k = e / kHid, j = e % kHid;
-        float s = 0.0f;
-        for (int rr = 0; rr < kRows; rr++) {
-            const int64_t rw = r0 + rr;
-            if (rw < batch) s += x[rw * kIn + k] * DZ1[rr][j];
-        }
-        pp[kOffW1 + e] = s;
-    }
-    if (t < kHid) {
-        float s1 = 0.0f, s2 = 0.0f;
-        for (int rr = 0; rr < kRows; rr++) {
-            s1 += DZ1[rr][t];
-            s2 += DZ2[rr][t];
-        }
-        pp[kOffB1 + t] = s1;
-        pp[kOffB2 + t] = s2;
-    }
-    // dW3[k][o] = sum_r h2[r][k] dy[r][o]; db3
-    if (t < kHid * kOut) {
-        const int k = t / kOut, o = t % kOut;
-        float s = 0.0f;
-        for (int rr = 0; rr < kRows; rr++) {
-            const int64_t rw = r0 + rr;
-            if (rw < batch) s += act[rw * 256 + 192 + k] * DY[rr][o];
-        }
-        pp[kOffW3 + t] = s;
-    }
-    if (t < kOut) {
-        float s = 0.0f;
-        for (int rr = 0; rr < kRows; rr++) s += DY[rr][t];
-        pp[kOffB3 + t] = s;
-    }
+#pragma unroll
+    for (int jt = 0; jt < 4; jt++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) pp[kOffW2 + (16 * w + 4 * q + i) * kHid + 16 * jt + n] = dw2[jt][i];
+    pp[kOffW1 + w * kHid + u] = g1[0];
+    if (w == 0) pp[kOffW1 + 4 * kHid + u] = g1[1];
+    else if (w == 1) pp[kOffB1 + u] = g1[1];
+    else if (w == 2) pp[kOffB2 + u] = g1[1];
+    if (w < kOut) pp[kOffW3 + u * kOut + w] = g3[0];
+    else if (u < kOut) pp[kOffB3 + u] = g3[0];
 }
 
-__global__ __launch_bounds__(256) void mlp_grad_reduce(const float *__restrict__ part, int nblocks,
-                                                       float *__restrict__ grads)
+// 64 parameters per block, each of its 16 waves a sixteenth of the partials
+// (a thread per parameter over all partials: 8.6 us at 32 of them)
+__global__ __launch_bounds__(1024) void mlp_grad_reduce(const float *__restrict__ part, int nblocks,
+                                                        float *__restrict__ grads)
 {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= kNParams) return;
+    __shared__ float S[16][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int e = blockIdx.x * 64 + lane;
     float s = 0.0f;
-    for (int b = 0; b < nblocks; b++) s += part[(int64_t)b * kNParams + e];
-    grads[e] = s;
+    if (e < kNParams)
+        for (int b = w; b < nblocks; b += 16) s += part[(int64_t)b * kNParams + e];
+    S[w][lane] = s;
+    __syncthreads();
+    if (w == 0 && e < kNParams) {
+        for (int k = 1; k < 16; k++) s += S[k][lane];
+        grads[e] = s;
+    }
 }
 
 __global__ __launch_bounds__(256) void mlp_adam_kernel(float *__restrict__ p, const float *__restrict__ gr,
@@ -1246,14 +1303,15 @@ int imogen_mlp_backward(const float *params, int64_t batch, const float *x, cons
     if (batch <= 0) return SUCCESSFUL;
     DeviceState *st = state();
     if (!st) return ERROR_CUDA_BLEW_UP;
-    const int64_t blocks = (batch + kRows - 1) / kRows;
+    int64_t blocks = (batch + kRows - 1) / kRows;
+    if (blocks > kBwdBlocks) blocks = kBwdBlocks;
     float *part = (float *)scratch_block((size_t)blocks * kNParams * sizeof(float));
     if (!part) return IM_FAIL(ERROR_NOMEM, "no scratch for gradient partials");
     hipLaunchKernelGGL(mlp_bwd_kernel, dim3((unsigned)blocks), dim3(256), 0, st->stream, params, batch, x, act, dy,
                        part);
     int rc = IM_LAUNCHED("mlp_bwd_kernel");
     if (rc) return rc;
-    hipLaunchKernelGGL(mlp_grad_reduce, dim3((kNParams + 255) / 256), dim3(256), 0, st->stream, part, (int)blocks,
+    hipLaunchKernelGGL(mlp_grad_reduce, dim3((kNParams + 63) / 64), dim3(1024), 0, st->stream, part, (int)blocks,
                        grads);
     return IM_LAUNCHED("mlp_grad_reduce");
 }
