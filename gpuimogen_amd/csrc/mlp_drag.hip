@@ -816,52 +816,28 @@ __global__ __launch_bounds__(256) void drag_samples_kernel(int64_t n, const doub
 }
 
 // ---------------------------------------------------------------------------
-// FP32 training kernels: groups of 16 rows per block of 256 threads
+// FP32 training kernels, blocks of 256 threads
 // ---------------------------------------------------------------------------
 // The 64 x 64 products run on the FP32 MFMA (16x16x4, FP32 operands and
-// accumulation): wave w of a block owns hidden units 16 w .. 16 w + 15, and 16
-// rows are one tile, so a batch of 2048 makes 128 blocks (64 rows per block on
-// VALU loops: 32 blocks, forward 20 us and backward 126 us at that batch; the
-// launches are bound by their latency, not by the 0.06 GFLOP). The MFMA's
-// contraction index is free as long as both operands use the same one, so
-// lane group q = lane / 16 takes k = 16 q + i at step i: 16 consecutive
-// values, read as four 16-byte words.
-constexpr int kRows = 16;
-constexpr int kPadH = kHid + 4;      // LDS row of hidden units, 16-byte aligned
-constexpr int kBwdBlocks = 256;      // backward blocks at most (each leaves one partial gradient)
+// accumulation), every sum one accumulator in the order of a plain loop over
+// its terms (step i, lane group q = lane / 16 holds term 4 i + q). The forward
+// pass takes 16 rows per block, wave w the hidden units 16 w .. 16 w + 15; the
+// backward one 64 rows and 16 hidden units, four blocks per row group, so a
+// batch of 2048 makes 128 blocks of each (64 rows per block in VALU loops over
+// global activations: 32 blocks, forward 20 us and backward 126 us at that
+// batch, now 5 and 8). The launches are bound by their latency, not by the
+// 0.06 GFLOP.
+constexpr int kRows = 16;        // rows of a forward block
+constexpr int kBwdRows = 64;     // rows of a backward group: one partial gradient each
+constexpr int kPadH = kHid + 4;  // LDS row of hidden units
+
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // four floats of a caller's buffer
 
 __device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c)
 {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // a caller's buffer
-
-// 16 consecutive floats of a 16-byte aligned row
-__device__ __forceinline__ void load16(const float *p, float (&v)[16])
-{
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const float4 x = *reinterpret_cast<const float4 *>(p + 4 * i);
-        v[4 * i] = x.x;
-        v[4 * i + 1] = x.y;
-        v[4 * i + 2] = x.z;
-        v[4 * i + 3] = x.w;
-    }
-}
-
-// D = A B with A's row lane % 16 at k = 16 q + i in a[i] and B's column
-// lane % 16 there in b[i]; four accumulators, so no MFMA waits for the last
-__device__ __forceinline__ f32x4 mfma_k64(const float (&a)[16], const float (&b)[16])
-{
-    f32x4 c[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
-#pragma unroll
-    for (int i = 0; i < 16; i++) c[i & 3] = mfma_f32(a[i], b[i], c[i & 3]);
-    return (c[0] + c[1]) + (c[2] + c[3]);
-}
-
-// The forward pass adds its terms in the order of the units (k = 4 i + q at
-// step i, one accumulator that starts as the bias), the order of a plain loop.
 __global__ __launch_bounds__(256) void mlp_fwd_kernel(const float *__restrict__ P, int64_t batch,
                                                       const float *__restrict__ x, float *__restrict__ act,
                                                       float *__restrict__ y)
@@ -924,114 +900,110 @@ __global__ __launch_bounds__(256) void mlp_fwd_kernel(const float *__restrict__ 
     }
 }
 
-// Per-block gradient partials (deterministic), summed over the block's row
-// groups in registers; added up by mlp_grad_reduce.
+// Gradient partials per group of 64 rows (deterministic); added up by
+// mlp_grad_reduce. Block (group, c) forms those of hidden units 16 c ..
+// 16 c + 15 (rows of W2 and W3, columns of W1).
 __global__ __launch_bounds__(256) void mlp_bwd_kernel(const float *__restrict__ P, int64_t batch,
                                                       const float *__restrict__ x, const float *__restrict__ act,
                                                       const float *__restrict__ dy, float *__restrict__ part)
 {
-    __shared__ alignas(16) float DZ2[kRows][kPadH];
-    __shared__ alignas(16) float DZ1[kRows][kPadH];
-    __shared__ alignas(16) float H1[kRows][kPadH];
-    __shared__ alignas(16) float H2[kRows][kPadH];
-    __shared__ float DY[kRows][kOut];
-    __shared__ float X[kRows][kIn];
-    const int t = threadIdx.x;
+    __shared__ alignas(16) float DZ2[kBwdRows][kPadH];
+    __shared__ alignas(16) float W2[16][kPadH];      // rows 16 c ..
+    __shared__ alignas(16) float H1[kBwdRows][20], H2[kBwdRows][20], DZ1[kBwdRows][20];  // units 16 c ..
+    __shared__ float DY[kBwdRows][kOut], X[kBwdRows][kIn];
+    const int t = threadIdx.x, c = blockIdx.y;
     const int lane = t & 63, w = t >> 6, q = lane >> 4, n = lane & 15;
-    float b[16];  // W2^T's column 16 w + n: W2's row, at its columns 16 q + i
+    const int64_t r0 = (int64_t)blockIdx.x * kBwdRows;
+    const int r = t >> 2, j0 = (t & 3) * 16, u0 = (t & 3) * 4;
+    const int64_t row = r0 + r;
+    const bool live = row < batch;
+    // rows past the batch: zero activations and zero gradients
+    const float *ar = act + (live ? row : 0) * 256;
+    f32x4 z2[4];
 #pragma unroll
-    for (int i = 0; i < 16; i++) b[i] = P[kOffW2 + (16 * w + n) * kHid + 16 * q + i];
-    const int r = t >> 4;
-    const int j0 = (t & 15) * 4;
-    float w3[4][kOut];
+    for (int k = 0; k < 4; k++) z2[k] = *reinterpret_cast<const f32x4u *>(ar + 128 + j0 + 4 * k);
+    const f32x4 z1 = *reinterpret_cast<const f32x4u *>(ar + 16 * c + u0);
+    f32x4 h1 = *reinterpret_cast<const f32x4u *>(ar + 64 + 16 * c + u0);
+    f32x4 h2 = *reinterpret_cast<const f32x4u *>(ar + 192 + 16 * c + u0);
+    if (!live) h1 = h2 = f32x4{0, 0, 0, 0};
+    *reinterpret_cast<f32x4 *>(&W2[t >> 4][(t & 15) * 4]) =
+        *reinterpret_cast<const f32x4u *>(P + kOffW2 + (16 * c + (t >> 4)) * kHid + (t & 15) * 4);
+    if (t < kBwdRows * kOut) (&DY[0][0])[t] = (r0 * kOut + t < batch * kOut) ? dy[r0 * kOut + t] : 0.0f;
+    for (int k = t; k < kBwdRows * kIn; k += 256) (&X[0][0])[k] = (r0 * kIn + k < batch * kIn) ? x[r0 * kIn + k] : 0.0f;
+    *reinterpret_cast<f32x4 *>(&H1[r][u0]) = h1;
+    *reinterpret_cast<f32x4 *>(&H2[r][u0]) = h2;
+    __syncthreads();
+    // dz2 = (dy W3^T) * gelu'(z2), all 64 units
 #pragma unroll
-    for (int jj = 0; jj < 4; jj++)
+    for (int jj = 0; jj < 16; jj++) {
+        const int j = j0 + jj;
+        float dh = 0.0f;
 #pragma unroll
-        for (int o = 0; o < kOut; o++) w3[jj][o] = P[kOffW3 + (j0 + jj) * kOut + o];
-    f32x4 dw2[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};  // rows 16 w + 4 q + i, columns 16 jt + n
-    // the other gradients: unit u = t & 63 and a quarter of the sums each
-    const int u = t & 63;
-    float g1[2] = {0.0f, 0.0f}, g3[2] = {0.0f, 0.0f};
-    for (int64_t r0 = (int64_t)blockIdx.x * kRows; r0 < batch; r0 += (int64_t)gridDim.x * kRows) {
-        const int64_t row = r0 + r;
-        const bool live = row < batch;
-        __syncthreads();  // the previous group's readers are done
-        if (t < kRows * kOut) (&DY[0][0])[t] = (r0 * kOut + t < batch * kOut) ? dy[r0 * kOut + t] : 0.0f;
-        else if (t >= 64 && t < 64 + kRows * kIn)
-            (&X[0][0])[t - 64] = (r0 * kIn + t - 64 < batch * kIn) ? x[r0 * kIn + t - 64] : 0.0f;
-        // rows past the batch: zero activations and zero gradients
-        const f32x4u *ar = reinterpret_cast<const f32x4u *>(act + (live ? row : 0) * 256 + j0);
-        f32x4 z1 = ar[0], h1 = ar[16], z2 = ar[32], h2 = ar[48];
-        if (!live) z1 = h1 = z2 = h2 = f32x4{0, 0, 0, 0};
-        *reinterpret_cast<f32x4 *>(&H1[r][j0]) = h1;
-        *reinterpret_cast<f32x4 *>(&H2[r][j0]) = h2;
-        __syncthreads();
-        // dz2 = (dy W3^T) * gelu'(z2)
-#pragma unroll
-        for (int jj = 0; jj < 4; jj++) {
-            float dh = 0.0f;
-#pragma unroll
-            for (int o = 0; o < kOut; o++) dh += DY[r][o] * w3[jj][o];
-            DZ2[r][j0 + jj] = dh * gelu_grad(z2[jj]);
-            DZ1[r][j0 + jj] = gelu_grad(z1[jj]);
-        }
-        __syncthreads();
-        // dz1 = (dz2 W2^T) * gelu'(z1)
-        float a[16];
-        load16(&DZ2[n][16 * q], a);
-        const f32x4 d = mfma_k64(a, b);
-#pragma unroll
-        for (int i = 0; i < 4; i++) DZ1[4 * q + i][16 * w + n] *= d[i];
-        // dW2 = h1^T dz2 over the 16 rows (row 4 q + i at step i)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const float ha = H1[4 * q + i][16 * w + n];
-#pragma unroll
-            for (int jt = 0; jt < 4; jt++) dw2[jt] = mfma_f32(ha, DZ2[4 * q + i][16 * jt + n], dw2[jt]);
-        }
-        __syncthreads();
-        // dW1 (wave w: input w; wave 0 also input 4), db1, db2 (waves 1, 2),
-        // dW3 (wave w < 3: output w), db3 (wave 3, first lanes)
-        for (int rr = 0; rr < kRows; rr++) {
-            const float d1 = DZ1[rr][u];
-            g1[0] += X[rr][w] * d1;
-            if (w == 0) g1[1] += X[rr][4] * d1;
-            else if (w == 1) g1[1] += d1;
-            else if (w == 2) g1[1] += DZ2[rr][u];
-            if (w < kOut) g3[0] += H2[rr][u] * DY[rr][w];
-            else if (u < kOut) g3[0] += DY[rr][u];
-        }
+        for (int o = 0; o < kOut; o++) dh += DY[r][o] * P[kOffW3 + j * kOut + o];
+        DZ2[r][j] = live ? dh * gelu_grad(z2[jj >> 2][jj & 3]) : 0.0f;
     }
+#pragma unroll
+    for (int jj = 0; jj < 4; jj++) DZ1[r][u0 + jj] = live ? gelu_grad(z1[jj]) : 0.0f;
+    __syncthreads();
+    // dz1 = (dz2 W2^T) * gelu'(z1): wave w's rows 16 w .., columns the block's units
+    f32x4 d = {0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < 16; i++) d = mfma_f32(DZ2[16 * w + n][4 * i + q], W2[n][4 * i + q], d);
+    // dW2 = h1^T dz2: rows the block's units, wave w's columns 16 w ..
+    f32x4 g = {0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < 16; i++) g = mfma_f32(H1[4 * i + q][n], DZ2[4 * i + q][16 * w + n], g);
+#pragma unroll
+    for (int i = 0; i < 4; i++) DZ1[16 * w + 4 * q + i][n] *= d[i];
     float *pp = part + (int64_t)blockIdx.x * kNParams;
 #pragma unroll
-    for (int jt = 0; jt < 4; jt++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) pp[kOffW2 + (16 * w + 4 * q + i) * kHid + 16 * jt + n] = dw2[jt][i];
-    pp[kOffW1 + w * kHid + u] = g1[0];
-    if (w == 0) pp[kOffW1 + 4 * kHid + u] = g1[1];
-    else if (w == 1) pp[kOffB1 + u] = g1[1];
-    else if (w == 2) pp[kOffB2 + u] = g1[1];
-    if (w < kOut) pp[kOffW3 + u * kOut + w] = g3[0];
-    else if (u < kOut) pp[kOffB3 + u] = g3[0];
+    for (int i = 0; i < 4; i++) pp[kOffW2 + (16 * c + 4 * q + i) * kHid + 16 * w + n] = g[i];
+    __syncthreads();
+    // the rest, one output per thread: dW1 (80), db1, db2 (16 each), dW3 (48), db3 (3, by c = 0)
+    float s = 0.0f;
+    int out = -1;
+    if (t < 80) {
+        const int k = t >> 4, u = t & 15;
+        for (int rr = 0; rr < kBwdRows; rr++) s += X[rr][k] * DZ1[rr][u];
+        out = kOffW1 + k * kHid + 16 * c + u;
+    } else if (t < 96) {
+        for (int rr = 0; rr < kBwdRows; rr++) s += DZ1[rr][t - 80];
+        out = kOffB1 + 16 * c + t - 80;
+    } else if (t >= 128 && t < 144) {
+        for (int rr = 0; rr < kBwdRows; rr++) s += DZ2[rr][16 * c + t - 128];
+        out = kOffB2 + 16 * c + t - 128;
+    } else if (t >= 144 && t < 147 && c == 0) {
+        for (int rr = 0; rr < kBwdRows; rr++) s += DY[rr][t - 144];
+        out = kOffB3 + t - 144;
+    } else if (t >= 192 && t < 240) {
+        const int k = (t - 192) / kOut, o = (t - 192) % kOut;
+        for (int rr = 0; rr < kBwdRows; rr++) s += H2[rr][k] * DY[rr][o];
+        out = kOffW3 + (16 * c + k) * kOut + o;
+    }
+    if (out >= 0) pp[out] = s;
 }
 
-// 64 parameters per block, each of its 16 waves a sixteenth of the partials
-// (a thread per parameter over all partials: 8.6 us at 32 of them)
+// 64 parameters per block: its 16 waves load the partials side by side, the
+// first adds them in group order (a thread per parameter loading them one
+// after another: 8.6 us at 32 of them)
+constexpr int kReduceChunk = 128;
 __global__ __launch_bounds__(1024) void mlp_grad_reduce(const float *__restrict__ part, int nblocks,
                                                         float *__restrict__ grads)
 {
-    __shared__ float S[16][64];
+    __shared__ float S[kReduceChunk][64];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int e = blockIdx.x * 64 + lane;
     float s = 0.0f;
-    if (e < kNParams)
-        for (int b = w; b < nblocks; b += 16) s += part[(int64_t)b * kNParams + e];
-    S[w][lane] = s;
-    __syncthreads();
-    if (w == 0 && e < kNParams) {
-        for (int k = 1; k < 16; k++) s += S[k][lane];
-        grads[e] = s;
+    for (int b0 = 0; b0 < nblocks; b0 += kReduceChunk) {
+        const int m = nblocks - b0 < kReduceChunk ? nblocks - b0 : kReduceChunk;
+        if (e < kNParams)
+            for (int b = w; b < m; b += 16) S[b][lane] = part[(int64_t)(b0 + b) * kNParams + e];
+        __syncthreads();
+        if (w == 0 && e < kNParams)
+            for (int b = 0; b < m; b++) s += S[b][lane];
+        __syncthreads();
     }
+    if (w == 0 && e < kNParams) grads[e] = s;
 }
 
 __global__ __launch_bounds__(256) void mlp_adam_kernel(float *__restrict__ p, const float *__restrict__ gr,
@@ -1303,11 +1275,10 @@ int imogen_mlp_backward(const float *params, int64_t batch, const float *x, cons
     if (batch <= 0) return SUCCESSFUL;
     DeviceState *st = state();
     if (!st) return ERROR_CUDA_BLEW_UP;
-    int64_t blocks = (batch + kRows - 1) / kRows;
-    if (blocks > kBwdBlocks) blocks = kBwdBlocks;
+    const int64_t blocks = (batch + kBwdRows - 1) / kBwdRows;
     float *part = (float *)scratch_block((size_t)blocks * kNParams * sizeof(float));
     if (!part) return IM_FAIL(ERROR_NOMEM, "no scratch for gradient partials");
-    hipLaunchKernelGGL(mlp_bwd_kernel, dim3((unsigned)blocks), dim3(256), 0, st->stream, params, batch, x, act, dy,
+    hipLaunchKernelGGL(mlp_bwd_kernel, dim3((unsigned)blocks, 4), dim3(256), 0, st->stream, params, batch, x, act, dy,
                        part);
     int rc = IM_LAUNCHED("mlp_bwd_kernel");
     if (rc) return rc;
