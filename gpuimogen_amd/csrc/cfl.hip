@@ -112,32 +112,33 @@ int launch_soundspeed(const double *base, int64_t pitch, int64_t n, double gamma
     return IM_LAUNCHED("soundspeed_kernel");
 }
 
-// devOut[0] receives tau; devOut[1..] is used as block scratch (<= 2048 blocks).
+int launch_cfl_partials(const double *base, int64_t pitch, int64_t n, const double *cs, double gamma, int fused,
+                        int dim, int xinjin, double hx, double hy, double hz, double hmin, double *blockMin,
+                        int *nblocks, hipStream_t s)
+{
+    DeviceState *st = state();
+    if (!st) return ERROR_CUDA_BLEW_UP;
+    int64_t blocks = (n / 4 + 255) / 256;
+    if (blocks > kCflBlocks) blocks = kCflBlocks;
+    if (blocks < 1) blocks = 1;
+    if ((pitch & 1) || (((uintptr_t)base | (uintptr_t)cs) & 15))
+        return IM_FAIL(ERROR_INVALID_ARGS, "CFL needs 16-byte aligned slabs with an even pitch");
+    *nblocks = (int)blocks;
+    CflArgs a{gamma * (gamma - 1), hx, hy, hz, hmin, fused, dim, xinjin};
+    hipLaunchKernelGGL(cfl_pass1, dim3((unsigned)blocks), dim3(256), 0, s, base, pitch, n, cs, a, blockMin, st->err);
+    return IM_LAUNCHED("cfl_pass1");
+}
+
+// devOut[0] receives tau; devOut[8..] is used as block scratch (kCflBlocks).
 int launch_cfl(const double *base, int64_t pitch, int64_t n, const double *cs, double gamma, int fused,
                int dim, int xinjin, int halve, double hx, double hy, double hz, double hmin, double *devOut,
                hipStream_t s)
 {
-    DeviceState *st = state();
-    if (!st) return ERROR_CUDA_BLEW_UP;
-    unsigned long long *err = st->err;
-    int64_t blocks = (n / 4 + 255) / 256;
-    if (blocks > 2048) blocks = 2048;
-    if (blocks < 1) blocks = 1;
-    if ((pitch & 1) || (((uintptr_t)base | (uintptr_t)cs) & 15))
-        return IM_FAIL(ERROR_INVALID_ARGS, "CFL needs 16-byte aligned slabs with an even pitch");
-    double *blockMin = devOut + 8;
-    CflArgs a{gamma * (gamma - 1), hx, hy, hz, hmin, fused, dim, xinjin};
-    hipLaunchKernelGGL(cfl_pass1, dim3((unsigned)blocks), dim3(256), 0, s, base, pitch, n, cs, a, blockMin, err);
-    int rc = IM_LAUNCHED("cfl_pass1");
+    int blocks;
+    int rc = launch_cfl_partials(base, pitch, n, cs, gamma, fused, dim, xinjin, hx, hy, hz, hmin, devOut + 8,
+                                 &blocks, s);
     if (rc) return rc;
-    hipLaunchKernelGGL(cfl_pass2, dim3(1), dim3(256), 0, s, blockMin, (int)blocks, halve ? 1.0 : 0.0, devOut);
-    return IM_LAUNCHED("cfl_pass2");
-}
-
-int launch_cfl_final(const double *part, int64_t n, int halve, double *devOut, hipStream_t s)
-{
-    if (n < 1 || n > (int64_t)1 << 30) return IM_FAIL(ERROR_INVALID_ARGS, "CFL partial count %lld", (long long)n);
-    hipLaunchKernelGGL(cfl_pass2, dim3(1), dim3(256), 0, s, part, (int)n, halve ? 1.0 : 0.0, devOut);
+    hipLaunchKernelGGL(cfl_pass2, dim3(1), dim3(256), 0, s, devOut + 8, blocks, halve ? 1.0 : 0.0, devOut);
     return IM_LAUNCHED("cfl_pass2");
 }
 

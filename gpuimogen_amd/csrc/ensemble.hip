@@ -12,15 +12,13 @@
 // needs no host round trip and is captured once per sweep-order residue
 // (iteration mod 6) as a HIP graph and replayed.
 //
-// Work decomposition: X sweeps group problems by line length into the
-// register-blocking classes of the single-array X kernel (K cells per lane,
-// one launch per class, one wave per group of whole lines); Y sweeps use the
-// column march with columns cut into segments. Each fluid step has one X and
-// one Y sweep: the first goes from the pool to a second pool and the other
-// back, so neither has to leave cells for its neighbours and a problem's
-// segments fill waves of their own. Where the second pool does not fit the
-// device, the sweeps work in place (a column's segments in one wave).
-// The autotuner picks the segment counts per size class by timing the
+// Work decomposition: each fluid step has one X and one Y sweep. The first goes
+// from the pool to a second pool and the other back, so neither has to leave
+// cells for its neighbours: Y columns are cut into segments whose (segment,
+// column) pairs fill the lanes of a wave, X lines are swept whole or as two
+// halves with K cells per lane, one launch per K. The second pool is bounded; an
+// ensemble larger than it goes through it group by group. The autotuner picks
+// the segment counts per size class and K per line-length group by timing the
 // candidates on the ensemble itself.
 #include <algorithm>
 #include <cstring>
@@ -37,25 +35,26 @@ namespace imogen {
 // problems' gas; dusty problems add an entry for their dust.
 struct EnsProblem {
     double *q;
-    double *q2;     // the array's image in the second pool (q when there is none)
+    double *q2;     // the array's place in the second pool
     int64_t pitch;  // doubles between slabs
     int nx, ny;
     double hx, hy;
-    double gamma;
+    HydroConsts hc;
     int owner;  // problem whose clock and time step this entry follows
     int dust;   // gas entries: the entry of the problem's dust, -1 if none
     int fold;   // 1: the iteration's last sweep folds this entry's CFL minimum (fold_eligible)
     int pad;
 };
 
+// a wave's work: X: part b of c of line a, or (c = 0) the whole lines from a
+// on, periodic within their lanes; Y: 64 (segment, column) pairs from a on, of
+// b segments
 struct EnsItem {
-    int p;   // problem
-    int a;   // X: first line; Y: first column (in place) or first (segment, column) pair
-    int b;   // Y: segments S
-    int pad;
+    int p;  // entry
+    int a, b, c;
 };
 
-// which pool a sweep reads and writes (nothing to choose in place, q2 == q)
+// which pool a sweep reads and writes
 struct EnsSweep {
     const double *src;
     double *dst;
@@ -67,7 +66,6 @@ __device__ __forceinline__ EnsSweep ens_arrays(const EnsProblem &P, int fromSeco
 
 constexpr int kEnsCflBlocks = 32;  // CFL partial minima per problem
 constexpr int kEnsGhost = 4;       // ghost cells per face set by the boundary kernel
-constexpr double kEnsCflNone = 1e37;  // CFL minimum of an entry with no limiting cell
 
 // CFL minimum folded into the last sweep of an iteration. A problem without
 // dust whose sides both exceed 2 kEnsGhost cells ends its iteration with that
@@ -83,35 +81,19 @@ static bool fold_eligible(const EnsProblem &P, bool gas)
     return gas && P.dust < 0 && P.nx > 2 * kEnsGhost && P.ny > 2 * kEnsGhost;
 }
 
-// Order-preserving map of doubles (NaN aside) to unsigned 64-bit keys, so that
-// waves of any problem can take a problem's minimum with one integer atomic.
-__host__ __device__ inline unsigned long long ens_order_key(double v)
-{
-    unsigned long long b;
-    memcpy(&b, &v, sizeof b);
-    return (b >> 63) ? ~b : (b | 0x8000000000000000ull);
-}
-
-__device__ __forceinline__ double ens_order_value(unsigned long long k)
-{
-    const unsigned long long b = (k >> 63) ? (k & 0x7fffffffffffffffull) : ~k;
-    return __longlong_as_double((long long)b);
-}
-
 // Per-wave end of a folding sweep: the wave's minimum into its problem's slot
-// (lane values past the kept cells stay kEnsCflNone), NaN limits counted as
+// (lane values past the kept cells stay kCflNone), NaN limits counted as
 // the reduction pass counts them. All 64 lanes reach it.
 __device__ __forceinline__ void ens_fold_wave(double cmin, unsigned nan, unsigned long long *slot,
                                               unsigned long long *err)
 {
     wave_count(err + ERRW_CFL_NAN, nan);
     cmin = wave_min(cmin);
-    if ((threadIdx.x & 63) == 0 && cmin < kEnsCflNone) atomicMin(slot, ens_order_key(cmin));
+    if ((threadIdx.x & 63) == 0) fold_min(slot, cmin);
 }
 // X line classes: K cells per lane; lines of up to 256 cells are swept whole
-// (several short lines per wave), longer ones split into two halves swept by
-// a pair of waves (ens_sweep_xh)
-constexpr int kXClasses = 7;
+// (several short lines per wave), longer ones as two halves, a wave each
+constexpr int kXClasses = 7, kMaxK = 5;
 static const int kXClassK[kXClasses] = {1, 2, 3, 4, 3, 4, 5};
 static const bool kXClassSplit[kXClasses] = {false, false, false, false, true, true, true};
 
@@ -121,9 +103,9 @@ static int x_class_of(int N)
     if (N <= 128) return 1;
     if (N <= 192) return 2;
     if (N <= 256) return 3;
-    if (N <= 3 * 64 * 2 - 16) return 4;  // halves of <= 184 cells + 8 halo cells in 3-cell lanes
-    if (N <= 4 * 64 * 2 - 16) return 5;  // halves of <= 248 cells + 8 halo cells in 4-cell lanes
-    if (N <= 512) return 6;              // halves of <= 256 cells + 8 halo cells in 5-cell lanes
+    if (N <= 3 * 64 * 2 - 16) return 4;  // halves of <= 184 cells + 8 window cells in 3-cell lanes
+    if (N <= 4 * 64 * 2 - 16) return 5;  // halves of <= 248 cells + 8 window cells in 4-cell lanes
+    if (N <= 512) return 6;              // halves of <= 256 cells + 8 window cells in 5-cell lanes
     return -1;
 }
 
@@ -140,13 +122,22 @@ static int x_class_for(int N, int K, bool split)
     return K - 1;
 }
 
+// Waves per line: two halves, or one whose window holds the whole line and its
+// 4 periodic cells beyond each end (its lanes then need no select at the line's
+// end); 0: the lines fill their lanes (or share a wave) and wrap in them.
+static int x_parts(int N, int cls)
+{
+    if (kXClassSplit[cls]) return 2;
+    return (N > 32 * kXClassK[cls] && N + 8 <= 64 * kXClassK[cls]) ? 1 : 0;
+}
+
 // ---------------------------------------------------------------------------
 // kernels
 // ---------------------------------------------------------------------------
 // the CFL arguments of a 2D entry (cflTimestep.cu:292-335, fused sound speed)
 __device__ __forceinline__ CflArgs ens_cfl_args(const EnsProblem &P)
 {
-    return CflArgs{P.gamma * (P.gamma - 1), P.hx, P.hy, 1.0, P.hx < P.hy ? P.hx : P.hy, 1, 2, 0};
+    return CflArgs{P.hc.gamma * (P.hc.gamma - 1), P.hx, P.hy, 1.0, P.hx < P.hy ? P.hx : P.hy, 1, 2, 0};
 }
 
 // partial minima of the entries listed in `entries` (workgroups (block, list index))
@@ -158,7 +149,7 @@ __global__ __launch_bounds__(256) void ens_cfl_pass1(const EnsProblem *__restric
     const EnsProblem P = probs[ent];
     const int64_t n = (int64_t)P.nx * P.ny;
     const CflArgs a = ens_cfl_args(P);
-    double m = kEnsCflNone;
+    double m = kCflNone;
     unsigned nan = 0;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
         const double *c = P.q + i;
@@ -196,7 +187,7 @@ __global__ __launch_bounds__(64) void ens_cfl_pass2(const EnsProblem *__restrict
     // min over fluids of each fluid's halved limit, as TimeManager takes it
     double m = 1e38;
     if (useFold && probs[p].fold) {
-        m = ens_order_value(fold[p]);
+        m = order_value(fold[p]);
     } else {
         for (int k = threadIdx.x; k < nb; k += 64)
             m = (part[(int64_t)p * nb + k] < m) ? part[(int64_t)p * nb + k] : m;
@@ -224,16 +215,18 @@ __global__ __launch_bounds__(64) void ens_cfl_pass2(const EnsProblem *__restrict
         }
         dtp[p] = dt;
         clock[p] += 2 * dt;
-        fold[p] = ens_order_key(kEnsCflNone);
+        fold[p] = order_key(kCflNone);
     }
 }
 
 // the HLLC constants of an entry (launch_fluid_sweep's, from the entry's gamma)
-__device__ __forceinline__ HydroConsts ens_consts(double gamma)
+static HydroConsts ens_consts(double gamma)
 {
     HydroConsts hc;
     hc.gamma = gamma;
     hc.gm1 = gamma - 1.0;
+    hc.hgm1 = .5 * (gamma - 1.0);
+    hc.igm1 = 1.0 / (gamma - 1.0);
     hc.govergm1 = gamma / (gamma - 1.0);
     hc.rhomin = 0.0;
     hc.emin = 1e-5 / (gamma - 1.0);
@@ -242,153 +235,111 @@ __device__ __forceinline__ HydroConsts ens_consts(double gamma)
     return hc;
 }
 
-// X sweep of whole lines (K <= 4 cells per lane, two waves per SIMD); one
-// work item (problem, first line) per wave. CFL: fold the CFL minimum of the
-// output cells into fold[problem] (entries with P.fold set).
+// The wave's index in the launch, in a scalar register: its item and that
+// entry's record are then scalar loads (in vector registers the march spilled).
+__device__ __forceinline__ int ens_wave()
+{
+    return __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+}
+
+// X sweep with K cells per lane, one work item per wave. CFL: fold the CFL
+// minimum of the output cells into fold[problem] (entries with P.fold set).
 template <int K, int LIM, bool CFL>
 __global__ __launch_bounds__(256, 2) void ens_sweep_x(const EnsProblem *__restrict__ probs,
                                                    const EnsItem *__restrict__ work, int nwork, int fromSecond,
                                                    const double *__restrict__ lam, int rt,
-                                                   double *__restrict__ dummy, unsigned long long *__restrict__ fold,
+                                                   unsigned long long *__restrict__ fold,
                                                    unsigned long long *__restrict__ err)
 {
-    const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    const int wave = ens_wave();
     if (wave >= nwork) return;
-    const int lane = threadIdx.x & 63;
     const EnsItem it = work[wave];
-    const EnsProblem P = probs[it.p];
-    const HydroConsts hc = ens_consts(P.gamma);
+    const EnsProblem &P = probs[it.p];
+    const EnsSweep A = ens_arrays(P, fromSecond);
     const double lambda = lam[2 * it.p];
     const int N = P.nx;
-    const int nl = (N + K - 1) / K;
-    const int lpw = 64 / nl;
-    const int sub = lane / nl;
-    const int j = lane - sub * nl;
-    const int line = it.a + sub;
-    const bool own = sub < lpw && line < P.ny;
-    const int lbase = sub * nl;
-    const bool laneUsed = sub < lpw;
-    const int srcL = laneUsed ? lbase + (j == 0 ? nl - 1 : j - 1) : lane;
-    const int srcR = laneUsed ? lbase + (j == nl - 1 ? 0 : j + 1) : lane;
-    const int x0 = laneUsed ? j * K : 0;
-    int cnt = N - x0;
-    cnt = cnt < K ? cnt : K;
-    if (!laneUsed) cnt = 0;
-    const int lc = line < P.ny ? line : P.ny - 1;
-    const EnsSweep A = ens_arrays(P, fromSecond);
-    const double *b = A.src + (int64_t)lc * N + x0;
-    V5 Q[K];
-#pragma unroll
-    for (int k = 0; k < K; k++) Q[k] = (k < cnt) ? load_cell<Hllc, 1>(b + k, P.pitch) : V5{1.0, 1.0, 0.0, 0.0, 0.0};
-    V5 F[K], Fm;
-    x_fluxes<Hllc, K, LIM>(hc, rt, Q, cnt, srcL, srcR, F, Fm);
-    V5 U1[K];
-#pragma unroll
-    for (int k = 0; k < K; k++) U1[k] = axpy_update(Q[k], lambda, F[k], k == 0 ? Fm : F[k > 0 ? k - 1 : 0]);
-    x_fluxes<Hllc, K, LIM>(hc, rt, U1, cnt, srcL, srcR, F, Fm);
-    const int64_t gtid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t nthr = (int64_t)gridDim.x * blockDim.x;
-    double *dst = own ? A.dst + (int64_t)lc * N + x0 : dummy + gtid;
-    const int64_t st = own ? P.pitch : nthr;
-    const bool fl = CFL && own && P.fold;
-    const CflArgs ca = ens_cfl_args(P);
-    double cmin = kEnsCflNone;
+    const bool fl = CFL && P.fold;
+    const CflFuse cf{nullptr, ens_cfl_args(P), fl ? kEnsGhost : 0, fl ? N - kEnsGhost : 0};
+    double cmin = kCflNone;
     unsigned nan = 0;
+    if (it.c) {
+        const int64_t row = (int64_t)it.a * N;
+        xp_body<Hllc, K, LIM, CFL>(A.src + row, A.dst + row, P.pitch, N, it.b, it.c, true, false, lambda, P.hc, rt,
+                                   cf, cmin, nan);
+    } else if (K <= 4) {
+        const int lane = threadIdx.x & 63;
+        const int nl = (N + K - 1) / K;
+        const int lpw = 64 / nl;
+        const int sub = lane / nl;
+        const int j = lane - sub * nl;
+        const int line = it.a + sub;
+        const bool used = sub < lpw;
+        const bool own = used && line < P.ny;
+        const int x0 = used ? j * K : 0;
+        int cnt = N - x0;
+        cnt = cnt < K ? cnt : K;
+        if (!used) cnt = 0;
+        const int64_t off = (int64_t)(line < P.ny ? line : P.ny - 1) * N + x0;
+        V5 Q[K];
 #pragma unroll
-    for (int k = 0; k < K; k++) {
-        if (k < cnt) {
-            const V5 o = avg_update(add5(U1[k], Q[k]), lambda, F[k], k == 0 ? Fm : F[k > 0 ? k - 1 : 0]);
-            store_cell<Hllc, 1>(own ? dst + k : dst, st, o);
-            if (fl && x0 + k >= kEnsGhost && x0 + k < N - kEnsGhost) {
-                const double u = cfl_of_cell<Hllc, 1>(ca, o);
-                cmin = (u < cmin) ? u : cmin;
-                nan += (u != u);
+        for (int k = 0; k < K; k++)
+            Q[k] = (k < cnt) ? load_cell<Hllc, 1>(A.src + off + k, P.pitch) : V5{1.0, 1.0, 0.0, 0.0, 0.0};
+        const int first = sub * nl;
+        x_stages<Hllc, K, LIM>(P.hc, rt, Q, cnt, used ? first + (j == 0 ? nl - 1 : j - 1) : lane,
+                               used ? first + (j == nl - 1 ? 0 : j + 1) : lane, lambda);
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            if (own && k < cnt) {
+                store_cell<Hllc, 1>(A.dst + off + k, P.pitch, Q[k]);
+                if (CFL && x0 + k >= cf.lo && x0 + k < cf.hi) {
+                    const double u = cfl_of_cell<Hllc, 1>(cf.a, Q[k]);
+                    cmin = (u < cmin) ? u : cmin;
+                    nan += (u != u);
+                }
             }
         }
     }
     if (CFL) ens_fold_wave(cmin, nan, fold + P.owner, err);
 }
 
-// X sweep of lines split into two halves, one wave per half (xp_body). The two
-// waves of a line are in one workgroup (4 waves: 2 lines), as the in-place form
-// needs. One work item (problem, line) per wave pair; lines of at most
-// 2 (64 K - 8) cells.
-template <int K, int LIM, bool CFL>
-__global__ __launch_bounds__(256, 2) void ens_sweep_xh(const EnsProblem *__restrict__ probs,
-                                                    const EnsItem *__restrict__ work, int nwork, int fromSecond,
-                                                    const double *__restrict__ lam, int rt,
-                                                    unsigned long long *__restrict__ fold,
-                                                    unsigned long long *__restrict__ err)
-{
-    const int wib = threadIdx.x >> 6;
-    int item = (int)blockIdx.x * 2 + (wib >> 1);
-    const bool itemValid = item < nwork;
-    item = itemValid ? item : nwork - 1;  // waves past the list still meet the barrier
-    const EnsItem it = work[item];
-    const EnsProblem P = probs[it.p];
-    const EnsSweep A = ens_arrays(P, fromSecond);
-    const int64_t row = (int64_t)it.a * P.nx;
-    const bool fl = CFL && P.fold;
-    const CflFuse cf{nullptr, ens_cfl_args(P), fl ? kEnsGhost : 0, fl ? P.nx - kEnsGhost : 0, 0};
-    double cmin = kEnsCflNone;
-    unsigned nan = 0;
-    xp_body<Hllc, K, LIM, CFL>(A.src + row, A.dst + row, P.pitch, P.nx, wib & 1, 2, itemValid, A.src == A.dst,
-                               lam[2 * it.p], ens_consts(P.gamma), rt, cf, cmin, nan);
-    if (CFL) ens_fold_wave(cmin, nan, fold + P.owner, err);
-}
-
-// workgroups of an X class launch over n work items
-static int64_t x_blocks(int cls, int64_t n)
-{
-    return kXClassSplit[cls] ? (n + 1) / 2 : (n + 3) / 4;
-}
-
-// Y sweep: column march, one work item per wave. In place (problem, first
-// column, S): 64/S columns, their S segments side by side in the lanes.
-// Otherwise (problem, first pair, S): 64 of the problem's (segment, column)
-// pairs, numbered segment * nx + column, so all lanes but the last wave's
-// carry one (short problems leave none idle past their last column).
+// Y sweep: column march, one work item per wave: 64 of the entry's (segment,
+// column) pairs, numbered segment * nx + column, so all lanes but the last
+// wave's carry one (a wave of 64 columns leaves lanes past the last column).
 template <int LIM, bool CFL>
-__global__ __launch_bounds__(256) void ens_sweep_y(const EnsProblem *__restrict__ probs,
+__global__ __launch_bounds__(256, 2) void ens_sweep_y(const EnsProblem *__restrict__ probs,
                                                    const EnsItem *__restrict__ work, int nwork, int fromSecond,
                                                    const double *__restrict__ lam, int rt,
-                                                   double *__restrict__ defer, unsigned long long *__restrict__ fold,
+                                                   double *__restrict__ dummy, unsigned long long *__restrict__ fold,
                                                    unsigned long long *__restrict__ err)
 {
     __shared__ double sring[4][4][5][64];
-    const int wib = threadIdx.x >> 6;
-    const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    const int wave = ens_wave();
     if (wave >= nwork) return;
     const int lane = threadIdx.x & 63;
     const EnsItem it = work[wave];
-    const EnsProblem P = probs[it.p];
+    const EnsProblem &P = probs[it.p];
     const EnsSweep A = ens_arrays(P, fromSecond);
-    const bool inplace = A.src == A.dst;
-    const HydroConsts hc = ens_consts(P.gamma);
     const double lambda = lam[2 * it.p + 1];
     const int S = it.b;
-    const int W = inplace ? 64 / S : P.nx;
-    const int id = (inplace ? 0 : it.a) + lane;
-    const int s = id / W;
-    const int x = (inplace ? it.a : 0) + id % W;
-    const bool colValid = (x < P.nx) && (s < S);
+    const int s = (it.a + lane) / P.nx;
+    const int x = (it.a + lane) - s * P.nx;
+    const bool valid = s < S;
     const int N = P.ny;
     const int seglen = (N + S - 1) / S;
-    const int j0 = colValid ? s * seglen : 0;  // lanes of no column: zero-length segment at row 0
+    const int j0 = valid ? s * seglen : 0;  // lanes of no pair: zero-length segment at row 0
     int L = N - j0;
     L = L < seglen ? L : seglen;
-    if (!colValid || L < 0) L = 0;
-    const int off = colValid ? x : 0;
+    if (!valid) L = 0;
+    const int off = valid ? x : 0;
     const int64_t gtid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t nthr = (int64_t)gridDim.x * blockDim.x;
     // cells [kEnsGhost, N - kEnsGhost) of the column fold their CFL limits
     const bool fl = CFL && P.fold;
-    const CflFuse cf{nullptr, ens_cfl_args(P), fl ? kEnsGhost : 0, fl ? N - kEnsGhost : 0, 0};
-    double cmin = kEnsCflNone;
+    const CflFuse cf{nullptr, ens_cfl_args(P), fl ? kEnsGhost : 0, fl ? N - kEnsGhost : 0};
+    double cmin = kCflNone;
     unsigned nan = 0;
-    march_body<Hllc, 2, LIM, CFL>(A.src + off, A.dst + off, P.pitch, (int64_t)P.nx, N, seglen, j0, L,
-                                  inplace ? 4 : 0, lambda, hc, rt, defer, gtid, nthr, sring[wib], lane, cf, cmin,
-                                  nan);
+    march_body<Hllc, 2, LIM, CFL>(A.src + off, A.dst + off, P.pitch, (int64_t)P.nx, N, seglen, j0, L, 0, lambda,
+                                  P.hc, rt, dummy, gtid, nthr, sring[wave & 3], lane, cf, cmin, nan);
     if (CFL) ens_fold_wave(cmin, nan, fold + P.owner, err);
 }
 
@@ -401,10 +352,10 @@ __global__ __launch_bounds__(256) void ens_sweep_y(const EnsProblem *__restrict_
 // its boundaries (flux.cu:99-107, the swept direction rotated into memory x);
 // 0: the y kernel's innermost-ghost copy (cudaStatics.cu:1461-1466), as
 // src0001.m's boundary calls on unrotated arrays
-__global__ __launch_bounds__(256) void ens_bc_const(const EnsProblem *__restrict__ probs, int second, int dir, int d,
-                                                    int xrules)
+__global__ __launch_bounds__(256) void ens_bc_const(const EnsProblem *__restrict__ probs, int first, int second,
+                                                    int dir, int d, int xrules)
 {
-    const EnsProblem P = probs[blockIdx.x];
+    const EnsProblem P = probs[first + blockIdx.x];
     double *q = second ? P.q2 : P.q;
     const int nx = P.nx, ny = P.ny;
     const int N = (dir == 1) ? nx : ny;
@@ -461,16 +412,27 @@ __global__ __launch_bounds__(256) void ens_bc_const(const EnsProblem *__restrict
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
+// Entries [e0, e1) that go through the second pool together, and their part of
+// the work lists.
+struct EnsGroup {
+    int e0, e1;
+    int x0[kMaxK], nx[kMaxK];  // X items by K - 1
+    int y0, ny;
+};
+
+// Bytes of the second pool (or the largest problem's, if that is more).
+constexpr int64_t kSecondPool = (int64_t)1 << 30;
+
 struct EnsembleImpl {
     int P = 0;   // problems (gas entries 0..P-1)
     int NE = 0;  // table entries: gas, then the dusty problems' dust
     double gamma = 1.4, cfl = 0.4;
     int limiter = 0;
     std::vector<EnsProblem> host;
-    std::vector<int> segS;  // Y segments per problem: the count (in place) or a factor on the base count
+    std::vector<int> segS;  // factor on the Y segment count per problem
     std::vector<int> xcls;  // X line class per problem (x_class_of unless tuned)
-    double *pool = nullptr, *pool2 = nullptr;  // pool2: the sweeps' second arrays (null: in place)
-    int segLen = 64;  // cells per Y segment the base counts aim at (second pool)
+    double *pool = nullptr, *pool2 = nullptr;
+    std::vector<EnsGroup> groups;
     EnsProblem *dprobs = nullptr;
     double *lam = nullptr, *clock = nullptr, *cflPart = nullptr;
     // folded CFL minima (one key per problem) and the entries the reduction
@@ -478,22 +440,18 @@ struct EnsembleImpl {
     unsigned long long *fold = nullptr;
     int *cflList = nullptr;
     int nNoFold = 0;
-    EnsItem *xwork[kXClasses] = {nullptr};
-    int nx_work[kXClasses] = {0};
-    EnsItem *ywork = nullptr;
-    int ny_work = 0;
-    double *xdummy = nullptr, *ydefer = nullptr;
-    int64_t xThreads = 0, yThreads = 0;
-    int64_t xcells[kXClasses] = {0};  // cells of each X line class (the stream balance)
-    // The X line classes sweep disjoint lines: their launches fork onto these
-    // streams (default priority) and join back, parallel branches of the graph
+    EnsItem *work = nullptr;    // every group's X items, then every group's Y items
+    double *ydummy = nullptr;   // 5 doubles per thread of the largest Y launch
+    int64_t yThreads = 0;
+    // The X launches of one sweep (a K each) go to disjoint lines: they fork onto
+    // these streams (default priority) and join back, parallel branches of the graph
     hipStream_t side[2] = {nullptr, nullptr};
     hipEvent_t fork = nullptr, join[2] = {nullptr, nullptr};
     hipGraphExec_t graph[2][6] = {{nullptr}};  // [reduction reads the folded minima][sweep order]
     int64_t cells = 0;
     // dust (imogen_ensemble_set_dust)
     int Pd = 0;
-    double *dpool = nullptr, *dpool2 = nullptr, *dtp = nullptr;
+    double *dpool = nullptr, *dtp = nullptr;
     EnsDragTable *dragTab = nullptr;
     EnsDragItem *dragItems = nullptr;
     int nDragItems = 0;
@@ -514,31 +472,30 @@ static void free_graphs(EnsembleImpl *e)
         }
 }
 
-// segments of entry k's columns: the chosen count in place, or the chosen
-// factor times the count that cuts them into about segLen cells
-static int y_segments(const EnsembleImpl *e, int k)
+// Segments of entry k's columns: the chosen factor times the count that cuts
+// them into about segLen cells.
+static int y_segments(const EnsembleImpl *e, int k, int segLen)
 {
     const EnsProblem &P = e->host[k];
-    int S = e->segS[P.owner];
-    if (!e->pool2) return S;
-    S *= (P.ny + e->segLen - 1) / e->segLen;
+    int S = e->segS[P.owner] * ((P.ny + segLen - 1) / segLen);
     S = std::min(S, std::max(1, P.ny / 4));
     const int len = (P.ny + S - 1) / S;
     return (P.ny + len - 1) / len;  // no empty segment
 }
 
-// Cells per segment of the out-of-place Y march: with w waves of L cells the
-// launch takes about (w / 1024 + 1/2) (L + 9) steps (the waves go to the SIMDs
-// longest first; the last one's steps are half hidden), a wave's steps taking
-// their issue time however many share a SIMD. 60 problems of 64..512 cells
-// (3.7 M): 339 us per launch with up to 2 segments per column in place.
-static int ens_segment_cells(const EnsembleImpl *e)
+// Cells per Y segment of a group: with w waves of L cells the launch takes
+// about (w / 1024 + 1/2) (L + 9) steps (the waves go to the SIMDs longest
+// first; the last one's steps are half hidden), a wave's steps taking their
+// issue time however many share a SIMD. 60 problems of 64..512 cells (3.7 M):
+// 106 us per launch, 339 with up to 2 segments per column, in place.
+static int segment_cells(const EnsembleImpl *e, const EnsGroup &g)
 {
     int best = 8;
     double bestCost = 0.0;
     for (int L = 8; L <= 512; L += (L < 64 ? 4 : 16)) {
         int64_t waves = 0;
-        for (const EnsProblem &P : e->host) waves += ((int64_t)P.nx * ((P.ny + L - 1) / L) + 63) / 64;
+        for (int k = g.e0; k < g.e1; k++)
+            waves += ((int64_t)e->host[k].nx * ((e->host[k].ny + L - 1) / L) + 63) / 64;
         const double cost = std::max(1.0, waves / 1024.0 + 0.5) * (L + 9);
         if (L == 8 || cost < bestCost) {
             best = L;
@@ -546,6 +503,39 @@ static int ens_segment_cells(const EnsembleImpl *e)
         }
     }
     return best;
+}
+
+// Groups of consecutive entries that fit the second pool; every entry's place
+// in it, and the size (doubles) it needs.
+static int64_t make_groups(EnsembleImpl *e)
+{
+    e->groups.clear();
+    int64_t size = 0, at = 0;
+    for (int p = 0; p < e->NE; p++) {
+        const int64_t n = 5 * e->host[p].pitch;
+        if (e->groups.empty() || (at + n) * (int64_t)sizeof(double) > kSecondPool) {
+            EnsGroup g{};
+            g.e0 = p;
+            e->groups.push_back(g);
+            at = 0;
+        }
+        e->host[p].q2 = e->pool2 + at;  // rebased once the pool is there
+        at += n;
+        size = std::max(size, at);
+        e->groups.back().e1 = p + 1;
+    }
+    return size;
+}
+
+// (Re)allocates the second pool for the present entries.
+static int second_pool(EnsembleImpl *e)
+{
+    if (e->pool2) (void)hipFree(e->pool2);
+    e->pool2 = nullptr;
+    const int64_t size = make_groups(e);
+    if (IM_HIP(hipMalloc(&e->pool2, (size_t)size * sizeof(double)))) return ERROR_CUDA_BLEW_UP;
+    (void)make_groups(e);
+    return SUCCESSFUL;
 }
 
 static int build_work(EnsembleImpl *e)
@@ -571,64 +561,58 @@ static int build_work(EnsembleImpl *e)
     if (IM_HIP(hipMalloc(&e->cflList, cl.size() * sizeof(int)))) return ERROR_CUDA_BLEW_UP;
     if (IM_HIP(hipMemcpy(e->cflList, cl.data(), cl.size() * sizeof(int), hipMemcpyHostToDevice)))
         return ERROR_CUDA_BLEW_UP;
-    std::vector<EnsItem> xw[kXClasses], yw;
-    e->segLen = ens_segment_cells(e);
-    for (int c = 0; c < kXClasses; c++) e->xcells[c] = 0;
-    for (int p = 0; p < e->NE; p++) {
-        const EnsProblem &P = e->host[p];
-        const int cls = e->xcls[P.owner];
-        const int K = kXClassK[cls];
-        const int nl = (P.nx + K - 1) / K;
-        const int lpw = kXClassSplit[cls] ? 1 : 64 / nl;  // split classes: one item per line
-        for (int l = 0; l < P.ny; l += lpw) xw[cls].push_back(EnsItem{p, l, 0, 0});
-        e->xcells[cls] += (int64_t)P.nx * P.ny;
-        const int S = y_segments(e, p);
-        if (e->pool2)
-            for (int id = 0; id < P.nx * S; id += 64) yw.push_back(EnsItem{p, id, S, 0});
-        else
-            for (int x = 0; x < P.nx; x += 64 / S) yw.push_back(EnsItem{p, x, S, 0});
+    std::vector<EnsItem> w;
+    for (EnsGroup &g : e->groups) {
+        for (int K = 1; K <= kMaxK; K++) {
+            g.x0[K - 1] = (int)w.size();
+            for (int p = g.e0; p < g.e1; p++) {
+                const EnsProblem &P = e->host[p];
+                const int cls = e->xcls[P.owner];
+                if (kXClassK[cls] != K) continue;
+                const int parts = x_parts(P.nx, cls);
+                const int lines = parts ? 1 : 64 / ((P.nx + K - 1) / K);
+                for (int l = 0; l < P.ny; l += lines)
+                    for (int k = 0; k < std::max(1, parts); k++) w.push_back(EnsItem{p, l, k, parts});
+            }
+            g.nx[K - 1] = (int)w.size() - g.x0[K - 1];
+        }
     }
-    for (int c = 0; c < kXClasses; c++) {
-        std::stable_sort(xw[c].begin(), xw[c].end(),
-                         [e](const EnsItem &a, const EnsItem &b) { return e->host[a.p].nx > e->host[b.p].nx; });
-        if (e->xwork[c]) (void)hipFree(e->xwork[c]);
-        e->xwork[c] = nullptr;
-        e->nx_work[c] = (int)xw[c].size();
-        if (xw[c].empty()) continue;
-        if (IM_HIP(hipMalloc(&e->xwork[c], xw[c].size() * sizeof(EnsItem)))) return ERROR_CUDA_BLEW_UP;
-        if (IM_HIP(hipMemcpy(e->xwork[c], xw[c].data(), xw[c].size() * sizeof(EnsItem), hipMemcpyHostToDevice)))
-            return ERROR_CUDA_BLEW_UP;
+    int64_t yt = 0;
+    for (EnsGroup &g : e->groups) {
+        g.y0 = (int)w.size();
+        const int segLen = segment_cells(e, g);
+        for (int p = g.e0; p < g.e1; p++) {
+            const int S = y_segments(e, p, segLen);
+            for (int id = 0; id < e->host[p].nx * S; id += 64) w.push_back(EnsItem{p, id, S, 0});
+        }
+        g.ny = (int)w.size() - g.y0;
+        // longest marches first, so that the short ones fill in behind them
+        std::stable_sort(w.begin() + g.y0, w.end(), [e](const EnsItem &a, const EnsItem &b) {
+            return (e->host[a.p].ny + a.b - 1) / a.b > (e->host[b.p].ny + b.b - 1) / b.b;
+        });
+        yt = std::max<int64_t>(yt, ((int64_t)g.ny + 3) / 4 * 256);
     }
-    // longest marches first, so that the short ones fill in behind them
-    std::stable_sort(yw.begin(), yw.end(), [e](const EnsItem &a, const EnsItem &b) {
-        return (e->host[a.p].ny + a.b - 1) / a.b > (e->host[b.p].ny + b.b - 1) / b.b;
-    });
-    if (e->ywork) (void)hipFree(e->ywork);
-    e->ny_work = (int)yw.size();
-    if (IM_HIP(hipMalloc(&e->ywork, yw.size() * sizeof(EnsItem)))) return ERROR_CUDA_BLEW_UP;
-    if (IM_HIP(hipMemcpy(e->ywork, yw.data(), yw.size() * sizeof(EnsItem), hipMemcpyHostToDevice)))
+    if (e->work) (void)hipFree(e->work);
+    e->work = nullptr;
+    if (IM_HIP(hipMalloc(&e->work, w.size() * sizeof(EnsItem)))) return ERROR_CUDA_BLEW_UP;
+    if (IM_HIP(hipMemcpy(e->work, w.data(), w.size() * sizeof(EnsItem), hipMemcpyHostToDevice)))
         return ERROR_CUDA_BLEW_UP;
-    // per-lane scratch: X dummy slots (5 doubles), Y deferred outputs (25 doubles)
-    int64_t xt = 0;
-    for (int c = 0; c < kXClasses; c++) xt = std::max<int64_t>(xt, x_blocks(c, e->nx_work[c]) * 256);
-    const int64_t yt = (((int64_t)e->ny_work + 3) / 4) * 256;
-    if (xt > e->xThreads) {
-        if (e->xdummy) (void)hipFree(e->xdummy);
-        if (IM_HIP(hipMalloc(&e->xdummy, (size_t)xt * 5 * sizeof(double)))) return ERROR_CUDA_BLEW_UP;
-        e->xThreads = xt;
-    }
     if (yt > e->yThreads) {
-        if (e->ydefer) (void)hipFree(e->ydefer);
-        if (IM_HIP(hipMalloc(&e->ydefer, (size_t)yt * 25 * sizeof(double)))) return ERROR_CUDA_BLEW_UP;
+        if (e->ydummy) (void)hipFree(e->ydummy);
+        e->ydummy = nullptr;
+        e->yThreads = 0;
+        if (IM_HIP(hipMalloc(&e->ydummy, (size_t)yt * 5 * sizeof(double)))) return ERROR_CUDA_BLEW_UP;
         e->yThreads = yt;
     }
     free_graphs(e);
     return SUCCESSFUL;
 }
 
-static int ens_bc(EnsembleImpl *e, int second, int dir, hipStream_t s, int xrules)
+// const boundaries of entries [e0, e1), in the pool or the second one
+static int ens_bc(EnsembleImpl *e, int e0, int e1, int second, int dir, hipStream_t s, int xrules)
 {
-    hipLaunchKernelGGL(ens_bc_const, dim3((unsigned)e->NE, 16), dim3(256), 0, s, e->dprobs, second, dir, 4, xrules);
+    hipLaunchKernelGGL(ens_bc_const, dim3((unsigned)(e1 - e0), 16), dim3(256), 0, s, e->dprobs, e0, second, dir, 4,
+                       xrules);
     return IM_LAUNCHED("ens_bc_const");
 }
 
@@ -642,81 +626,72 @@ static int ens_source(EnsembleImpl *e, double fraction, hipStream_t s)
                              e->dragMethod, e->queue, e->qcount, s, 2);
     if (rc) return rc;
     for (int d = 1; d <= 2; d++) {
-        rc = ens_bc(e, 0, d, s, 0);
+        rc = ens_bc(e, 0, e->NE, 0, d, s, 0);
         if (rc) return rc;
     }
     return SUCCESSFUL;
 }
 
-// one sweep of every entry in direction dir, from the pool to the second one
-// or (fromSecond) back, then that direction's boundaries; CFL: the sweep folds
-// the CFL minima of the entries that fold
+// one sweep of a group's entries in direction dir, from the pool to the second
+// one or (fromSecond) back, then that direction's boundaries; CFL: the sweep
+// folds the CFL minima of the entries that fold
 template <int LIM, bool CFL>
-static int ens_sweep(EnsembleImpl *e, int dir, int fromSecond, int rt, hipStream_t s)
+static int ens_sweep(EnsembleImpl *e, const EnsGroup &g, int dir, int fromSecond, int rt, hipStream_t s)
 {
     unsigned long long *err = state()->err;
+    const dim3 block(256);
+    int rc;
     if (dir == 1) {
-        // classes to the three streams, largest first to the least loaded
-        int order[kXClasses], nc = 0;
-        for (int c = 0; c < kXClasses; c++)
-            if (e->nx_work[c]) order[nc++] = c;
-        std::sort(order, order + nc, [e](int a, int b) { return e->xcells[a] > e->xcells[b]; });
+        // largest launches first, each to the least loaded of the three streams
+        int order[kMaxK], nk = 0;
+        for (int k = 0; k < kMaxK; k++)
+            if (g.nx[k]) order[nk++] = k;
+        std::sort(order, order + nk, [&g](int a, int b) { return g.nx[a] * (a + 1) > g.nx[b] * (b + 1); });
         int64_t load[3] = {0, 0, 0};
-        if (IM_HIP(hipEventRecord(e->fork, s))) return ERROR_CUDA_BLEW_UP;
-        for (int k = 0; k < 2; k++)
+        const int forks = std::min(nk, 3) - 1;
+        if (forks > 0 && IM_HIP(hipEventRecord(e->fork, s))) return ERROR_CUDA_BLEW_UP;
+        for (int k = 0; k < forks; k++)
             if (IM_HIP(hipStreamWaitEvent(e->side[k], e->fork, 0))) return ERROR_CUDA_BLEW_UP;
-        for (int i = 0; i < nc; i++) {
-            const int c = order[i];
-            const int sl = (int)(std::min_element(load, load + 3) - load);
-            load[sl] += e->xcells[c];
+        for (int i = 0; i < nk; i++) {
+            const int k = order[i], n = g.nx[k];
+            const int sl = (int)(std::min_element(load, load + forks + 1) - load);
+            load[sl] += (int64_t)n * (k + 1);
             hipStream_t sx = sl == 0 ? s : e->side[sl - 1];
-            const unsigned blocks = (unsigned)x_blocks(c, e->nx_work[c]);
+            const dim3 grid((unsigned)((n + 3) / 4));
 #define IM_EX(KK)                                                                                              \
-    hipLaunchKernelGGL((ens_sweep_x<KK, LIM, CFL>), dim3(blocks), dim3(256), 0, sx, e->dprobs, e->xwork[c],     \
-                       e->nx_work[c], fromSecond, e->lam, rt, e->xdummy, e->fold, err)
-#define IM_EXH(KK)                                                                                             \
-    hipLaunchKernelGGL((ens_sweep_xh<KK, LIM, CFL>), dim3(blocks), dim3(256), 0, sx, e->dprobs, e->xwork[c],    \
-                       e->nx_work[c], fromSecond, e->lam, rt, e->fold, err)
-            if (kXClassSplit[c]) {
-                switch (kXClassK[c]) {
-                case 3: IM_EXH(3); break;
-                case 4: IM_EXH(4); break;
-                case 5: IM_EXH(5); break;
-                }
-            } else {
-                switch (kXClassK[c]) {
-                case 1: IM_EX(1); break;
-                case 2: IM_EX(2); break;
-                case 3: IM_EX(3); break;
-                case 4: IM_EX(4); break;
-                }
+    case KK - 1:                                                                                               \
+        hipLaunchKernelGGL((ens_sweep_x<KK, LIM, CFL>), grid, block, 0, sx, e->dprobs, e->work + g.x0[k], n,   \
+                           fromSecond, e->lam, rt, e->fold, err);                                              \
+        break;
+            switch (k) {
+                IM_EX(1)
+                IM_EX(2)
+                IM_EX(3)
+                IM_EX(4)
+                IM_EX(5)
             }
 #undef IM_EX
-#undef IM_EXH
-            int rc = IM_LAUNCHED("ens_sweep_x");
-            if (rc) return rc;
+            if ((rc = IM_LAUNCHED("ens_sweep_x"))) return rc;
         }
-        for (int k = 0; k < 2; k++) {
+        for (int k = 0; k < forks; k++) {
             if (IM_HIP(hipEventRecord(e->join[k], e->side[k]))) return ERROR_CUDA_BLEW_UP;
             if (IM_HIP(hipStreamWaitEvent(s, e->join[k], 0))) return ERROR_CUDA_BLEW_UP;
         }
     } else {
-        const unsigned blocks = (unsigned)((e->ny_work + 3) / 4);
-        hipLaunchKernelGGL((ens_sweep_y<LIM, CFL>), dim3(blocks), dim3(256), 0, s, e->dprobs, e->ywork,
-                           e->ny_work, fromSecond, e->lam, rt, e->ydefer, e->fold, err);
-        int rc = IM_LAUNCHED("ens_sweep_y");
-        if (rc) return rc;
+        hipLaunchKernelGGL((ens_sweep_y<LIM, CFL>), dim3((unsigned)((g.ny + 3) / 4)), block, 0, s, e->dprobs,
+                           e->work + g.y0, g.ny, fromSecond, e->lam, rt, e->ydummy, e->fold, err);
+        if ((rc = IM_LAUNCHED("ens_sweep_y"))) return rc;
     }
-    return ens_bc(e, !fromSecond, dir, s, 1);
+    return ens_bc(e, g.e0, g.e1, !fromSecond, dir, s, 1);
 }
 
 template <bool CFL>
-static int ens_sweep_lim(EnsembleImpl *e, int dir, int fromSecond, hipStream_t s)
+static int ens_sweep_lim(EnsembleImpl *e, const EnsGroup &g, int dir, int fromSecond, hipStream_t s)
 {
     switch (e->limiter) {
-    case LIMITER_OSPRE: return ens_sweep<0, CFL>(e, dir, fromSecond, 0, s);
-    case LIMITER_VANLEER: return ens_sweep<1, CFL>(e, dir, fromSecond, 1, s);
-    default: return ens_sweep<-1, CFL>(e, dir, fromSecond, e->limiter, s);
+    case LIMITER_OSPRE: return ens_sweep<0, CFL>(e, g, dir, fromSecond, 0, s);
+    case LIMITER_VANLEER: return ens_sweep<1, CFL>(e, g, dir, fromSecond, 1, s);
+    default: return ens_sweep<-1, CFL>(e, g, dir, fromSecond, e->limiter, s);
     }
 }
 
@@ -747,14 +722,16 @@ static int ens_iteration(EnsembleImpl *e, int it, hipStream_t s, bool useFold)
         int last = 0;
         for (int n = 0; n < 3; n++)
             if (kFluxcall[n][sweep] != 3) last = n;
-        int fromSecond = 0;  // the step's first sweep leaves the pool, its other one returns
-        for (int n = 0; n < 3; n++) {
-            const int d = kFluxcall[n][sweep];
-            if (d == 3) continue;  // 2D problems
-            rc = (dirn < 0 && n == last) ? ens_sweep_lim<true>(e, d, fromSecond, s)
-                                         : ens_sweep_lim<false>(e, d, fromSecond, s);
-            if (rc) return rc;
-            fromSecond = !fromSecond;
+        for (const EnsGroup &g : e->groups) {
+            int fromSecond = 0;  // the step's first sweep leaves the pool, its other one returns
+            for (int n = 0; n < 3; n++) {
+                const int d = kFluxcall[n][sweep];
+                if (d == 3) continue;  // 2D problems
+                rc = (dirn < 0 && n == last) ? ens_sweep_lim<true>(e, g, d, fromSecond, s)
+                                             : ens_sweep_lim<false>(e, g, d, fromSecond, s);
+                if (rc) return rc;
+                fromSecond = !fromSecond;
+            }
         }
         if ((rc = ens_source(e, dirn > 0 ? 1.0 : 0.5, s))) return rc;
     }
@@ -770,20 +747,6 @@ struct ImogenEnsemble {
 };
 
 extern "C" {
-
-// A second pool of n doubles, or null when it would not leave half of the
-// device's free memory (the sweeps then work in place).
-static double *second_pool(int64_t n)
-{
-    size_t freeB = 0, totalB = 0;
-    double *p = nullptr;
-    if (hipMemGetInfo(&freeB, &totalB) != hipSuccess || (size_t)n * sizeof(double) > freeB / 2 ||
-        hipMalloc(&p, (size_t)n * sizeof(double)) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    return p;
-}
 
 int imogen_ensemble_create(int nprob, const int *nx, const int *ny, const double *hx, const double *hy, double gamma,
                            int limiter, double cfl, ImogenEnsemble **out)
@@ -813,18 +776,15 @@ int imogen_ensemble_create(int nprob, const int *nx, const int *ny, const double
         const int64_t pitch = (n + 31) / 32 * 32;  // 256-byte slabs
         off[p] = total;
         total += 5 * pitch;
-        e->host.push_back(EnsProblem{nullptr, nullptr, pitch, nx[p], ny[p], hx[p], hy[p], gamma, p, -1, 0, 0});
+        e->host.push_back(EnsProblem{nullptr, nullptr, pitch, nx[p], ny[p], hx[p], hy[p], ens_consts(gamma), p, -1, 0, 0});
         e->cells += n;
+        e->segS.push_back(1);
         e->xcls.push_back(x_class_of(nx[p]));
     }
     int rc = SUCCESSFUL;
     if (IM_HIP(hipMalloc(&e->pool, (size_t)total * sizeof(double)))) rc = ERROR_CUDA_BLEW_UP;
-    if (!rc) e->pool2 = second_pool(total);
-    for (int p = 0; p < nprob && !rc; p++) {
-        e->host[p].q = e->pool + off[p];
-        e->host[p].q2 = (e->pool2 ? e->pool2 : e->pool) + off[p];
-        e->segS.push_back(!e->pool2 && ny[p] >= 256 ? 2 : 1);
-    }
+    for (int p = 0; p < nprob && !rc; p++) e->host[p].q = e->pool + off[p];
+    if (!rc) rc = second_pool(e);
     if (!rc && IM_HIP(hipMalloc(&e->dprobs, nprob * sizeof(EnsProblem)))) rc = ERROR_CUDA_BLEW_UP;
     if (!rc && IM_HIP(hipMemcpy(e->dprobs, e->host.data(), nprob * sizeof(EnsProblem), hipMemcpyHostToDevice)))
         rc = ERROR_CUDA_BLEW_UP;
@@ -840,7 +800,7 @@ int imogen_ensemble_create(int nprob, const int *nx, const int *ny, const double
     if (!rc && IM_HIP(hipMalloc(&e->cflPart, (size_t)nprob * kEnsCflBlocks * sizeof(double)))) rc = ERROR_CUDA_BLEW_UP;
     if (!rc && IM_HIP(hipMalloc(&e->fold, nprob * sizeof(unsigned long long)))) rc = ERROR_CUDA_BLEW_UP;
     if (!rc) {
-        const std::vector<unsigned long long> none(nprob, ens_order_key(kEnsCflNone));
+        const std::vector<unsigned long long> none(nprob, order_key(kCflNone));
         if (IM_HIP(hipMemcpy(e->fold, none.data(), nprob * sizeof(unsigned long long), hipMemcpyHostToDevice)))
             rc = ERROR_CUDA_BLEW_UP;
     }
@@ -907,7 +867,7 @@ int imogen_ensemble_set_dust(ImogenEnsemble *E, const int *hasDust, double dustG
         }
     if (dusty.empty()) return SUCCESSFUL;
     const int NE = e->P + (int)dusty.size();
-    double *dpool = nullptr, *dpool2 = nullptr, *lam = nullptr, *part = nullptr;
+    double *dpool = nullptr, *lam = nullptr, *part = nullptr;
     EnsProblem *dprobs = nullptr;
     EnsDragTable *tab = nullptr;
     EnsDragItem *items = nullptr;
@@ -918,13 +878,11 @@ int imogen_ensemble_set_dust(ImogenEnsemble *E, const int *hasDust, double dustG
     std::vector<EnsDragItem> hitems;
     int64_t off = 0;
     int rc = IM_HIP(hipMalloc(&dpool, (size_t)total * sizeof(double)));
-    if (!rc && e->pool2) dpool2 = second_pool(total);
     for (size_t k = 0; k < dusty.size() && !rc; k++) {
         const int p = dusty[k];
         EnsProblem D = host[p];
         D.q = dpool + off;
-        D.q2 = (dpool2 ? dpool2 : dpool) + off;
-        D.gamma = dustGamma;
+        D.hc = ens_consts(dustGamma);
         D.owner = p;
         D.dust = -1;
         off += 5 * D.pitch;
@@ -945,7 +903,7 @@ int imogen_ensemble_set_dust(ImogenEnsemble *E, const int *hasDust, double dustG
     if (!rc) rc = IM_HIP(hipMalloc(&queue, (size_t)cells * 2 * sizeof(int64_t)));  // queue + second-call list
     if (!rc) rc = IM_HIP(hipMalloc(&qcount, 3 * sizeof(unsigned long long)));
     if (rc) {
-        void *bufs[] = {dpool, dpool2, dprobs, lam, part, tab, items, queue, qcount};
+        void *bufs[] = {dpool, dprobs, lam, part, tab, items, queue, qcount};
         for (void *b : bufs)
             if (b) (void)hipFree(b);
         return ERROR_CUDA_BLEW_UP;
@@ -957,13 +915,6 @@ int imogen_ensemble_set_dust(ImogenEnsemble *E, const int *hasDust, double dustG
     e->NE = NE;
     e->Pd = (int)dusty.size();
     e->dpool = dpool;
-    e->dpool2 = dpool2;
-    if (e->pool2 && !dpool2) {  // one mode for all: in place
-        (void)hipFree(e->pool2);
-        e->pool2 = nullptr;
-        for (EnsProblem &P : e->host) P.q2 = P.q;
-        for (int p = 0; p < e->P; p++) e->segS[p] = e->host[p].ny >= 256 ? 2 : 1;
-    }
     e->dprobs = dprobs;
     e->lam = lam;
     e->cflPart = part;
@@ -976,7 +927,8 @@ int imogen_ensemble_set_dust(ImogenEnsemble *E, const int *hasDust, double dustG
     e->dc = drag_consts(gas, dust);
     e->dragMethod = dragMethod;
     e->modelGen = learned_model_generation();
-    return build_work(e);
+    rc = second_pool(e);
+    return rc ? rc : build_work(e);
 }
 
 static int dust_entry(EnsembleImpl *e, int p)
@@ -1025,6 +977,7 @@ int imogen_ensemble_run(ImogenEnsemble *E, int firstIteration, int iterations, i
     }
     if (!E) return IM_FAIL(ERROR_NULL_POINTER, "null ensemble");
     EnsembleImpl *e = &E->impl;
+    if (!e->pool2) return IM_FAIL(ERROR_NOMEM, "the ensemble has no second pool (adding its dust failed)");
     DeviceState *st = state();
     if (!st) return ERROR_CUDA_BLEW_UP;
     for (int k = 0; k < iterations; k++) {
@@ -1068,6 +1021,7 @@ int imogen_ensemble_autotune(ImogenEnsemble *E, int trials, int *chosen)
 {
     if (!E) return IM_FAIL(ERROR_NULL_POINTER, "null ensemble");
     EnsembleImpl *e = &E->impl;
+    if (!e->pool2) return IM_FAIL(ERROR_NOMEM, "the ensemble has no second pool (adding its dust failed)");
     DeviceState *st = state();
     if (!st) return ERROR_CUDA_BLEW_UP;
     if (trials < 1) trials = 1;
@@ -1087,13 +1041,12 @@ int imogen_ensemble_autotune(ImogenEnsemble *E, int trials, int *chosen)
         return rc;
     };
     int rc = SUCCESSFUL;
-    // Y-march segments (factors on the base counts when there is a second pool)
-    // per size class (ny <= 128, <= 256, <= 512) among {1, 2, 4}:
-    // the class's default first, another count only when it is 1 % faster (two
+    // factor on the Y-march segment counts per size class (ny <= 128, <= 256,
+    // <= 512) among {1, 2, 4}: 1 first, another one only when it is 1 % faster (two
     // trial iterations differ by about that)
-    const int cand[3][3] = {{1, 2, 4}, {1, 2, 4}, {e->pool2 ? 1 : 2, e->pool2 ? 2 : 1, 4}};
+    static const int cand[3] = {1, 2, 4};
     auto cls_of = [](int ny) { return ny <= 128 ? 0 : (ny <= 256 ? 1 : 2); };
-    int best[3] = {1, 1, cand[2][0]};
+    int best[3] = {1, 1, 1};
     for (int cls = 0; cls < 3 && !rc; cls++) {
         bool any = false;
         for (int p = 0; p < e->P; p++) any = any || cls_of(e->host[p].ny) == cls;
@@ -1101,12 +1054,12 @@ int imogen_ensemble_autotune(ImogenEnsemble *E, int trials, int *chosen)
         float bestMs = 1e30f;
         for (int ci = 0; ci < 3 && !rc; ci++) {
             for (int p = 0; p < e->P; p++)
-                if (cls_of(e->host[p].ny) == cls) e->segS[p] = cand[cls][ci];
+                if (cls_of(e->host[p].ny) == cls) e->segS[p] = cand[ci];
             float ms = 0;
             rc = timed(&ms);
             if (!rc && (ci == 0 || ms < 0.99f * bestMs)) {
                 bestMs = ms;
-                best[cls] = cand[cls][ci];
+                best[cls] = cand[ci];
             }
         }
         for (int p = 0; p < e->P; p++)
@@ -1175,10 +1128,8 @@ int imogen_ensemble_destroy(ImogenEnsemble *E)
     DeviceState *st = state();
     if (st) (void)hipStreamSynchronize(st->stream);
     free_graphs(e);
-    for (int c = 0; c < kXClasses; c++)
-        if (e->xwork[c]) (void)hipFree(e->xwork[c]);
-    void *bufs[] = {e->pool,   e->pool2,    e->dpool2,    e->dprobs,   e->lam,       e->clock, e->cflPart, e->fold, e->cflList, e->ywork, e->xdummy,
-                    e->ydefer, e->dpool,    e->dtp,       e->dragTab, e->dragItems, e->queue, e->qcount};
+    void *bufs[] = {e->pool, e->pool2, e->dprobs, e->lam,     e->clock,     e->cflPart, e->fold, e->cflList,
+                    e->work, e->ydummy, e->dpool, e->dtp, e->dragTab, e->dragItems, e->queue, e->qcount};
     for (void *p : bufs)
         if (p) (void)hipFree(p);
     for (int k = 0; k < 2; k++) {

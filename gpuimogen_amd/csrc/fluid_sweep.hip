@@ -103,14 +103,17 @@ struct XGeom {
 
 // A part's window is its cells and 8 more, so K cells per lane take parts of
 // at most 64 K - 8 cells. Measured (HLLC, van Leer, smooth states, us):
-//  * Lines of up to 256 cells fill most lanes whole and a wave prefetches its
-//    next lines (65536 lines of 256: whole K=4 365, K=3 in 2 parts 534), as do
-//    lines of exactly 384 (36864 lines: whole K=6 363, K=4 in 2 parts 414,
-//    K=3 in 3 453).
-//  * Longer ones: K=3 (321: K=3 253, K=2 271, K=4 298; 512 x 32768: K=3 459,
-//    K=5 476, whole K=8 471; 1024 x 1024: K=3 39.5, K=5 44.1, K=4 55.6, and
-//    whole lines of 16 cells per lane, whose arrays left the registers, 130),
-//    but K=4 where two parts of it replace three (369..496).
+//  * Lines that fill their lanes (64, 128, 192, 256 cells) stay whole (16384 of
+//    128: 49, K=1 parts 64; 65536 of 256: 347, K=3 parts 477), as do lines of
+//    384 (36864: 341, K=4 parts 375) and of less than 64.
+//  * Others of up to 256 cells: K=1 parts, whose lanes need no select at a
+//    line's end and leave room for four waves per SIMD (13560 of 131: 54,
+//    whole 68; 20000 of 150: 77, 92), while the last-level cache holds the
+//    state and gives the parts' overlap for nothing (62500 of 250: 521, whole
+//    375; 40000 of 200: 240, 215).
+//  * Longer ones: K=3 (28700 of 321: 250, K=2 263, K=1 283; 1024 of 1024: 34,
+//    K=4 46, whole lines of 16 cells per lane, whose arrays left the
+//    registers, 130), but K=4 where two parts of it replace three (369..496).
 //  * Too few lines to fill the 1024 SIMDs: smaller K for a shorter chain per
 //    wave (17 lines of 300: K=1 5.3, K=2 5.7, K=3 6.6; 400 x 400: K=1 8.8,
 //    K=2 8.9, K=3 10.8), as far as 8 waves reach.
@@ -119,8 +122,9 @@ static XGeom x_geom(int N, int64_t nlines)
     XGeom g;
     if (N > 1024) return g;
     const auto parts = [N](int K) { return (N + 64 * K - 9) / (64 * K - 8); };
-    if (N > 64 && N <= 256 && nlines * parts(1) <= 1024) {
-        g.K = 1;
+    if (N > 64 && N <= 256) {
+        const bool cached = (int64_t)N * nlines * 5 * (int64_t)sizeof(double) <= (int64_t)256 << 20;
+        if ((N % 64 != 0 && cached) || nlines * parts(1) <= 1024) g.K = 1;
     } else if (N > 256 && N != 384) {
         if (nlines * parts(3) >= 1536) g.K = (N > 368 && N <= 496) ? 4 : 3;
         else g.K = parts(1) <= 8 ? 1 : (parts(2) <= 8 ? 2 : 3);
@@ -134,11 +138,7 @@ static XGeom x_geom(int N, int64_t nlines)
     g.K = (N == 384) ? 6 : (N + 63) / 64;
     g.nl = (N + g.K - 1) / g.K;
     const int lpw = 64 / g.nl;
-    int64_t waves = (nlines + lpw - 1) / lpw;
-    // Resident-wave budget: 2 waves per SIMD on 1024 SIMDs; beyond it a wave
-    // takes several line groups and prefetches the next one.
-    if (waves > 2048) waves = 2048;
-    g.blocks = (waves + 3) / 4;
+    g.blocks = ((nlines + lpw - 1) / lpw + 3) / 4;
     return g;
 }
 
@@ -180,14 +180,12 @@ static void *sweep_scratch(size_t off, size_t bytes)
 }
 
 template <class M, int LIM>
-static int launch_x(const double *src, double *dst, size_t scratchOff, int64_t pitch, int N, int64_t nlines,
-                    double lambda, const double *lamp, const HydroConsts &hc, int rt, const CflFuse &cf, hipStream_t s)
+static int launch_x(const double *src, double *dst, int64_t pitch, int N, int64_t nlines, double lambda,
+                    const double *lamp, const HydroConsts &hc, int rt, const CflFuse &cf, hipStream_t s)
 {
     const XGeom g = x_geom(N, nlines);
     if (g.K == 0) return IM_FAIL(ERROR_NOIMPLEMENT, "X sweep supports lines of at most 1024 cells (got %d)", N);
     const int K = g.K, nl = g.nl;
-    if (cf.part && g.blocks * (g.threads / 64) > cf.cap)
-        return IM_FAIL(ERROR_INVALID_ARGS, "CFL partial buffer too small");
     if (g.blocks > INT32_MAX) return IM_FAIL(ERROR_INVALID_ARGS, "too many lines for one X launch");
     dim3 grid((unsigned)g.blocks), block((unsigned)g.threads);
     if (g.parts) {
@@ -196,7 +194,7 @@ static int launch_x(const double *src, double *dst, size_t scratchOff, int64_t p
                        lamp, hc, rt, cf)
 #define IM_XP_CASE(KK)                  \
     case KK:                            \
-        if (cf.part) IM_XP(KK, true);   \
+        if (cf.slots) IM_XP(KK, true);  \
         else IM_XP(KK, false);          \
         break;
         switch (K) {
@@ -210,17 +208,15 @@ static int launch_x(const double *src, double *dst, size_t scratchOff, int64_t p
         return IM_LAUNCHED("sweep_xp");
     }
     const bool full = (nl * K == N) && (64 % nl == 0);
-    double *dummy = (double *)sweep_scratch(scratchOff, (size_t)g.blocks * 256 * 5 * sizeof(double));
-    if (!dummy) return IM_FAIL(ERROR_NOMEM, "no scratch for the X sweep");
 #define IM_X(KK, F, C)                                                                                        \
     hipLaunchKernelGGL((sweep_x<M, KK, LIM, F, C>), grid, block, 0, s, src, dst, pitch, N, nlines, nl, lambda, lamp, \
-                       hc, rt, dummy, cf)
-#define IM_X_CASE(KK)                              \
-    case KK:                                       \
-        if (full && cf.part) IM_X(KK, true, true); \
-        else if (full) IM_X(KK, true, false);      \
-        else if (cf.part) IM_X(KK, false, true);   \
-        else IM_X(KK, false, false);               \
+                       hc, rt, cf)
+#define IM_X_CASE(KK)                               \
+    case KK:                                        \
+        if (full && cf.slots) IM_X(KK, true, true); \
+        else if (full) IM_X(KK, true, false);       \
+        else if (cf.slots) IM_X(KK, false, true);   \
+        else IM_X(KK, false, false);                \
         break;
     switch (K) {
         IM_X_CASE(1)
@@ -228,7 +224,7 @@ static int launch_x(const double *src, double *dst, size_t scratchOff, int64_t p
         IM_X_CASE(3)
         IM_X_CASE(4)
     case 6:  // 384 cells: every lane full
-        if (cf.part) IM_X(6, true, true);
+        if (cf.slots) IM_X(6, true, true);
         else IM_X(6, true, false);
         break;
     }
@@ -247,7 +243,6 @@ static int launch_march(const double *src, double *dst, size_t scratchOff, int64
     const MarchGeom g = march_geom(nx, ny, nz, dir, src == dst);
     if (g.blocks > INT32_MAX) return IM_FAIL(ERROR_INVALID_ARGS, "too many columns for one march launch");
     dim3 grid((unsigned)g.blocks), block(256);
-    if (cf.part && g.nthr / 64 > cf.cap) return IM_FAIL(ERROR_INVALID_ARGS, "CFL partial buffer too small");
     double *defer = (double *)sweep_scratch(scratchOff, (size_t)g.nthr * march_slots(src == dst) * sizeof(double));
     if (!defer) return IM_FAIL(ERROR_NOMEM, "no scratch for deferred outputs");
     // rows of a multiple of 16 cells in a 256-byte-aligned slab: every segment
@@ -265,10 +260,10 @@ static int launch_march(const double *src, double *dst, size_t scratchOff, int64
         else IM_MARCH(D, C, false);       \
     } while (0)
     if (dir == 2) {
-        if (cf.part) IM_MARCH_NT(2, true);
+        if (cf.slots) IM_MARCH_NT(2, true);
         else IM_MARCH_NT(2, false);
     } else {
-        if (cf.part) IM_MARCH_NT(3, true);
+        if (cf.slots) IM_MARCH_NT(3, true);
         else IM_MARCH_NT(3, false);
     }
 #undef IM_MARCH_NT
@@ -283,7 +278,7 @@ static int launch_dir(const double *src, double *dst, size_t off, int64_t pitch,
 {
     const int slot = prof_begin(PROF_SWEEP_X + dir - 1, s);
     int rc;
-    if (dir == 1) rc = launch_x<M, LIM>(src, dst, off, pitch, nx, (int64_t)ny * nz, lambda, lamp, hc, rt, cf, s);
+    if (dir == 1) rc = launch_x<M, LIM>(src, dst, pitch, nx, (int64_t)ny * nz, lambda, lamp, hc, rt, cf, s);
     else rc = launch_march<M, LIM>(src, dst, off, pitch, nx, ny, nz, dir, lambda, lamp, hc, rt, cf, s);
     prof_end(slot, s);
     return rc;
@@ -307,24 +302,11 @@ static int launch_method(const double *src, double *dst, size_t off, int64_t pit
     }
 }
 
-// The grid arithmetic of launch_x / launch_march, for sizing fused-CFL buffers.
-int64_t sweep_waves(int nx, int ny, int nz, int dir, bool inplace)
-{
-    if (dir == 1) {
-        const XGeom g = x_geom(nx, (int64_t)ny * nz);
-        return g.blocks * (g.threads / 64);
-    }
-    return march_geom(nx, ny, nz, dir, inplace).nthr / 64;
-}
-
 int64_t sweep_scratch_bytes(int nx, int ny, int nz, int dir, bool inplace)
 {
     const int N = (dir == 1) ? nx : (dir == 2 ? ny : nz);
     if (dir < 1 || dir > 3 || N < 3) return 0;
-    if (dir == 1) {
-        const XGeom g = x_geom(nx, (int64_t)ny * nz);
-        return g.parts ? 0 : g.blocks * 256 * 5 * (int64_t)sizeof(double);
-    }
+    if (dir == 1) return 0;
     return march_geom(nx, ny, nz, dir, inplace).nthr * march_slots(inplace) * (int64_t)sizeof(double);
 }
 
@@ -338,6 +320,8 @@ int launch_fluid_sweep(const double *src, double *dst, size_t scratchOff, int64_
     HydroConsts hc;
     hc.gamma = gamma;
     hc.gm1 = gamma - 1.0;
+    hc.hgm1 = .5 * (gamma - 1.0);
+    hc.igm1 = 1.0 / (gamma - 1.0);
     hc.govergm1 = gamma / (gamma - 1.0);
     hc.rhomin = rhomin;
     hc.emin = 1e-5 / (gamma - 1.0);  // cudaFluidStep.cu:298

@@ -357,11 +357,6 @@ static unsigned paired_dirs(const MGArray *fluid, int method)
     return scratch_available(bytes + (size_t)need) ? dirs : 0;
 }
 
-bool sweep_out_of_place(const MGArray *fluid, int method, int dir)
-{
-    return paired_dirs(fluid, method) >> (dir - 1) & 1;
-}
-
 // flux.cu:27-155 on one rank: the sweep order of (stepNumber, stepDirection),
 // each sweep followed by that direction's boundary conditions.
 int last_sweep_dir(const MGArray *fluid, int stepNumber, int stepDirection)

@@ -102,7 +102,7 @@ int launch_permute_copy(const double *src, double *dst, const int sdim[3], const
 // performFluidUpdate_1D / _3D without the topology check. lampBase: when not
 // null, the sweeps of direction d read lambda from lampBase[d - 1] (device).
 // lastCfl (update_3d): when not null, the last sweep of the step also leaves
-// per-wave CFL minima (its lo/hi are filled in from the boundary modes).
+// CFL minima (its lo/hi are filled in from the boundary modes).
 int update_1d(MGArray *fluid, const FluidStepParams &params, const double *lampBase,
               const CflFuse *cfl = nullptr);
 int update_3d(MGArray *fluid, const FluidStepParams &fsp, const double *lampBase, const CflFuse *lastCfl = nullptr);
@@ -111,9 +111,6 @@ int update_3d(MGArray *fluid, const FluidStepParams &fsp, const double *lampBase
 int fluid_boundary(MGArray *fluid, int direction, int xrules, const GeometryParams *geo);
 // Direction swept last by update_3d for (stepNumber, stepDirection), 0 if none.
 int last_sweep_dir(const MGArray *fluid, int stepNumber, int stepDirection);
-// Whether update_3d runs direction dir of a step of this fluid and method out
-// of place, as one of a pair of sweeps through a second state array.
-bool sweep_out_of_place(const MGArray *fluid, int method, int dir);
 // Cells [lo, hi) of direction dir whose swept values survive the boundary
 // conditions update_3d sets after the sweep, when every other ghost they write
 // is a copy or mirror image of one of them (modes circular, mirror, const).
@@ -125,8 +122,8 @@ int cfl_keep_range(MGArray *fluid, int dir, int *lo, int *hi);
 // method: METHOD_HLLC or METHOD_HLL. rhomin, ciso: HLL floors and isothermal
 // sound speed (-1: adiabatic). lamp: when not null, the kernels read lambda
 // = dt/h from this device address instead of the `lambda` argument.
-// cfl: when not null, the sweep also writes the per-wave CFL minima of the
-// cells it stores (cfl_device.h).
+// cfl: when not null, the sweep also takes the CFL minima of the cells it
+// stores (cfl_device.h).
 // src == dst: in place; otherwise the swept state goes to dst, another array
 // of the same pitch, and src stays as it was. scratchOff: bytes at the start of
 // the scratch block the launch leaves alone.
@@ -164,11 +161,11 @@ int launch_soundspeed(const double *base, int64_t pitch, int64_t n, double gamma
 int launch_cfl(const double *base, int64_t pitch, int64_t n, const double *cs, double gamma, int fused,
                int dim, int xinjin, int halve, double hx, double hy, double hz, double hmin, double *devOut,
                hipStream_t s);
-// devOut[0] = min(part[0..n)) (x 1/2 when halve): the second pass over
-// per-wave minima a fused sweep left
-int launch_cfl_final(const double *part, int64_t n, int halve, double *devOut, hipStream_t s);
-// Wave count of a sweep launch over an nx x ny x nz HLLC/HLL array in
-// direction dir (the entries a fused CFL needs).
-int64_t sweep_waves(int nx, int ny, int nz, int dir, bool inplace);
+// The first of launch_cfl's two passes: nblocks (at most kCflBlocks) minima
+// that are still to be reduced and halved.
+constexpr int kCflBlocks = 2048;
+int launch_cfl_partials(const double *base, int64_t pitch, int64_t n, const double *cs, double gamma, int fused,
+                        int dim, int xinjin, double hx, double hy, double hz, double hmin, double *blockMin,
+                        int *nblocks, hipStream_t s);
 
 }  // namespace imogen

@@ -1,6 +1,6 @@
 // sweep_device.h -- per-cell arithmetic of the HLLC and HLL sweeps (gfx950, FP64).
 //
-// Same formulas, in the same operation order, as the reference kernels
+// Same formulas as the reference kernels
 // cukern_HLLC_2ndorder (gpuclass/cudaFluidStep.cu:1124-1716) and
 // cukern_HLL_step + cukern_PressureSolverHydro (:1801-2422, 2813-2864):
 // primitive recovery (RECONSTRUCT_VELOCITY, gpuclass/Makefile:5), half-slope
@@ -25,6 +25,8 @@ struct V5 {
 struct HydroConsts {
     double gamma;     // adiabatic index
     double gm1;       // gamma - 1
+    double hgm1;      // (gamma - 1) / 2
+    double igm1;      // 1 / (gamma - 1)
     double govergm1;  // gamma / (gamma - 1)
     double rhomin;    // density floor (HLL)
     double emin;      // specific internal energy floor 1e-5/(gamma-1) (cudaFluidStep.cu:298)
@@ -88,47 +90,38 @@ __device__ __forceinline__ double sqrt_nr(double x)
 // Goldschmidt step for the square root (~5e-15). The sweep results stay far
 // inside the 1e-12 parity bar; the correctly rounded quotient (div_cr) keeps
 // the full-precision reciprocal.
-#ifndef IMOGEN_SWEEP_FAST_MATH
-#define IMOGEN_SWEEP_FAST_MATH 1
-#endif
 __device__ __forceinline__ double rcp_fast(double x)
 {
-#if IMOGEN_SWEEP_FAST_MATH
     const double r = __builtin_amdgcn_rcp(x);
     return fma(r, fma(-x, r, 1.0), r);
-#else
-    return rcp_nr(x);
-#endif
 }
 
 __device__ __forceinline__ double div_fast(double a, double b)
 {
-    return a * rcp_fast(b);
+    // the Newton step on the quotient: q (2 - b r), q = a r
+    const double r = __builtin_amdgcn_rcp(b);
+    const double q = a * r;
+    return fma(q, fma(-b, r, 1.0), q);
 }
 
-__device__ __forceinline__ double sqrt_fast(double x)
-{
-#if IMOGEN_SWEEP_FAST_MATH
-    const double y = __builtin_amdgcn_rsq(x + 1e-300);
-    const double g = x * y;
-    const double r = fma(-g, 0.5 * y, 0.5);
-    return fma(g, r, g);
-#else
-    return sqrt_nr(x);
-#endif
-}
-
-// sqrt_fast for arguments known to be > 0 (ratios of densities)
+// sqrt(x), x > 0. Callers add the smallest step kTinySq to a sum that may be
+// exactly 0 (in an FMA they need anyway), so that its root is ~0 and not NaN;
+// it changes no sum >= 1e-284, and negative ones stay NaN.
+constexpr double kTinySq = 1e-300;
 __device__ __forceinline__ double sqrt_fast_pos(double x)
 {
-#if IMOGEN_SWEEP_FAST_MATH
     const double y = __builtin_amdgcn_rsq(x);
     const double g = x * y;
     const double r = fma(-g, 0.5 * y, 0.5);
     return fma(g, r, g);
-#else
-    return sqrt_nr(x);
-#endif
+}
+
+// 1/sqrt(|x|) to full precision (third-order step: error ~ e^3)
+__device__ __forceinline__ double rsqrt_abs(double x)
+{
+    const double y = __builtin_amdgcn_rsq(fabs(x));
+    const double e = fma(-(fabs(x) * y), y, 1.0);
+    return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
 // ---- half-slope limiters (limiter_functions.h) ----------------------------
@@ -138,6 +131,10 @@ __device__ __forceinline__ double flux_minmod(double a, double b)
     return (fabs(a) > fabs(b)) ? b : a;
 }
 
+// The limited half slope is slope_scale<LIM> * slope_limit<LIM>(a, b).
+// Products of opposite signs are raised to 0 (v_max_f64) in place of a compare
+// and two selects on the result, so a NaN difference gives no slope, as the
+// reference's `r > 0` does.
 template <int LIM>
 __device__ __forceinline__ double slope_limit(double a, double b, int rt)
 {
@@ -148,15 +145,17 @@ __device__ __forceinline__ double slope_limit(double a, double b, int rt)
         // |A|, |B| < 1.5e-154, where the numerator has already underflowed to
         // zero and the quotient is +-0; the hardware reciprocal of such a
         // denominator is infinite, so it is raised to the smallest normal.
-        double r = a * b;
-        double s = a + b;
-        double v = div_fast(.75 * r * s, fmax(s * s - r, 0x1p-1022));
-        return (r > 0) ? v : 0.0;
+        const double r = fmax(a * b, 0.0);
+        const double s = a + b;
+        return div_fast(((LIM >= 0) ? 1.0 : .75) * r * s, fmax(fma(s, s, -r), 0x1p-1022));
     }
     case 1: {  // van Leer: A B / (A+B)
-        double r = a * b;
-        double v = div_fast(r, a + b);
-        return (r > 0.0) ? v : 0.0;
+        // A+B = 0 only with A B <= 0: 0 times the infinite reciprocal is NaN,
+        // which the minimum (a number against NaN) turns into |A+B| = 0; it
+        // leaves every other value, at most |A+B|/4 in size, as it is
+        const double r = fmax(a * b, 0.0);
+        const double s = a + b;
+        return fmin(div_fast(r, s), fabs(s));
     }
     case 2: {  // minmod, returned through float as the reference does (:70)
         if (a * b < 0) return 0.0;
@@ -185,13 +184,33 @@ __device__ __forceinline__ double slope_limit(double a, double b, int rt)
     }
 }
 
-// Conserved (rho, E, pN, pT1, pT2) -> primitive (rho, e_int, vN, vT1, vT2),
-// cudaFluidStep.cu:1218-1234.
-__device__ __forceinline__ V5 to_prim(const V5 &q)
+template <int LIM>
+constexpr double slope_scale = (LIM == 0) ? .75 : 1.0;
+
+// w -+ the limited half slope, one FMA each
+template <int LIM>
+__device__ __forceinline__ void face_pair(double w, double dl, double dr, int rt, double &L, double &R)
 {
-    double F = rcp_fast(q.a);
-    double B = q.b - .5 * (q.c * q.c + q.d * q.d + q.e * q.e) * F;
-    return V5{q.a, B, q.c * F, q.d * F, q.e * F};
+    const double s = slope_limit<LIM>(dl, dr, rt);
+    L = fma(-slope_scale<LIM>, s, w);
+    R = fma(slope_scale<LIM>, s, w);
+}
+
+// Limiters with lim(c a, c b) = c lim(a, b): pressure and internal energy then
+// reconstruct alike, and the pressure is formed once per cell instead of on
+// both faces. (Minmod's pass through float is not of these.)
+template <int LIM>
+constexpr bool slope_homogeneous = (LIM == 0 || LIM == 1);
+
+// Conserved (rho, E, pN, pT1, pT2) -> primitive (rho, e_int, vN, vT1, vT2),
+// cudaFluidStep.cu:1218-1234; with a homogeneous limiter P in place of e_int.
+template <int LIM>
+__device__ __forceinline__ V5 to_prim(const HydroConsts &k, const V5 &q)
+{
+    const double F = rcp_fast(q.a);
+    const double u = q.c * F, v = q.d * F, w = q.e * F;
+    const double e = fma(-.5, fma(q.e, w, fma(q.d, v, q.c * u)), q.b);
+    return V5{q.a, slope_homogeneous<LIM> ? k.gm1 * e : e, u, v, w};
 }
 
 // Left/right face states of a cell from its primitive w and the backward
@@ -201,114 +220,109 @@ template <int LIM>
 __device__ __forceinline__ void faces(const HydroConsts &k, const V5 &w, const V5 &dl, const V5 &dr,
                                       int rt, V5 &L, V5 &R)
 {
-    double s;
-    s = slope_limit<LIM>(dl.a, dr.a, rt);
-    L.a = w.a - s;
-    R.a = w.a + s;
-    s = slope_limit<LIM>(dl.b, dr.b, rt);
-    L.b = k.gm1 * (w.b - s);
-    R.b = k.gm1 * (w.b + s);
-    s = slope_limit<LIM>(dl.c, dr.c, rt);
-    L.c = w.c - s;
-    R.c = w.c + s;
-    s = slope_limit<LIM>(dl.d, dr.d, rt);
-    L.d = w.d - s;
-    R.d = w.d + s;
-    s = slope_limit<LIM>(dl.e, dr.e, rt);
-    L.e = w.e - s;
-    R.e = w.e + s;
+    face_pair<LIM>(w.a, dl.a, dr.a, rt, L.a, R.a);
+    face_pair<LIM>(w.b, dl.b, dr.b, rt, L.b, R.b);
+    if (!slope_homogeneous<LIM>) {
+        L.b *= k.gm1;
+        R.b *= k.gm1;
+    }
+    face_pair<LIM>(w.c, dl.c, dr.c, rt, L.c, R.c);
+    face_pair<LIM>(w.d, dl.d, dr.d, rt, L.d, R.d);
+    face_pair<LIM>(w.e, dl.e, dr.e, rt, L.e, R.e);
+}
+
+// Roe weights and sound speeds of an interface from its face densities and
+// pressures. One reciprocal root y = |rhoL rhoR|^-1/2 gives both densities'
+// reciprocals (+-y^2 rhoR, +-y^2 rhoL) and sqrt(rhoR / rhoL) = y |rhoR|, the
+// last only where the densities have one sign (`roe`: the reference's root is
+// NaN otherwise, and the bounds formed of it lose every comparison). SHARED
+// false: a reciprocal per side, for the limiters among which van Albada makes
+// NaN slopes of constant states: a NaN of one side must not reach the other
+// side's sound speed there.
+struct RoeTerms {
+    double csql, csqr;  // gamma P / rho
+    double Fa, Fb;      // sqrt(rhoR / rhoL), 1 / (1 + Fa)
+    bool roe;
+};
+template <bool SHARED>
+__device__ __forceinline__ RoeTerms roe_terms(const HydroConsts &k, double rl, double rr, double Pl, double Pr)
+{
+    const double d = rl * rr;
+    const double y = rsqrt_abs(d);
+    const double p = copysign(y * y, d);
+    RoeTerms t;
+    t.csql = fma(k.gamma * Pl, SHARED ? p * rr : rcp_fast(rl), kTinySq);
+    t.csqr = fma(k.gamma * Pr, SHARED ? p * rl : rcp_fast(rr), kTinySq);
+    t.Fa = y * fabs(rr);
+    t.Fb = rcp_fast(1.0 + t.Fa);
+    t.roe = d > 0;
+    return t;
+}
+
+// Einfeldt bounds (cudaFluidStep.cu:1728-1754) of normal velocities vl, vr and
+// squared velocity jump dvsq. The reference's selects, not fmin/fmax: a NaN
+// bound (negative face pressure) must propagate as it does there.
+__device__ __forceinline__ void einfeldt(const HydroConsts &k, const RoeTerms &t, double vl, double vr, double dvsq,
+                                         double &sl, double &sr)
+{
+    const double Vroe = fma(t.Fa, vr, vl) * t.Fb;
+    const double x = fma(k.hgm1 * dvsq, t.Fa * t.Fb, fma(t.Fa, t.csqr, t.csql));
+    const double C = sqrt_fast_pos(fma(x, t.Fb, kTinySq));
+    sl = vl - sqrt_fast_pos(t.csql);
+    sr = vr + sqrt_fast_pos(t.csqr);
+    sl = (t.roe & (Vroe - C < sl)) ? Vroe - C : sl;
+    sr = (t.roe & (Vroe + C > sr)) ? Vroe + C : sr;
 }
 
 // HLLC flux through the interface between face state L (right face of cell i)
 // and R (left face of cell i+1). Returns (mass, energy, pN, pT1, pT2) fluxes.
 // The four reference cases are evaluated without divergence: the upwind side
-// and its wave speed are selected first, then the plain and star fluxes of
-// that side are both formed and one is kept.
-// BRANCH: form the plain or the star flux under a branch (fewer live values;
-// the X kernel's register budget needs it) instead of the select form below.
-template <bool BRANCH>
+// and its wave speed are selected first; that side's plain flux (cases 0/1,
+// cudaFluidStep.cu:1372-1383, 1416-1430) is its star flux (cases 2/3,
+// :1384-1415) with the contact speed replaced by the side's own velocity and
+// rho beta by rho, so two selects choose between them. With mass flux m the
+// energy flux is m (c^2/(gamma-1) + |v|^2/2 + S_K (S_M - v)) and the
+// tangential ones are v_t m.
+template <int LIM>
 __device__ __forceinline__ V5 hllc_flux(const HydroConsts &k, const V5 &L, const V5 &R)
 {
     // velocity jump squared (cudaFluidStep.cu:1318-1322)
-    double C = L.c - R.c;
-    double D = L.d - R.d;
-    double E = L.e - R.e;
-    double dvsq = C * C + D * D + E * E;
-
-    // Einfeldt bounds (cudaFluidStep.cu:1728-1754). The two face densities'
-    // reciprocals serve both sound speeds, the Roe ratio and the star flux.
-    const double iL = rcp_fast(L.a);
-    const double iR = rcp_fast(R.a);
-    double csql = k.gamma * L.b * iL;
-    double csqr = k.gamma * R.b * iR;
-    double Fa = sqrt_fast_pos(R.a * iL);
-    double Fb = rcp_fast(1.0 + Fa);
-    double Croe = ((csql + Fa * csqr) + .5 * k.gm1 * dvsq * Fa * Fb) * Fb;
-    double Vroe = (L.c + Fa * R.c) * Fb;
-    Croe = Vroe - sqrt_fast(Croe);
-    double sl = L.c - sqrt_fast(csql);
-    double sr = R.c + sqrt_fast(csqr);
-    // the reference's selects, not fmin/fmax: a NaN bound (negative face
-    // pressure) must propagate as it does there
-    sl = (Croe < sl) ? Croe : sl;
-    Croe = 2 * Vroe - Croe;
-    sr = (Croe > sr) ? Croe : sr;
+    const double C = L.c - R.c;
+    const double D = L.d - R.d;
+    const double E = L.e - R.e;
+    const RoeTerms t = roe_terms<(LIM >= 0)>(k, L.a, R.a, L.b, R.b);
+    double sl, sr;
+    einfeldt(k, t, L.c, R.c, fma(E, E, fma(D, D, C * C)), sl, sr);
 
     // contact speed, Batten et al. eq. 34 (cudaFluidStep.cu:1352-1357)
-    double A = L.a * (sl - L.c);
-    double B = R.a * (sr - R.c);
-    double sm = div_fast(B * R.c - R.b - A * L.c + L.b, B - A);
+    const double A = L.a * (sl - L.c);
+    const double B = R.a * (sr - R.c);
+    const double sm = div_fast(fma(B, R.c, fma(-A, L.c, L.b - R.b)), B - A);
 
     // case selection (cudaFluidStep.cu:1363-1369)
     const bool left = sm > 0;
     const bool star = left ? !(sl > 0) : (sr > 0);
     const V5 S = left ? L : R;
     const double sk = left ? sl : sr;
-    const double iS = left ? iL : iR;
+    const double csq = left ? t.csql : t.csqr;
+    const double AS = left ? A : B;
 
-    double ksum = S.c * S.c + S.d * S.d + S.e * S.e;  // |v|^2 of the upwind face
-    if (BRANCH) {
-        V5 out;
-        if (!star) {
-            // cases 0/1 (cudaFluidStep.cu:1372-1383, 1416-1430)
-            const double Ek = .5 * ksum * S.a;
-            const double m = S.a * S.c;
-            out.a = m;
-            out.b = S.c * (Ek + k.govergm1 * S.b);
-            out.c = m * S.c + S.b;
-            out.d = S.d * m;
-            out.e = S.e * m;
-        } else {
-            // cases 2/3 (cudaFluidStep.cu:1384-1415)
-            const double rb = div_fast(S.a * (sk - S.c), sk - sm);  // rho * beta
-            const double G = .5 * ksum;
-            const double m = rb * sm;
-            const double Cc = sk * (sm - S.c);
-            out.a = m;
-            out.b = rb * sm * (k.govergm1 * S.b * iS + G + Cc);
-            out.c = S.b + rb * (Cc + sm * S.c);
-            out.d = S.d * m;
-            out.e = S.e * m;
-        }
-        return out;
-    }
-    // Plain flux of the upwind side (cases 0/1, cudaFluidStep.cu:1372-1383,
-    // 1416-1430) and its star flux (cases 2/3, :1384-1415) share their form:
-    // with mass flux m (rho v of the face, or rho beta S_M), the energy flux
-    // is m (gamma/(gamma-1) P/rho + |v|^2/2 [+ S_K (S_M - v)]) and the
-    // tangential fluxes are v_t m, so one select per differing term replaces
-    // forming both fluxes and selecting five results.
-    const double rb = div_fast(S.a * (sk - S.c), sk - sm);  // rho * beta (star)
-    const double G = .5 * ksum;
-    const double mp = S.a * S.c;
-    const double Cc = sk * (sm - S.c);
-    const double m = star ? rb * sm : mp;
-    const double cz = star ? Cc : 0.0;
-    const double tn = star ? rb * (Cc + sm * S.c) : mp * S.c;
+    double rb = div_fast(AS, sk - sm);  // rho beta
+    // the empty asm keeps the quotient out of a branch on `star` (which the
+    // compiler would form around its one use): nearly every interface is a
+    // star one, and a branch per interface splits the code the two stages'
+    // chains interleave in
+    asm("" : "+v"(rb));
+    rb = star ? rb : S.a;
+    const double vm = star ? sm : S.c;
+    const double ksum = fma(S.e, S.e, fma(S.d, S.d, S.c * S.c));  // |v|^2 of the upwind face
+    // 0 in the plain case also where the bound of the other side is NaN
+    const double Cc = (star ? sk : 0.0) * (vm - S.c);
+    const double m = rb * vm;
     V5 out;
     out.a = m;
-    out.b = m * (k.govergm1 * S.b * iS + G + cz);
-    out.c = S.b + tn;
+    out.b = m * fma(csq, k.igm1, fma(.5, ksum, Cc));
+    out.c = fma(rb, fma(vm, S.c, Cc), S.b);
     out.d = S.d * m;
     out.e = S.e * m;
     return out;
@@ -324,14 +338,16 @@ __device__ __forceinline__ V5 hllc_flux(const HydroConsts &k, const V5 &L, const
 // flux(): interface flux in slab order (mass, energy, normal, t1, t2).
 
 struct Hllc {
+    static constexpr bool floors = false;  // floor() leaves the cell as it is
     template <int DIR>
     __device__ static __forceinline__ double floor(const HydroConsts &, V5 &)
     {
         return 0.0;
     }
-    __device__ static __forceinline__ V5 prims(const HydroConsts &, const V5 &q, double)
+    template <int LIM>
+    __device__ static __forceinline__ V5 prims(const HydroConsts &k, const V5 &q, double)
     {
-        return to_prim(q);
+        return to_prim<LIM>(k, q);
     }
     template <int LIM>
     __device__ static __forceinline__ void face(const HydroConsts &k, const V5 &w, const V5 &dl, const V5 &dr,
@@ -339,14 +355,15 @@ struct Hllc {
     {
         faces<LIM>(k, w, dl, dr, rt, L, R);
     }
-    template <bool LOWREG = false>
+    template <int LIM>
     __device__ static __forceinline__ V5 flux(const HydroConsts &k, const V5 &L, const V5 &R)
     {
-        return hllc_flux<LOWREG>(k, L, R);
+        return hllc_flux<LIM>(k, L, R);
     }
 };
 
 struct Hll {
+    static constexpr bool floors = true;
     // q = (rho, E, pN, pT1, pT2) in HLL's component order for direction DIR:
     // X (px,py,pz), Y (py,px,pz), Z (pz,px,py) (cudaFluidStep.cu:1869-1885).
     // The floors accumulate |p|^2 in physical x,y,z order (:2821-2843).
@@ -377,6 +394,7 @@ struct Hll {
         return e;
     }
     // (rho, vN, P, vT1, vT2); velocities are quotients, as in the reference (:1887-1889)
+    template <int LIM>
     __device__ static __forceinline__ V5 prims(const HydroConsts &k, const V5 &q, double e)
     {
         return V5{q.a, div_cr(q.c, q.a), e * k.gm1, div_cr(q.d, q.a), div_cr(q.e, q.a)};
@@ -385,46 +403,24 @@ struct Hll {
     __device__ static __forceinline__ void face(const HydroConsts &, const V5 &w, const V5 &dl, const V5 &dr,
                                                 int rt, V5 &L, V5 &R)
     {
-        double s;
-        s = slope_limit<LIM>(dl.a, dr.a, rt);
-        L.a = w.a - s;
-        R.a = w.a + s;
-        s = slope_limit<LIM>(dl.b, dr.b, rt);
-        L.b = w.b - s;
-        R.b = w.b + s;
-        s = slope_limit<LIM>(dl.c, dr.c, rt);
-        L.c = w.c - s;
-        R.c = w.c + s;
-        s = slope_limit<LIM>(dl.d, dr.d, rt);
-        L.d = w.d - s;
-        R.d = w.d + s;
-        s = slope_limit<LIM>(dl.e, dr.e, rt);
-        L.e = w.e - s;
-        R.e = w.e + s;
+        face_pair<LIM>(w.a, dl.a, dr.a, rt, L.a, R.a);
+        face_pair<LIM>(w.b, dl.b, dr.b, rt, L.b, R.b);
+        face_pair<LIM>(w.c, dl.c, dr.c, rt, L.c, R.c);
+        face_pair<LIM>(w.d, dl.d, dr.d, rt, L.d, R.d);
+        face_pair<LIM>(w.e, dl.e, dr.e, rt, L.e, R.e);
     }
     // L, R = (rho, vN, P, vT1, vT2), the reference's A..E (cudaFluidStep.cu:2124-2196)
-    template <bool LOWREG = false>
+    template <int LIM>
     __device__ static __forceinline__ V5 flux(const HydroConsts &k, const V5 &L, const V5 &R)
     {
         const double Ut = R.b - L.b, St1 = R.d - L.d, St2 = R.e - L.e;
-        const double dvsq = Ut * Ut + St1 * St1 + St2 * St2;
+        const RoeTerms t = roe_terms<(LIM >= 0)>(k, L.a, R.a, L.c, R.c);
         double sl, sr;
-        const double iL = rcp_fast(L.a);
-        const double Fa = sqrt_fast(R.a * iL);
-        const double Fb = rcp_fast(1.0 + Fa);
-        const double Vroe = (L.b + Fa * R.b) * Fb;
         if (k.ciso == -1) {
-            const double csql = k.gamma * L.c * iL;
-            const double csqr = k.gamma * R.c * rcp_fast(R.a);
-            double Croe = ((csql + Fa * csqr) + .5 * k.gm1 * dvsq * Fa * Fb) * Fb;
-            Croe = Vroe - sqrt_fast(Croe);
-            sl = L.b - sqrt_fast(csql);
-            sr = R.b + sqrt_fast(csqr);
-            sl = (Croe < sl) ? Croe : sl;
-            Croe = 2 * Vroe - Croe;
-            sr = (Croe > sr) ? Croe : sr;
+            einfeldt(k, t, L.b, R.b, fma(St2, St2, fma(St1, St1, Ut * Ut)), sl, sr);
         } else {
             // computeEinfeldtBounds_isothermal, passed C_iso^2 for the sound speed (:2131)
+            const double Vroe = fma(t.Fa, R.b, L.b) * t.Fb;
             double cs = Vroe - k.cisosq;
             sl = L.b - cs;
             sr = R.b + cs;
@@ -462,7 +458,7 @@ struct Hll {
                 const double kl = .5 * L.a * (L.b * L.b + L.d * L.d + L.e * L.e);
                 const double kr = .5 * R.a * (R.b * R.b + R.d * R.d + R.e * R.e);
                 const double e = (wl * kl - wr * kr);
-                o.b = (e + (k.govergm1 * (sr * L.c * L.b - sl * R.c * R.b) + sl * sr * (R.c - L.c) / k.gm1)) * At;
+                o.b = (e + (k.govergm1 * (sr * L.c * L.b - sl * R.c * R.b) + sl * sr * (R.c - L.c) * k.igm1)) * At;
             } else {
                 // no 1/(Sr-Sl) on the isothermal energy flux in the reference (:2185-2189)
                 const double kl = .5 * L.a * (L.b * L.b + L.d * L.d + L.e * L.e) + L.c;

@@ -26,25 +26,20 @@ __device__ __forceinline__ V5 sel5(bool c, const V5 &x, const V5 &y)
     return c ? x : y;
 }
 
-__device__ __forceinline__ V5 axpy_update(const V5 &q, double lam, const V5 &fr, const V5 &fl)
+__device__ __forceinline__ V5 axpy5(const V5 &q, double c, const V5 &d)
 {
-    // Qout = Qin - lambda*(F_{i+1/2} - F_{i-1/2})      (cudaFluidStep.cu:1510-1516)
-    return V5{q.a - lam * (fr.a - fl.a), q.b - lam * (fr.b - fl.b), q.c - lam * (fr.c - fl.c),
-              q.d - lam * (fr.d - fl.d), q.e - lam * (fr.e - fl.e)};
+    return V5{fma(c, d.a, q.a), fma(c, d.b, q.b), fma(c, d.c, q.c), fma(c, d.d, q.d), fma(c, d.e, q.e)};
 }
 
-__device__ __forceinline__ V5 avg_update(const V5 &s, double lam, const V5 &fr, const V5 &fl)
+// The SSP-RK2 stages (cudaFluidStep.cu:1510-1516, 1555-1561): with dF = F_{i+1/2}
+// - F_{i-1/2}, U1 = Q - lambda dF(Q) and Qout = (Q + U1)/2 - lambda/2 dF(U1).
+// The half sum (Q + U1)/2 is Q - lambda/2 dF(Q) where the method has no floors
+// that change U1.
+template <class M>
+__device__ __forceinline__ V5 half_sum(const V5 &q, const V5 &u, const V5 &dF, double mhl)
 {
-    // Qout = .5*((Qin + Qout) - lambda*(F_{i+1/2} - F_{i-1/2}))   (cudaFluidStep.cu:1555-1561)
-    // s already holds (Qin + Qout).
-    return V5{.5 * (s.a - lam * (fr.a - fl.a)), .5 * (s.b - lam * (fr.b - fl.b)),
-              .5 * (s.c - lam * (fr.c - fl.c)), .5 * (s.d - lam * (fr.d - fl.d)),
-              .5 * (s.e - lam * (fr.e - fl.e))};
-}
-
-__device__ __forceinline__ V5 add5(const V5 &x, const V5 &y)
-{
-    return V5{x.a + y.a, x.b + y.b, x.c + y.c, x.d + y.d, x.e + y.e};
+    if (!M::floors) return axpy5(q, mhl, dF);
+    return V5{.5 * (q.a + u.a), .5 * (q.b + u.b), .5 * (q.c + u.c), .5 * (q.d + u.d), .5 * (q.e + u.e)};
 }
 
 // NT: loads and stores with the nontemporal hint. The single-grid Y/Z
@@ -111,7 +106,7 @@ __device__ __forceinline__ void x_fluxes(const HydroConsts &hc, int rt, V5 (&U)[
 #pragma unroll
     for (int k = 0; k < K; k++) {
         const double e = M::template floor<1>(hc, U[k]);
-        w[k] = M::prims(hc, U[k], e);
+        w[k] = M::template prims<LIM>(hc, U[k], e);
     }
 
     V5 wlast = w[0];
@@ -135,7 +130,9 @@ __device__ __forceinline__ void x_fluxes(const HydroConsts &hc, int rt, V5 (&U)[
 #pragma unroll
     for (int k = 0; k < K; k++) {
         const V5 right = (k + 1 < K) ? sel5(k + 1 < cnt, Lf[(k + 1 < K) ? k + 1 : 0], LfR) : LfR;
-        F[k] = M::template flux<(K >= 4)>(hc, Rf[k], right);
+        F[k] = M::template flux<LIM>(hc, Rf[k], right);
+        // keep the cells' fluxes apart: interleaved they spill at 4 cells per lane
+        if (K >= 4) __builtin_amdgcn_sched_barrier(0);
     }
     V5 Flast = F[0];
 #pragma unroll
@@ -143,23 +140,42 @@ __device__ __forceinline__ void x_fluxes(const HydroConsts &hc, int rt, V5 (&U)[
     Fm = shfl5(Flast, srcL);
 }
 
-// Each wave loops over groups of lines (lpw lines per group, groups strided by
-// the number of waves in the grid). While one group is computed, the next
-// group's cells are already being loaded. FULL: every line is exactly nl*K
-// cells and nl divides 64, so every lane holds K cells and all memory
-// operations are unconditional (the compiler can then count them exactly and
-// wait only for the loads it needs); lanes past the last line read a clamped
-// valid line and write into a private dummy slot.
+// Both stages of the cells a lane owns, Q in, the new state out (in Q).
+template <class M, int K, int LIM>
+__device__ __forceinline__ void x_stages(const HydroConsts &hc, int rt, V5 (&Q)[K], int cnt, int srcL, int srcR,
+                                         double lambda)
+{
+    const double ml = -lambda, mhl = -.5 * lambda;
+    V5 F[K], Fm, U1[K];
+    x_fluxes<M, K, LIM>(hc, rt, Q, cnt, srcL, srcR, F, Fm);
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        const V5 dF = F[k] - (k == 0 ? Fm : F[k > 0 ? k - 1 : 0]);
+        U1[k] = axpy5(Q[k], ml, dF);
+        if (!M::floors) Q[k] = half_sum<M>(Q[k], U1[k], dF, mhl);
+    }
+    x_fluxes<M, K, LIM>(hc, rt, U1, cnt, srcL, srcR, F, Fm);
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        const V5 dF = F[k] - (k == 0 ? Fm : F[k > 0 ? k - 1 : 0]);
+        if (M::floors) Q[k] = half_sum<M>(Q[k], U1[k], dF, mhl);  // U1 as its floors left it
+        Q[k] = axpy5(Q[k], mhl, dF);
+    }
+}
+
+// Whole lines, 64 / nl of them per wave (nl lanes of K cells each). FULL: every
+// line is exactly nl*K cells and nl divides 64, so every lane holds K cells.
+// A wave takes one group of lines: fresh waves hide the load latency better
+// than a wave that prefetched its next group, whose second register set cost
+// spills (256^3: 347 us against 475 prefetching; 128^3 49 against 56).
 template <class M, int K, int LIM, bool FULL, bool CFL>
 __global__ __launch_bounds__(256, (K <= 4) ? 2 : 1) void sweep_x(const double *src, double *dst, int64_t pitch, int N,
                                                int64_t nlines, int nl, double lambda,
-                                               const double *__restrict__ lamp, HydroConsts hc, int rt,
-                                               double *__restrict__ dummy, CflFuse cf)
+                                               const double *__restrict__ lamp, HydroConsts hc, int rt, CflFuse cf)
 {
     if (lamp) lambda = lamp[0];  // time step kept on the device
     const int lane = threadIdx.x & 63;
     const int64_t wave = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    const int64_t nwaves = (int64_t)gridDim.x * (blockDim.x >> 6);
     const int lpw = 64 / nl;
     const int sub = lane / nl;
     const int j = lane - sub * nl;
@@ -168,75 +184,29 @@ __global__ __launch_bounds__(256, (K <= 4) ? 2 : 1) void sweep_x(const double *s
     const int srcL = laneUsed ? lbase + (j == 0 ? nl - 1 : j - 1) : lane;
     const int srcR = laneUsed ? lbase + (j == nl - 1 ? 0 : j + 1) : lane;
     const int x0 = laneUsed ? j * K : 0;
-    int cntL = N - x0;
-    cntL = cntL < K ? cntL : K;
-    if (!laneUsed) cntL = 0;
-    const int cnt = FULL ? K : cntL;
-    const int64_t gtid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t nthr = (int64_t)gridDim.x * blockDim.x;
-    double *mydummy = dummy + gtid;
-    const int64_t groupStride = nwaves * lpw;
-
-    auto line_off = [&](int64_t ln) {
-        const int64_t c = ln < nlines ? ln : nlines - 1;
-        return c * (int64_t)N + x0;
-    };
-    auto load_group = [&](int64_t ln, V5 (&Qd)[K]) {
-        const double *b = src + line_off(ln);
+    int cnt = N - x0;
+    cnt = cnt < K ? cnt : K;
+    if (FULL) cnt = K;
+    else if (!laneUsed) cnt = 0;
+    const int64_t line = wave * lpw + (laneUsed ? sub : 0);
+    const bool own = laneUsed && line < nlines;
+    const int64_t off = (line < nlines ? line : nlines - 1) * (int64_t)N + x0;
+    V5 Q[K];
 #pragma unroll
-        for (int k = 0; k < K; k++) {
-            if (k < cnt) Qd[k] = load_cell<M, 1>(b + k, pitch);
-            else Qd[k] = V5{1.0, 1.0, 0.0, 0.0, 0.0};
-        }
-    };
-
-    int64_t line = wave * lpw + (laneUsed ? sub : 0);
-    int64_t gbase = wave * lpw;  // first line of this wave's group (uniform)
-    if (gbase >= nlines) {
-        if (CFL && lane == 0) cf.part[wave] = 1e38;
-        return;
-    }
-    double cmin = 1e38;
-    V5 Q[K], Qn[K];
-    load_group(line, Q);
-
-    for (;;) {
-        const bool more = gbase + groupStride < nlines;  // uniform across the wave
-        load_group(line + groupStride, Qn);  // unconditional: clamped to a valid line when !more
-
-        // stage A: U1 = Q - lambda dF(Q)
-        V5 F[K], Fm;
-        x_fluxes<M, K, LIM>(hc, rt, Q, cnt, srcL, srcR, F, Fm);
-        V5 U1[K];
+    for (int k = 0; k < K; k++) Q[k] = (k < cnt) ? load_cell<M, 1>(src + off + k, pitch) : V5{1.0, 1.0, 0.0, 0.0, 0.0};
+    x_stages<M, K, LIM>(hc, rt, Q, cnt, srcL, srcR, lambda);
+    double cmin = kCflNone;
 #pragma unroll
-        for (int k = 0; k < K; k++) U1[k] = axpy_update(Q[k], lambda, F[k], k == 0 ? Fm : F[k > 0 ? k - 1 : 0]);
-
-        // stage B: Q = .5((U1 + Q) - lambda dF(U1))
-        x_fluxes<M, K, LIM>(hc, rt, U1, cnt, srcL, srcR, F, Fm);
-        const bool own = laneUsed && line < nlines;
-        double *to = own ? dst + line_off(line) : mydummy;
-        const int64_t st = own ? pitch : nthr;
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            if (k < cnt) {
-                const V5 o = avg_update(add5(U1[k], Q[k]), lambda, F[k], k == 0 ? Fm : F[k > 0 ? k - 1 : 0]);
-                store_cell<M, 1>(own ? to + k : to, st, o);
-                if (CFL && own && x0 + k >= cf.lo && x0 + k < cf.hi) {
-                    const double u = cfl_of_cell<M, 1>(cf.a, o);
-                    cmin = (u < cmin) ? u : cmin;
-                }
+    for (int k = 0; k < K; k++) {
+        if (own && k < cnt) {
+            store_cell<M, 1>(dst + off + k, pitch, Q[k]);
+            if (CFL && x0 + k >= cf.lo && x0 + k < cf.hi) {
+                const double u = cfl_of_cell<M, 1>(cf.a, Q[k]);
+                cmin = (u < cmin) ? u : cmin;
             }
         }
-        if (!more) break;
-#pragma unroll
-        for (int k = 0; k < K; k++) Q[k] = Qn[k];
-        line += groupStride;
-        gbase += groupStride;
     }
-    if (CFL) {
-        cmin = wave_min(cmin);
-        if (lane == 0) cf.part[wave] = cmin;
-    }
+    if (CFL) cfl_fold(cf, wave, cmin);
 }
 
 // One wave's part of an X line: part `part` of `parts` (near-equal runs of
@@ -245,8 +215,9 @@ __global__ __launch_bounds__(256, (K <= 4) ? 2 : 1) void sweep_x(const double *s
 // so it forms its outputs alone; the window's outer cells only feed discarded
 // values. inplace: the waves of a line share a workgroup and every load of the
 // workgroup precedes the barrier while every store follows it, so no wave
-// overwrites a cell another has still to read. valid false: nothing is stored. CFL: cmin takes the minimum CFL
-// limit of the outputs at cells [cf.lo, cf.hi), nanc counts the NaN limits.
+// overwrites a cell another has still to read. valid false: nothing is stored.
+// CFL: cmin takes the minimum CFL limit of the outputs at cells [cf.lo, cf.hi),
+// nanc counts the NaN limits.
 template <class M, int K, int LIM, bool CFL>
 __device__ __forceinline__ void xp_body(const double *src, double *dst, int64_t pitch, int N, int part, int parts,
                                         bool valid, bool inplace, double lambda, const HydroConsts &hc, int rt,
@@ -255,14 +226,7 @@ __device__ __forceinline__ void xp_body(const double *src, double *dst, int64_t 
     const int lane = threadIdx.x & 63;
     const int s0 = (int)((int64_t)N * part / parts);  // first output cell of this part
     const int Wn = (int)((int64_t)N * (part + 1) / parts) - s0 + 8;
-    const int nl = (Wn + K - 1) / K;
-    const bool laneUsed = lane < nl;
-    const int srcL = laneUsed ? (lane == 0 ? nl - 1 : lane - 1) : lane;
-    const int srcR = laneUsed ? (lane == nl - 1 ? 0 : lane + 1) : lane;
     const int w0 = lane * K;
-    int cnt = Wn - w0;
-    cnt = cnt < K ? cnt : K;
-    if (!laneUsed) cnt = 0;
     V5 Q[K];
 #pragma unroll
     for (int k = 0; k < K; k++) {
@@ -270,21 +234,18 @@ __device__ __forceinline__ void xp_body(const double *src, double *dst, int64_t 
         g = (g < 0) ? g + N : g;
         g = (g >= N) ? g - N : g;
         g = (g < N) ? g : N - 1;
-        Q[k] = (k < cnt) ? load_cell<M, 1>(src + g, pitch) : V5{1.0, 1.0, 0.0, 0.0, 0.0};
+        // every lane of the window has K cells (the last one's run past it);
+        // idle lanes compute on a constant state
+        Q[k] = (w0 < Wn) ? load_cell<M, 1>(src + g, pitch) : V5{1.0, 1.0, 0.0, 0.0, 0.0};
     }
     if (inplace) __syncthreads();
-    V5 F[K], Fm;
-    x_fluxes<M, K, LIM>(hc, rt, Q, cnt, srcL, srcR, F, Fm);
-    V5 U1[K];
-#pragma unroll
-    for (int k = 0; k < K; k++) U1[k] = axpy_update(Q[k], lambda, F[k], k == 0 ? Fm : F[k > 0 ? k - 1 : 0]);
-    x_fluxes<M, K, LIM>(hc, rt, U1, cnt, srcL, srcR, F, Fm);
+    x_stages<M, K, LIM>(hc, rt, Q, K, (lane + 63) & 63, (lane + 1) & 63, lambda);
 #pragma unroll
     for (int k = 0; k < K; k++) {
         const int w = w0 + k;
-        if (k < cnt && valid && w >= 4 && w < Wn - 4) {
+        if (valid && w >= 4 && w < Wn - 4) {
             const int x = s0 + w - 4;
-            const V5 o = avg_update(add5(U1[k], Q[k]), lambda, F[k], k == 0 ? Fm : F[k > 0 ? k - 1 : 0]);
+            const V5 &o = Q[k];
             store_cell<M, 1>(dst + x, pitch, o);
             if (CFL && x >= cf.lo && x < cf.hi) {
                 const double u = cfl_of_cell<M, 1>(cf.a, o);
@@ -304,16 +265,13 @@ __global__ __launch_bounds__(512, 2) void sweep_xp(const double *src, double *ds
                                                   int rt, CflFuse cf)
 {
     if (lamp) lambda = lamp[0];  // time step kept on the device
-    const int wib = threadIdx.x >> 6;
+    const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // in a scalar register
     const int64_t line = blockIdx.x;
-    double cmin = 1e38;
+    double cmin = kCflNone;
     unsigned nanc = 0;  // not reported by the single-array fold
     xp_body<M, K, LIM, CFL>(src + line * (int64_t)N, dst + line * (int64_t)N, pitch, N, wib, parts, true, src == dst,
                             lambda, hc, rt, cf, cmin, nanc);
-    if (CFL) {
-        cmin = wave_min(cmin);
-        if ((threadIdx.x & 63) == 0) cf.part[(int64_t)blockIdx.x * (blockDim.x >> 6) + wib] = cmin;
-    }
+    if (CFL) cfl_fold(cf, (int64_t)blockIdx.x * (blockDim.x >> 6) + wib, cmin);
 }
 
 // ---------------------------------------------------------------------------
@@ -341,6 +299,7 @@ __device__ __forceinline__ void march_body(const double *col, double *out, int64
     double *outp = out + (int64_t)(j0 - 9) * sstride;  // address of output t - 9
     double *const dfr = defer + gtid;
     const int64_t dstride = 5 * nthr;
+    const double ml = -lambda, mhl = -.5 * lambda;
 
     const V5 one = V5{1.0, 1.0, 0.0, 0.0, 0.0};
     const V5 zero = V5{0.0, 0.0, 0.0, 0.0, 0.0};
@@ -354,7 +313,7 @@ __device__ __forceinline__ void march_body(const double *col, double *out, int64
 
     // Stage B runs one step behind stage A (it consumes the previous step's
     // U1), so the two long dependency chains of a step are independent and
-    // interleave. (U1+Q) of a cell is needed three steps after it is formed:
+    // interleave. (U1+Q)/2 of a cell is needed three steps after it is formed:
     // it waits in a 4-slot ring in LDS, private to the lane.
 
     auto step = [&](int t, V5 &Qcur, V5 &Qs, const V5 &U1p, V5 &U1n, const double &ep, double &en,
@@ -364,16 +323,17 @@ __device__ __forceinline__ void march_body(const double *col, double *out, int64
         // stage A at cell m-2
         {
             const double e = M::template floor<DIR>(hc, Qcur);
-            wn = M::prims(hc, Qcur, e);
+            wn = M::template prims<LIM>(hc, Qcur, e);
         }
         dn = wn - wp;
         V5 Lc;
         M::template face<LIM>(hc, wp, dp, dn, rt, Lc, Rn);  // faces of cell m-1
-        FAn = M::flux(hc, Rp, Lc);                           // interface (m-2)+1/2
-        U1n = axpy_update(Qs, lambda, FAn, FAp);
+        FAn = M::template flux<LIM>(hc, Rp, Lc);                           // interface (m-2)+1/2
+        const V5 dA = FAn - FAp;
+        U1n = axpy5(Qs, ml, dA);
         en = M::template floor<DIR>(hc, U1n);
         {
-            const V5 S2 = add5(U1n, Qs);  // (U1+Q) of cell m-2, used at step m+3
+            const V5 S2 = half_sum<M>(Qs, U1n, dA, mhl);  // (U1+Q)/2 of cell m-2, used at step m+3
             double *r = &ring[t & 3][0][lane];
             r[0] = S2.a;
             r[64] = S2.b;
@@ -384,14 +344,14 @@ __device__ __forceinline__ void march_body(const double *col, double *out, int64
         Qs = Qcur;
 
         // stage B at cell m-5, from the previous step's U1 (cell m-3)
-        w1n = M::prims(hc, U1p, ep);
+        w1n = M::template prims<LIM>(hc, U1p, ep);
         d1n = w1n - w1p;
         V5 L1c;
         M::template face<LIM>(hc, w1p, d1p, d1n, rt, L1c, R1n);  // faces of cell m-4
-        FBn = M::flux(hc, R1p, L1c);                              // interface (m-5)+1/2
+        FBn = M::template flux<LIM>(hc, R1p, L1c);                              // interface (m-5)+1/2
         const double *r = &ring[(t + 1) & 3][0][lane];  // slot of step t-3
         const V5 S5{r[0], r[64], r[128], r[192], r[256]};
-        const V5 o = avg_update(S5, lambda, FBn, FBp);  // cell m-5
+        const V5 o = axpy5(S5, mhl, FBn - FBp);  // cell m-5
 
         // Every step stores exactly 5 doubles: to the cell (outputs first..L-1),
         // to a deferred slot (earlier ones) or to this lane's dummy slot (no
@@ -465,15 +425,12 @@ __global__ __launch_bounds__(256) void sweep_march(const double *src, double *ds
 {
     if (lamp) lambda = lamp[0];  // time step kept on the device
     const int lane = threadIdx.x & 63;
-    const int wib = threadIdx.x >> 6;
+    const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // in a scalar register
     const int64_t wave = (int64_t)blockIdx.x * (blockDim.x >> 6) + wib;
     const bool inplace = src == dst;
     const int W = inplace ? 64 / S : 64;
     const int64_t colWaves = (columns + W - 1) / W;
-    if (wave >= (inplace ? colWaves : colWaves * S)) {
-        if (CFL && lane == 0) cf.part[wave] = 1e38;
-        return;
-    }
+    if (wave >= (inplace ? colWaves : colWaves * S)) return;
     const int64_t cw = inplace ? wave : wave % colWaves;
     const int s = inplace ? lane / W : (int)(wave / colWaves);
     const int64_t cid = cw * W + lane % W;
@@ -491,14 +448,11 @@ __global__ __launch_bounds__(256) void sweep_march(const double *src, double *ds
     const int64_t gtid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t nthr = (int64_t)gridDim.x * blockDim.x;
     __shared__ double sring[4][4][5][64];  // [wave in block][slot][variable][lane]
-    double cmin = 1e38;
+    double cmin = kCflNone;
     unsigned nanc = 0;  // not reported by the single-array fold
     march_body<M, DIR, LIM, CFL, NT>(src + off, dst + off, pitch, sstride, N, seglen, j0, L, inplace ? 4 : 0, lambda,
                                      hc, rt, defer, gtid, nthr, sring[wib], lane, cf, cmin, nanc);
-    if (CFL) {
-        cmin = wave_min(cmin);
-        if (lane == 0) cf.part[wave] = cmin;
-    }
+    if (CFL) cfl_fold(cf, wave, cmin);
 }
 
 }  // namespace imogen

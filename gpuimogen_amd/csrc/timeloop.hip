@@ -29,21 +29,50 @@ namespace imogen {
 
 // device clock: [0] time, [1] dTime, [2..4] lambda x, y, z
 constexpr int kClockDoubles = 8;
-constexpr int kCflSlot = 2056;  // tau + 7 spare + up to 2048 block minima (launch_cfl)
 constexpr int kMaxFluids = 4;
 
-// A limit tau that is not positive and below 1e36 (every cell NaN, or no cell
-// limiting: the reductions' 1e37 / 1e38 sentinels) takes no time step: dTime
-// = 0 and the refusal is counted in the device error word.
-__global__ void clock_advance(const double *__restrict__ cflOut, int nfluids, double cfl, double tmax,
-                              double hx, double hy, double hz, double *__restrict__ clk,
-                              unsigned long long *__restrict__ err)
+// Where a fluid's CFL limit comes from: the keys the previous iteration's last
+// sweep left (n = 0), or n block minima of a full pass. Either way the keys are
+// reset for this iteration's last sweep.
+struct ClockFluid {
+    unsigned long long *slots;  // null: this fluid never folds
+    const double *part;
+    int n, halve;
+};
+struct ClockFluids {
+    ClockFluid f[kMaxFluids];
+    int n;
+};
+
+// The reduction of every fluid's limit, dTime and the clock in one block (as
+// launches of their own: 4 us each in a small grid's iteration). A limit tau
+// that is not positive and below 1e36 (every cell NaN, or no cell limiting: the
+// reductions' 1e37 / 1e38 sentinels) takes no time step: dTime = 0 and the
+// refusal is counted in the device error word.
+__global__ __launch_bounds__(kCflSlots) void clock_advance(ClockFluids fl, double cfl, double tmax, double hx,
+                                                          double hy, double hz, double *__restrict__ clk,
+                                                          unsigned long long *__restrict__ err)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    double tau = cflOut[0];
-    for (int f = 1; f < nfluids; f++) {
-        const double t = cflOut[(int64_t)f * kCflSlot];
-        tau = (t < tau) ? t : tau;
+    __shared__ double part[kMaxFluids][kCflSlots / 64];
+    for (int f = 0; f < fl.n; f++) {
+        const ClockFluid &c = fl.f[f];
+        double m = 1e38;
+        if (c.slots) {
+            if (c.n == 0) m = order_value(c.slots[threadIdx.x]);
+            c.slots[threadIdx.x] = order_key(kCflNone);
+        }
+        for (int k = threadIdx.x; k < c.n; k += kCflSlots) m = (c.part[k] < m) ? c.part[k] : m;
+        m = wave_min(m);
+        if ((threadIdx.x & 63) == 0) part[f][threadIdx.x >> 6] = m;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    double tau = 1e38;
+    for (int f = 0; f < fl.n; f++) {
+        double m = part[f][0];
+        for (int k = 1; k < kCflSlots / 64; k++) m = (part[f][k] < m) ? part[f][k] : m;
+        m = fl.f[f].halve ? m / 2 : m;  // cflTimestep.cu:232-237
+        tau = (f == 0 || m < tau) ? m : tau;
     }
     double dt = cfl * tau;
     const double t = clk[0];
@@ -66,12 +95,12 @@ struct TimeloopImpl {
     double cflGamma[kMaxFluids];  // gamma of the CFL sound speed (the fluid's own)
     GeometryParams geo;
     double cfl = 0.4, tmax = HUGE_VAL;
-    double *dbuf = nullptr;  // clock, then one CFL slot per fluid
+    double *dbuf = nullptr;  // clock, then kCflBlocks CFL block minima per fluid
     hipGraphExec_t graph[6] = {nullptr};
     void *scratchAt = nullptr;  // scratch block the graphs were captured with
     size_t scratchBytes = 0;
     // CFL folded into the last sweep of each iteration: per fluid, whether its
-    // method and boundaries allow it, the per-wave minima and their capacity
+    // method and boundaries allow it, and its slots
     bool fuse[kMaxFluids] = {false};
     CflFuse cf[kMaxFluids];
     // drag source coupling fluid 0 (gas) and fluid 1 (dust); -1 = none
@@ -97,8 +126,8 @@ static void drop_graphs(TimeloopImpl *L)
         }
 }
 
-// CFL limit of fluid f into its slot (cfl_common in fluidstep.hip, on the device)
-static int cfl_of(TimeloopImpl *L, int f, hipStream_t s)
+// block minima of fluid f's CFL limit (cfl_common in fluidstep.hip, on the device)
+static int cfl_of(TimeloopImpl *L, int f, ClockFluid *c, hipStream_t s)
 {
     double *base;
     int64_t pitch;
@@ -112,12 +141,12 @@ static int cfl_of(TimeloopImpl *L, int f, hipStream_t s)
     double hmin = g.h[0];
     if (dim > 1 && g.h[1] < hmin) hmin = g.h[1];
     if (dim > 2 && g.h[2] < hmin) hmin = g.h[2];
-    const int method = (int)L->p[f].stepMethod;
-    const int xj = (method == METHOD_XINJIN) && dim > 1;
-    const int halve = (method == METHOD_HLL || method == METHOD_HLLC);
+    const int xj = (L->p[f].stepMethod == METHOD_XINJIN) && dim > 1;
+    double *part = L->dbuf + kClockDoubles + (int64_t)f * kCflBlocks;
+    c->part = part;
     const int slot = prof_begin(PROF_CFL, s);
-    rc = launch_cfl(base, pitch, L->fluid[f][0].partNumel[0], nullptr, L->cflGamma[f], 1, dim, xj, halve,
-                    g.h[0], g.h[1], g.h[2], hmin, L->dbuf + kClockDoubles + (int64_t)f * kCflSlot, s);
+    rc = launch_cfl_partials(base, pitch, L->fluid[f][0].partNumel[0], nullptr, L->cflGamma[f], 1, dim, xj, g.h[0],
+                             g.h[1], g.h[2], hmin, part, &c->n, s);
     prof_end(slot, s);
     return rc;
 }
@@ -170,20 +199,15 @@ static int source(TimeloopImpl *L, double fraction, hipStream_t s)
 static int iteration(TimeloopImpl *L, int it, bool fusedCfl, hipStream_t s)
 {
     int rc;
+    ClockFluids fl{};
+    fl.n = L->nf;
     for (int f = 0; f < L->nf; f++) {
-        if (fusedCfl && L->fuse[f]) {
-            const MGArray *a = L->fluid[f];
-            const int last = last_sweep_dir(a, it - 1, -1);
-            const int64_t n = sweep_waves(a->dim[0], a->dim[1], a->dim[2], last,
-                                          !sweep_out_of_place(a, (int)L->p[f].stepMethod, last));
-            rc = launch_cfl_final(L->cf[f].part, n, 1, L->dbuf + kClockDoubles + (int64_t)f * kCflSlot, s);
-        } else {
-            rc = cfl_of(L, f, s);
-        }
-        if (rc) return rc;
+        const FluidMethods m = L->p[f].stepMethod;
+        fl.f[f] = ClockFluid{L->cf[f].slots, nullptr, 0, m == METHOD_HLL || m == METHOD_HLLC};
+        if (!(fusedCfl && L->fuse[f]) && (rc = cfl_of(L, f, &fl.f[f], s))) return rc;
     }
-    hipLaunchKernelGGL(clock_advance, dim3(1), dim3(64), 0, s, L->dbuf + kClockDoubles, L->nf, L->cfl, L->tmax,
-                       L->geo.h[0], L->geo.h[1], L->geo.h[2], L->dbuf, state()->err);
+    hipLaunchKernelGGL(clock_advance, dim3(1), dim3(kCflSlots), 0, s, fl, L->cfl, L->tmax, L->geo.h[0], L->geo.h[1],
+                       L->geo.h[2], L->dbuf, state()->err);
     if ((rc = IM_LAUNCHED("clock_advance"))) return rc;
     if ((rc = source(L, 0.5, s))) return rc;
     for (int sgn = 1; sgn >= -1; sgn -= 2) {
@@ -244,31 +268,26 @@ int imogen_timeloop_create(MGArray *fluids, int nfluids, const GeometryParams *g
     for (int f = 0; f < nfluids; f++) {
         const int m = (int)L->p[f].stepMethod;
         MGArray *a = L->fluid[f];
-        bool ok = (m == METHOD_HLLC || m == METHOD_HLL);
-        int64_t cap = 0;
+        bool ok = (m == METHOD_HLLC || m == METHOD_HLL), any = false;
         for (int d = 1; d <= 3 && ok; d++) {
             const bool swept = (a->dim[1] == 1 && a->dim[2] == 1) ? (d == 1) : (a->dim[d - 1] > 3);
             if (!swept) continue;
             int lo, hi;
             if (a->dim[d - 1] <= 3 || cfl_keep_range(a, d, &lo, &hi)) ok = false;
-            for (int in = 0; in < 2; in++) {
-                const int64_t w = sweep_waves(a->dim[0], a->dim[1], a->dim[2], d, in);
-                cap = (w > cap) ? w : cap;
-            }
+            any = true;
         }
-        if (!ok || cap == 0) continue;
+        if (!ok || !any) continue;
         CflFuse &c = L->cf[f];
         c = CflFuse{};
-        if (IM_HIP(hipMalloc(&c.part, (size_t)cap * sizeof(double)))) {
-            c.part = nullptr;
+        if (IM_HIP(hipMalloc(&c.slots, kCflSlots * sizeof(unsigned long long)))) {
+            c.slots = nullptr;
             imogen_timeloop_destroy(T);
             return ERROR_NOMEM;
         }
         c.a = cfl_args(L, f);
-        c.cap = cap;
         L->fuse[f] = true;
     }
-    const size_t bytes = sizeof(double) * (kClockDoubles + (size_t)nfluids * kCflSlot);
+    const size_t bytes = sizeof(double) * (kClockDoubles + (size_t)nfluids * kCflBlocks);
     if (IM_HIP(hipMalloc(&L->dbuf, bytes))) {
         L->dbuf = nullptr;
         imogen_timeloop_destroy(T);
@@ -423,7 +442,7 @@ int imogen_timeloop_destroy(ImogenTimeloop *T)
     drop_graphs(&T->impl);
     if (T->impl.dbuf) (void)hipFree(T->impl.dbuf);
     for (int f = 0; f < T->impl.nf; f++)
-        if (T->impl.cf[f].part) (void)hipFree(T->impl.cf[f].part);
+        if (T->impl.cf[f].slots) (void)hipFree(T->impl.cf[f].slots);
     delete T;
     return SUCCESSFUL;
 }

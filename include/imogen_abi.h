@@ -255,9 +255,8 @@ int performFluidUpdate_3D(MGArray *fluid, ParallelTopology *parallelTopo, FluidS
  * harnesses that forbid hipMalloc). It takes its sweeps' scratch from a fixed
  * 64 MiB device array that each GPU the library runs on holds from the
  * library's first call until the process ends, and calls no hipMalloc/hipFree.
- * Limit: every sweep's scratch must fit 64 MiB (HLLC/HLL: 40 B per X-sweep
- * thread and 200 B per Y/Z marching lane, which fits every cube up to 256^3,
- * e.g. 29.5 MB at 192^3; Xin-Jin: 5 slabs, up to about 1.6 M cells); larger
+ * Limit: every sweep's scratch must fit 64 MiB (HLLC/HLL: 200 B per Y/Z
+ * marching lane, which fits every cube up to 256^3, e.g. 29.5 MB at 192^3; Xin-Jin: 5 slabs, up to about 1.6 M cells); larger
  * steps return ERROR_NOMEM before any launch. XYZ-ordered canisters only (ERROR_INVALID_ARGS for rotated ones).
  * All calls on a GPU share the array: they are ordered by the library's
  * stream; two executions that overlap on one GPU (e.g. a captured graph of
@@ -451,13 +450,13 @@ int imogen_ensemble_run(ImogenEnsemble *e, int firstIteration, int iterations, i
 /* Simulation time reached by every problem (nprob doubles; waits). */
 int imogen_ensemble_times(ImogenEnsemble *e, double *t);
 /* Times `trials` iterations per candidate and keeps, per size class (ny <= 128,
- * <= 256, <= 512), the fastest segment count S in {1, 2, 4} of the Y-sweep
- * march (chosen[3], optional, receives them), then per line-length group of
- * the X sweep (nx <= 64, <= 128, <= 192, <= 256, <= 368, <= 496, <= 512) the
- * fastest cells per lane K among the least K that fits and up to two more. A
- * candidate replaces the default (S = 1, 1, 2; the least K) only when it is 1 %
- * faster. The ensemble state advances during tuning and the clocks are reset
- * to 0 afterwards. */
+ * <= 256, <= 512), the fastest factor S in {1, 2, 4} on the number of segments
+ * the Y-sweep march cuts a column into (chosen[3], optional, receives them),
+ * then per line-length group of the X sweep (nx <= 64, <= 128, <= 192, <= 256,
+ * <= 368, <= 496, <= 512) the fastest cells per lane K among the least K that
+ * fits and up to two more. A candidate replaces the default (S = 1; the least
+ * K) only when it is 1 % faster. The ensemble state advances during tuning and
+ * the clocks are reset to 0 afterwards. */
 int imogen_ensemble_autotune(ImogenEnsemble *e, int trials, int *chosen);
 /* The X sweep's cells per lane and split mode (1: lines swept as two halves)
  * per line-length group as above (7 ints each; 0 for groups with no problem). */
