@@ -62,7 +62,7 @@ __global__ __launch_bounds__(256) void drag_kernel(double *__restrict__ g, doubl
                 overrun += (k < 0 && k != kDragInvalid);
             } else {
                 invalid += !drag_cell_defined(s.rg, s.rd, s.s0, s.u0);
-                f = exp(-dt * drag_logtrap_rate(c, s.rg, s.rd, s.s0, s.u0, dt, METHOD == DRAG_LOGTRAP3 ? 3 : 2));
+                f = exp_decay(-dt * drag_logtrap_rate(c, s.rg, s.rd, s.s0, s.u0, dt, METHOD == DRAG_LOGTRAP3 ? 3 : 2));
             }
             drag_apply(G, D, 1, s, f);
         }

@@ -2,11 +2,21 @@
 //
 // Drag rate: cukern_GasDustDrag_GeneralLinearCore + allregimeCdrag
 // (gpuclass/cudaSource2FluidDrag.cu:819-890). Powers of the normalised
-// temperature share one logarithm: x^a = exp(a ln x) (within a few ulp of pow).
+// temperature and of Re share their logarithms: x^a = exp(a ln x) (within a few
+// ulp of pow).
+//
+// The drag kernels are bound by the issue of these functions (the adaptive
+// integrator spent 98 % of its issue slots): exp and log below are half the
+// instructions of the math library's, which carry a second word through and
+// treat overflow, subnormals and signed zeros, and quotients are products with
+// refined reciprocals. One LogTrap2 call on 2.99e6 cells: 130 -> 70 us; two
+// adaptive calls on 96^3 cells: 304 -> 146 us; 4.2e6 cells of the learned
+// source's fallback: 368 -> 259 us.
 #pragma once
 #include <hip/hip_runtime.h>
 
 #include "../../include/imogen_abi.h"
+#include "sweep_device.h"
 
 namespace imogen {
 
@@ -23,21 +33,126 @@ struct DragCell {
     double s0, u0;   // |dv| and gas specific internal energy
 };
 
-__device__ __forceinline__ double pow_from_log(double lx, double a)
+// e^x - 1 = 2^n (1 + p) - 1 with n = round(x / ln 2) and p = r + r^2 Q(r) on the
+// remainder |r| <= ln 2 / 2; Q is a degree-9 Chebyshev fit of (e^r - 1 - r)/r^2
+// (p within 1e-16). ln 2 is split so that n ln2hi is exact. Overflow gives inf
+// and underflow 0 through the exponent up to |x| = 1e12; NaN stays.
+__device__ __forceinline__ double exp_parts(double x, int &n)
 {
-    return (a == 0.0) ? 1.0 : exp(a * lx);
+    const double f = rint(x * 0x1.71547652b82fep+0);
+    const double r = fma(-f, 0x1.d1cf79ac00000p-32, fma(-f, 0x1.62e42fec00000p-1, x));
+    n = (int)f;
+    double q = 0x1.ae5b5adb47a68p-26;
+    q = fma(q, r, 0x1.287e80b64b99ep-22);
+    q = fma(q, r, 0x1.71de80ebc2248p-19);
+    q = fma(q, r, 0x1.a019c8b3fdbdcp-16);
+    q = fma(q, r, 0x1.a01a018d205fbp-13);
+    q = fma(q, r, 0x1.6c16c174b881ap-10);
+    q = fma(q, r, 0x1.111111110e1c4p-7);
+    q = fma(q, r, 0x1.5555555554696p-5);
+    q = fma(q, r, 0x1.5555555555555p-3);
+    q = fma(q, r, 0.5);
+    return fma(r * r, q, r);
+}
+
+__device__ __forceinline__ double exp_fast(double x)
+{
+    int n;
+    const double p = exp_parts(x, n);
+    return ldexp(1.0 + p, n);
+}
+
+// e^x for an exponent of any size (a decay over a very long time): 0 below -1100,
+// and for a trial stage thrown far off, inf above 1100
+__device__ __forceinline__ double exp_decay(double x)
+{
+    return exp_fast(x < -1100.0 ? -1100.0 : x);
+}
+__device__ __forceinline__ double exp_any(double x)
+{
+    return exp_decay(x > 1100.0 ? 1100.0 : x);
+}
+
+// e^x and e^x - 1 for a decay exponent, the latter to full relative precision near 0 (n = 0: p itself)
+__device__ __forceinline__ double exp_fast(double x, double &em1)
+{
+    int n;
+    const double p = exp_parts(x < -1100.0 ? -1100.0 : x, n);
+    em1 = ldexp(p, n) + (ldexp(1.0, n) - 1.0);
+    return ldexp(1.0 + p, n);
+}
+
+// ln x for normal x > 0, NaN otherwise: x = 2^e m, sqrt(1/2) <= m < sqrt(2),
+// ln m = 2 atanh(s) with s = (m - 1)/(m + 1); (2 atanh(s)/s - 2)/s^2 is a
+// degree-6 Chebyshev fit in s^2 (within 7e-18 of ln m).
+__device__ __forceinline__ double log_fast(double x)
+{
+    double m = __builtin_amdgcn_frexp_mant(x);
+    int e = __builtin_amdgcn_frexp_exp(x);
+    const bool low = m < 0x1.6a09e667f3bcdp-1;
+    m = low ? m + m : m;
+    e -= low ? 1 : 0;
+    const double f = m - 1.0;
+    const double s = div_cr(f, m + 1.0);
+    const double z = s * s;
+    double q = 0x1.2a30988db636ap-3;
+    q = fma(q, z, 0x1.3a1a8e48fafadp-3);
+    q = fma(q, z, 0x1.7461ad42ed849p-3);
+    q = fma(q, z, 0x1.c71c6777b76fcp-3);
+    q = fma(q, z, 0x1.24924929220f5p-2);
+    q = fma(q, z, 0x1.999999999933cp-2);
+    q = fma(q, z, 0x1.5555555555555p-1);
+    const double d = (double)e;
+    const double l = fma(d, 0x1.62e42fec00000p-1, fma(s, 2.0, fma(d, 0x1.d1cf79ac00000p-32, s * (z * q))));
+    return x > 0 ? l : __builtin_nan("");
+}
+
+// What a cell's rates share.
+struct DragPre {
+    double ls;   // ln(delta rho_g): ln Re = ls + ln|dv| + viscpow ln T
+    double brg;  // beta / rho_g
+    double C;    // (rho_g + rho_d) epsilon
+};
+__device__ __forceinline__ DragPre drag_pre(const DragConsts &c, double rhog, double rhod)
+{
+    return DragPre{log_fast(c.delta * rhog), c.beta * rcp_nr(rhog), (rhog + rhod) * c.epsilon};
+}
+
+// a ln T; T^0 = 1 for any T
+__device__ __forceinline__ double scaled_log(double a, double lT)
+{
+    return (a == 0.0) ? 0.0 : a * lT;
+}
+
+// e^{-0.999/Kn} of the Cunningham factor; 0 in double below Kn = 1.3e-3, so the
+// floor changes nothing and keeps the quotient finite at Kn = 0
+__device__ __forceinline__ double cunningham_exp(double Kn)
+{
+    return exp_fast(-0.999 * rcp_nr(fmax(Kn, 1e-3)));
+}
+
+// C_d |dv| (rho_g + rho_d) epsilon at |dv| = s, ls1 = ln(delta rho_g s) and gas
+// internal energy u. With q = 8710 + Re the drag coefficient's sum is
+// [q (3 + .45 Re^.681) + .0509 Re^2] / (Re q), one reciprocal with the
+// Cunningham factor's.
+__device__ __forceinline__ double drag_rate(const DragConsts &c, const DragPre &pre, double s, double ls1, double u)
+{
+    const double lT = log_fast(c.alpha * u);
+    const double lRe = ls1 + scaled_log(c.viscpow, lT);
+    const double Re = exp_fast(lRe);
+    const double Kn = pre.brg * exp_fast(scaled_log(c.lampow, lT));
+    const double cunningham = fma(Kn, fma(0.558, cunningham_exp(Kn), 1.142), 1.0);
+    const double q = 8710 + Re;
+    const double num = fma(q, fma(.45, exp_fast(.681 * lRe), 3.0), .0509 * Re * Re);
+    return num * s * pre.C * rcp_nr(Re * q * cunningham);
 }
 
 // drag rate k(|dv|, u); no drag below |dv| = 1e-9 (:853-859)
 __device__ __forceinline__ double drag_k(const DragConsts &c, double rhog, double rhod, double magdv, double u)
 {
     if (magdv < 1e-9) return 0.0;
-    const double lT = log(c.alpha * u);
-    const double Re = c.delta * rhog * magdv * pow_from_log(lT, c.viscpow);
-    const double Kn = c.beta * pow_from_log(lT, c.lampow) / rhog;
-    const double cunningham = 1 + Kn * (1.142 + 0.558 * exp(-0.999 / Kn));
-    const double Cd = (3 / Re + .45 * exp(-.319 * log(Re)) + .0509 * Re / (8710 + Re)) / cunningham;
-    return Cd * magdv * (rhog + rhod) * c.epsilon;
+    const DragPre pre = drag_pre(c, rhog, rhod);
+    return drag_rate(c, pre, magdv, pre.ls + log_fast(magdv), u);
 }
 
 // |dv| and u_0 of a cell (cukern_prepareForERK_h0, :1883-1908)
@@ -46,16 +161,17 @@ __device__ __forceinline__ DragCell drag_load(const double *g, const double *d, 
     DragCell s;
     s.rg = g[0];
     s.rd = d[0];
+    const double irg = rcp_nr(s.rg), ird = rcp_nr(s.rd);
     const double E = g[p], gx = g[2 * p], gy = g[3 * p], gz = g[4 * p];
     const double dx = d[2 * p], dy = d[3 * p], dz = d[4 * p];
-    double dv = gx / s.rg - dx / s.rd;
+    double dv = gx * irg - dx * ird;
     double dvsq = dv * dv;
-    dv = gy / s.rg - dy / s.rd;
+    dv = gy * irg - dy * ird;
     dvsq += dv * dv;
-    dv = gz / s.rg - dz / s.rd;
+    dv = gz * irg - dz * ird;
     dvsq += dv * dv;
-    s.s0 = sqrt(dvsq);
-    s.u0 = (E - .5 * (gx * gx + gy * gy + gz * gz) / s.rg) / s.rg;
+    s.s0 = sqrt_nr(dvsq);
+    s.u0 = (E - .5 * (gx * gx + gy * gy + gz * gz) * irg) * irg;
     return s;
 }
 
@@ -63,21 +179,22 @@ __device__ __forceinline__ DragCell drag_load(const double *g, const double *d, 
 // energy change conserving total energy (:1632-1676).
 __device__ __forceinline__ void drag_apply(double *g, double *d, int64_t p, const DragCell &s, double f)
 {
-    const double mu = s.rd / (s.rg + s.rd) * s.rg;
-    const double rhoginv = 1.0 / s.rg;
+    const double irs = rcp_nr(s.rg + s.rd);
+    const double mu = s.rd * irs * s.rg;
+    const double rhoginv = rcp_nr(s.rg), rhodinv = rcp_nr(s.rd);
     double pdustsq = 0.0;
 #pragma unroll
     for (int c = 2; c <= 4; c++) {
         const double pg = g[c * p], pd = d[c * p];
         pdustsq -= pd * pd;
-        const double vstick = (pg + pd) / (s.rg + s.rd);
-        const double dv_t = (pg * rhoginv - pd / s.rd) * f;
+        const double vstick = (pg + pd) * irs;
+        const double dv_t = (pg * rhoginv - pd * rhodinv) * f;
         g[c * p] = s.rg * vstick + dv_t * mu;
         const double q = s.rd * vstick - dv_t * mu;
         d[c * p] = q;
         pdustsq += q * q;
     }
-    g[p] -= .5 * pdustsq / s.rd;
+    g[p] -= .5 * pdustsq * rhodinv;
 }
 
 // Exponential Euler update (cukern_ETDRK1, :1426-1530, with ACCOUNT_GRADP
@@ -86,59 +203,54 @@ __device__ __forceinline__ void drag_apply(double *g, double *d, int64_t p, cons
 // e^{-kt} with dpdt = 0 (NaN when k0 = 0, as there)
 __device__ __forceinline__ void drag_etd1_apply(double *g, double *d, int64_t p, double t, double k)
 {
-    const double rhoginv = 1.0 / g[0];
-    const double mu = g[0] * d[0] / (g[0] + d[0]);
+    const double rhoginv = rcp_nr(g[0]), rhodinv = rcp_nr(d[0]), irs = rcp_nr(g[0] + d[0]);
+    const double mu = g[0] * d[0] * irs;
+    const double e = exp_decay(-t * k);
+    // dpdt/k: 0, and NaN where the rate is cut to 0
+    const double driven = (k == 0.0) ? __builtin_nan("") : 0.0;
     double pdustsq = 0.0;
 #pragma unroll
     for (int c = 2; c <= 4; c++) {
         const double pg = g[c * p], pd = d[c * p];
         pdustsq -= pd * pd;
-        const double vstick = (pg + pd) / (g[0] + d[0]);
-        const double dv_i = pg * rhoginv - pd / d[0];
-        double dpdt = 0.0;
-        dpdt *= mu * rhoginv;
-        const double dv_t = dpdt / k + (dv_i - dpdt / k) * exp(-t * k);
+        const double vstick = (pg + pd) * irs;
+        const double dv_i = pg * rhoginv - pd * rhodinv;
+        const double dv_t = driven + (dv_i - driven) * e;
         g[c * p] = g[0] * vstick + dv_t * mu;
         const double q = d[0] * vstick - dv_t * mu;
         d[c * p] = q;
         pdustsq += q * q;
     }
-    g[p] -= .5 * pdustsq / d[0];
+    g[p] -= .5 * pdustsq * rhodinv;
 }
 
 // path-averaged drag rate of LogTrap2 / LogTrap3 (cukern_LogTrapSolve, :1546-1630)
 __device__ __forceinline__ double drag_logtrap_rate(const DragConsts &c, double rhog, double rhod, double dv0,
                                                     double u0, double t, int order)
 {
-    const double mu = rhod / (rhog + rhod);
-    double tmp0 = dv0, tmp1 = u0;
-    double ksum = drag_k(c, rhog, rhod, tmp0, tmp1);
-    double k = ksum;
-    double dv_t = dv0 * exp(-t * k);
-    double duint = -.5 * dv0 * dv0 * mu * expm1(-2 * k * t);
-    tmp0 = sqrt(dv_t * dv_t);
-    tmp1 += duint;
-    ksum += drag_k(c, rhog, rhod, tmp0, tmp1);
-    if (order == 3) {
-        tmp1 -= duint;
-        k = .25 * ksum;
-        dv_t = dv0 * exp(-t * k);
-        duint = -0.5 * dv0 * dv0 * mu * expm1(-2 * k * t);
-        tmp0 = sqrt(dv_t * dv_t);
-        tmp1 += duint;
-        const double khalf = drag_k(c, rhog, rhod, tmp0, tmp1);
-        return 0.16666666666666666667 * ksum + 0.66666666666666666667 * khalf;
-    }
+    const DragPre pre = drag_pre(c, rhog, rhod);
+    const double heat = -.5 * dv0 * dv0 * rhod * rcp_nr(rhog + rhod);
+    const double l0 = pre.ls + log_fast(dv0);
+    // the rate at |dv| = dv0 e^{-t a} and the energy its decay at rate a leaves
+    auto end_rate = [&](double a) {
+        double em1;
+        const double e = exp_fast(-t * a, em1);
+        const double s = dv0 * e;
+        return s < 1e-9 ? 0.0 : drag_rate(c, pre, s, l0 - t * a, u0 + heat * (em1 * (1.0 + e)));
+    };
+    const double k0 = dv0 < 1e-9 ? 0.0 : drag_rate(c, pre, dv0, l0, u0);
+    const double ksum = k0 + end_rate(k0);
+    if (order == 3) return 0.16666666666666666667 * ksum + 0.66666666666666666667 * end_rate(.25 * ksum);
     return .5 * ksum;
 }
 
 // d ln|dv| / dt along the relaxation path, with the gas heated by the
 // dissipated relative kinetic energy
-__device__ __forceinline__ double drag_exact_rhs(const DragConsts &c, double rhog, double rhod, double s0sq,
-                                                 double u0, double h, double y)
+__device__ __forceinline__ double drag_exact_rhs(const DragConsts &c, const DragPre &pre, double s0sq, double u0,
+                                                 double h, double y)
 {
-    const double s = exp(y);
-    return -drag_k(c, rhog, rhod, s, u0 + h * (s0sq - s * s));
+    const double s = exp_any(y);
+    return s < 1e-9 ? 0.0 : -drag_rate(c, pre, s, pre.ls + y, u0 + h * (s0sq - s * s));
 }
 
 // Whether the relaxation problem is defined on a cell: positive finite
@@ -171,38 +283,40 @@ __device__ __forceinline__ double drag_exact_ratio(const DragConsts &c, double r
         return __builtin_nan("");
     }
     if (s0 < 1e-9 || t <= 0) return 1.0;
-    const double hc = .5 * rhod / (rhog + rhod);
+    const DragPre pre = drag_pre(c, rhog, rhod);
+    const double hc = .5 * rhod * rcp_nr(rhog + rhod);
     const double s0sq = s0 * s0;
-    const double y0 = log(s0);
+    const double y0 = log_fast(s0);
     double y = y0, tt = 0.0, h = t;
-    double k1 = drag_exact_rhs(c, rhog, rhod, s0sq, u0, hc, y);
+    double k1 = drag_exact_rhs(c, pre, s0sq, u0, hc, y);
     if (!(fabs(k1) <= big)) {
         *steps = kDragInvalid;
         return __builtin_nan("");
     }
+    const double itol = 1.0 / c.tol;
     int n = 0;
     while (tt < t) {
         if (n >= 4096) {
             *steps = -n;
-            return exp(y - y0);
+            return exp_decay(y - y0);
         }
         if (h > t - tt) h = t - tt;
-        const double k2 = drag_exact_rhs(c, rhog, rhod, s0sq, u0, hc, y + h * (1.0 / 5) * k1);
-        const double k3 = drag_exact_rhs(c, rhog, rhod, s0sq, u0, hc, y + h * ((3.0 / 40) * k1 + (9.0 / 40) * k2));
-        const double k4 = drag_exact_rhs(c, rhog, rhod, s0sq, u0, hc,
+        const double k2 = drag_exact_rhs(c, pre, s0sq, u0, hc, y + h * (1.0 / 5) * k1);
+        const double k3 = drag_exact_rhs(c, pre, s0sq, u0, hc, y + h * ((3.0 / 40) * k1 + (9.0 / 40) * k2));
+        const double k4 = drag_exact_rhs(c, pre, s0sq, u0, hc,
                                          y + h * ((44.0 / 45) * k1 - (56.0 / 15) * k2 + (32.0 / 9) * k3));
-        const double k5 = drag_exact_rhs(c, rhog, rhod, s0sq, u0, hc,
+        const double k5 = drag_exact_rhs(c, pre, s0sq, u0, hc,
                                          y + h * ((19372.0 / 6561) * k1 - (25360.0 / 2187) * k2 +
                                                   (64448.0 / 6561) * k3 - (212.0 / 729) * k4));
-        const double k6 = drag_exact_rhs(c, rhog, rhod, s0sq, u0, hc,
+        const double k6 = drag_exact_rhs(c, pre, s0sq, u0, hc,
                                          y + h * ((9017.0 / 3168) * k1 - (355.0 / 33) * k2 + (46732.0 / 5247) * k3 +
                                                   (49.0 / 176) * k4 - (5103.0 / 18656) * k5));
         const double yn = y + h * ((35.0 / 384) * k1 + (500.0 / 1113) * k3 + (125.0 / 192) * k4 -
                                    (2187.0 / 6784) * k5 + (11.0 / 84) * k6);
-        const double k7 = drag_exact_rhs(c, rhog, rhod, s0sq, u0, hc, yn);
+        const double k7 = drag_exact_rhs(c, pre, s0sq, u0, hc, yn);
         double err = h * ((71.0 / 57600) * k1 - (71.0 / 16695) * k3 + (71.0 / 1920) * k4 -
                           (17253.0 / 339200) * k5 + (22.0 / 525) * k6 - (1.0 / 40) * k7);
-        err = fabs(err) / c.tol;
+        err = fabs(err) * itol;
         n++;
         if (!(err <= big)) err = 1e300;  // reject, shrink by the minimum factor
         if (err <= 1.0) {
@@ -213,28 +327,23 @@ __device__ __forceinline__ double drag_exact_ratio(const DragConsts &c, double r
             tt += h;
             y = yn;
             k1 = k7;
+            if (!(tt < t)) break;  // most cells take one step: no next one to size
         }
-        double f = (err > 0) ? 0.9 * pow(err, -0.2) : 5.0;
+        double f = (err > 0) ? 0.9 * exp_fast(-0.2 * log_fast(err)) : 5.0;
         f = (f < 0.2) ? 0.2 : ((f > 5.0) ? 5.0 : f);
         h *= f;
     }
     *steps = n;
-    return exp(y - y0);
+    return exp_decay(y - y0);
 }
 
 // ---- explicit midpoint / RK4 on |dv| (solveDragEMP :305-370, solveDragRK4 :372-467) ----
 
 // d|dv|/dt of cukern_GasDustDrag_GeneralAccel (:898-946); unlike the linear
 // core it has no small-|dv| cut-off
-__device__ __forceinline__ double drag_rk_accel(const DragConsts &c, double rhog, double rhod, double magdv,
-                                                double u)
+__device__ __forceinline__ double drag_rk_accel(const DragConsts &c, const DragPre &pre, double magdv, double u)
 {
-    const double lT = log(c.alpha * u);
-    const double Re = c.delta * rhog * magdv * pow_from_log(lT, c.viscpow);
-    const double Kn = c.beta * pow_from_log(lT, c.lampow) / rhog;
-    const double cunningham = 1 + Kn * (1.142 + 0.558 * exp(-0.999 / Kn));
-    const double Cd = (3 / Re + .45 * exp(-.319 * log(Re)) + .0509 * Re / (8710 + Re)) / cunningham;
-    return -(Cd * magdv * magdv * (rhog + rhod) * c.epsilon);
+    return -(drag_rate(c, pre, magdv, pre.ls + log_fast(magdv), u) * magdv);
 }
 
 // |dv| after dt; the stage and accumulator updates of cukern_SolveRK_single /
@@ -244,25 +353,25 @@ template <int METHOD>
 __device__ __forceinline__ double drag_rk_magdv(const DragConsts &c, double rhog, double rhod, double s0,
                                                 double u0, double dt)
 {
-    const double hc = .5 * rhod;
-    const double rs = rhog + rhod;
-    auto u_at = [&](double s) { return u0 + hc * (s0 * s0 - s * s) / rs; };
-    double k = drag_rk_accel(c, rhog, rhod, s0, u0);
+    const DragPre pre = drag_pre(c, rhog, rhod);
+    const double hc = .5 * rhod * rcp_nr(rhog + rhod);
+    auto u_at = [&](double s) { return u0 + hc * (s0 * s0 - s * s); };
+    double k = drag_rk_accel(c, pre, s0, u0);
     if (METHOD == DRAG_EMP) {
         const double acc = 0.0 * k;
         const double s = s0 + (.5 * dt) * k;
-        k = drag_rk_accel(c, rhog, rhod, s, u_at(s));
+        k = drag_rk_accel(c, pre, s, u_at(s));
         return s0 + dt * (acc + 1.0 * k);
     }
     double acc = 1.0 * k;
     double s = s0 + (.5 * dt) * k;
-    k = drag_rk_accel(c, rhog, rhod, s, u_at(s));
+    k = drag_rk_accel(c, pre, s, u_at(s));
     s = s0 + (.5 * dt) * k;
     acc += 2.0 * k;
-    k = drag_rk_accel(c, rhog, rhod, s, u_at(s));
+    k = drag_rk_accel(c, pre, s, u_at(s));
     s = s0 + (1.0 * dt) * k;
     acc += 2.0 * k;
-    k = drag_rk_accel(c, rhog, rhod, s, u_at(s));
+    k = drag_rk_accel(c, pre, s, u_at(s));
     return s0 + (dt / 6.0) * (acc + 1.0 * k);
 }
 
@@ -272,7 +381,7 @@ __device__ __forceinline__ DragCell drag_rk_load(const double *g, const double *
     DragCell s;
     s.rg = g[0];
     s.rd = d[0];
-    const double rgi = 1 / s.rg, rdi = 1 / s.rd;
+    const double rgi = rcp_nr(s.rg), rdi = rcp_nr(s.rd);
     double q = g[2 * p];
     double u = q * rgi - d[2 * p] * rdi;
     double momsq = q * q;
@@ -285,7 +394,7 @@ __device__ __forceinline__ DragCell drag_rk_load(const double *g, const double *
     u = q * rgi - d[4 * p] * rdi;
     momsq += q * q;
     dvsq += u * u;
-    s.s0 = sqrt(dvsq);
+    s.s0 = sqrt_nr(dvsq);
     s.u0 = (g[p] - .5 * momsq * rgi) * rgi;
     return s;
 }
@@ -296,15 +405,16 @@ __device__ __forceinline__ DragCell drag_rk_load(const double *g, const double *
 __device__ __forceinline__ void drag_rk_apply(double *g, double *d, int64_t p, double s1)
 {
     const double rhog = g[0], rhod = d[0];
+    const double irg = rcp_nr(rhog), ird = rcp_nr(rhod), irs = rcp_nr(rhog + rhod);
     double vs[3], dv[3];
 #pragma unroll
     for (int k = 0; k < 3; k++) {
         const double p1 = g[(k + 2) * p], p2 = d[(k + 2) * p];
-        vs[k] = (p1 + p2) / (rhog + rhod);
-        dv[k] = p1 / rhog - p2 / rhod;
+        vs[k] = (p1 + p2) * irs;
+        dv[k] = p1 * irg - p2 * ird;
     }
-    const double a = s1 / sqrt(dv[0] * dv[0] + dv[1] * dv[1] + dv[2] * dv[2]);
-    const double b = rhog * rhod / (rhog + rhod);
+    const double a = s1 / sqrt_nr(dv[0] * dv[0] + dv[1] * dv[1] + dv[2] * dv[2]);
+    const double b = rhog * rhod * irs;
     double dustmom = 0.0, dustmomfin = 0.0;
 #pragma unroll
     for (int k = 0; k < 3; k++) {
@@ -316,8 +426,8 @@ __device__ __forceinline__ void drag_rk_apply(double *g, double *d, int64_t p, d
         d[(k + 2) * p] = q;
         dustmomfin = (k == 0) ? q * q : dustmomfin + q * q;
     }
-    g[p] += .5 * (dustmom - dustmomfin) / rhod;
-    d[p] = .5 * dustmomfin / rhod + 1e-4 * rhod;
+    g[p] += .5 * (dustmom - dustmomfin) * ird;
+    d[p] = .5 * dustmomfin * ird + 1e-4 * rhod;
 }
 
 // The time interval of a drag call: a host value, or frac * dTime read on the

@@ -237,12 +237,8 @@ struct DragRate {
     double lT;   // ln(alpha u), the rate's temperature logarithm
 };
 
-// The surrogate path's FP64 arithmetic restates the drag formulas of
-// drag_device.h (drag_k, drag_load, drag_apply) with refined reciprocals
-// (rcp_nr, within 1-2 ulp) in place of IEEE divisions: its accuracy bar (the
-// residual tolerance against the exact integrator) is many orders above these
-// ulps, and a reciprocal shared by several quotients costs a fraction of an
-// IEEE division each.
+// The surrogate path restates drag_load and drag_apply on register cells, with
+// the densities' reciprocals kept between them.
 
 // |dv| and u_0 of a register cell, with 1/rho_g and 1/rho_d
 __device__ __forceinline__ DragCell learned_load(const double (&G)[5], const double (&D)[5], double &irg,
@@ -290,42 +286,27 @@ __device__ __forceinline__ void learned_apply(double (&G)[5], double (&D)[5], co
 // d ln|dv|/d tau = -1, d ln u/d tau = (rho_d/(rho_g+rho_d)) |dv_0|^2/u_0:
 //   g = -(1 + a) + (a viscpow + b lampow) rho_d |dv_0|^2 / ((rho_g+rho_d) u_0)
 // with a = d ln N/d ln Re, b = -d ln Cu/d ln Kn for C_d = N(Re)/Cu(Kn).
-__device__ __forceinline__ DragRate drag_k_parts(const DragConsts &c, double rhog, double rhod, double magdv,
-                                                 double u)
+__device__ __forceinline__ DragRate drag_k_parts(const DragConsts &c, const DragPre &pre, double rhog, double rhod,
+                                                 double magdv, double u)
 {
     DragRate r;
-    r.lT = log(c.alpha * u);
-    r.Re = c.delta * rhog * magdv * pow_from_log(r.lT, c.viscpow);
-    r.Kn = c.beta * pow_from_log(r.lT, c.lampow) * rcp_nr(rhog);
-    const double E = exp(-0.999 * rcp_nr(r.Kn));
+    r.lT = log_fast(c.alpha * u);
+    r.lRe = pre.ls + log_fast(magdv) + scaled_log(c.viscpow, r.lT);
+    r.Re = exp_fast(r.lRe);
+    r.Kn = pre.brg * exp_fast(scaled_log(c.lampow, r.lT));
+    const double E = cunningham_exp(r.Kn);
     const double cunningham = 1 + r.Kn * (1.142 + 0.558 * E);
-    r.lRe = log(r.Re);
-    const double p319 = exp(-.319 * r.lRe);
+    const double p319 = exp_fast(-.319 * r.lRe);
     const double iRe = rcp_nr(r.Re);
     const double q = 8710 + r.Re;
     const double iq = rcp_nr(q);
     const double N = 3 * iRe + .45 * p319 + .0509 * r.Re * iq;
     const double icun = rcp_nr(cunningham);
-    r.k = N * icun * magdv * (rhog + rhod) * c.epsilon;
+    r.k = N * icun * magdv * pre.C;
     const double a = (-3 * iRe - .319 * .45 * p319 + .0509 * 8710 * r.Re * iq * iq) * rcp_nr(N);
     const double b = -(1.142 * r.Kn + 0.558 * E * (r.Kn + 0.999)) * icun;
     r.g = -(1.0 + a) + (a * c.viscpow + b * c.lampow) * rhod * magdv * magdv * rcp_nr((rhog + rhod) * u);
     return r;
-}
-
-// The rate at |dv| = s1 = s0 e^{-x}, u = u1 from the initial one r0: ln Re
-// follows as ln Re0 - x + viscpow (ln T1 - ln T0), one logarithm fewer than
-// drag_k.
-__device__ __forceinline__ double drag_k_next(const DragConsts &c, const DragRate &r0, double rhog, double rhod,
-                                              double s1, double x, double u1)
-{
-    const double lT = log(c.alpha * u1);
-    const double Re = c.delta * rhog * s1 * pow_from_log(lT, c.viscpow);
-    const double Kn = c.beta * pow_from_log(lT, c.lampow) * rcp_nr(rhog);
-    const double cunningham = 1 + Kn * (1.142 + 0.558 * exp(-0.999 * rcp_nr(Kn)));
-    const double lRe = r0.lRe - x + c.viscpow * (lT - r0.lT);
-    const double N = 3 * rcp_nr(Re) + .45 * exp(-.319 * lRe) + .0509 * Re * rcp_nr(8710 + Re);
-    return N * rcp_nr(cunningham) * s1 * (rhog + rhod) * c.epsilon;
 }
 
 // raw features: ln(dt k0), ln(rho_d/rho_g), ln(|dv|/c_s), ln Re0, ln Kn0
@@ -362,7 +343,11 @@ __device__ __forceinline__ void learned_step(const DragConsts &c, const DragCell
     const bool defined = drag_cell_defined(s.rg, s.rd, s.s0, s.u0);
     const bool moving = defined && s.s0 >= 1e-9;
     DragRate r0 = {0.0, 1.0, 1.0, 0.0};
-    if (moving) r0 = drag_k_parts(c, s.rg, s.rd, s.s0, s.u0);
+    DragPre pre = {0.0, 0.0, 0.0};
+    if (moving) {
+        pre = drag_pre(c, s.rg, s.rd);
+        r0 = drag_k_parts(c, pre, s.rg, s.rd, s.s0, s.u0);
+    }
     float f[5];
     drag_features(c, s, r0, dt, f);
     bool inside = moving;
@@ -386,10 +371,11 @@ __device__ __forceinline__ void learned_step(const DragConsts &c, const DragCell
         const double kend = r0.k * (1.0 + tau * (r0.g + tau * q2));
         // end state implied by kbar; its true rate checks the prediction
         const double x = kbar * dt;
-        fac = exp(-x);
+        fac = exp_decay(-x);
         const double s1 = s.s0 * fac;
         const double u1 = s.u0 + .5 * s.rd * rcp_nr(s.rg + s.rd) * (s.s0 * s.s0 - s1 * s1);
-        const double k1 = drag_k_next(c, r0, s.rg, s.rd, s1, x, u1);
+        // ln Re follows the decay: ln(delta rho_g s1) = ln Re0 - viscpow ln T0 - x
+        const double k1 = drag_rate(c, pre, s1, r0.lRe - scaled_log(c.viscpow, r0.lT) - x, u1);
         const double ksimp = (r0.k + 4.0 * kmid + k1) * (1.0 / 6.0);
         const double e1 = fabs(dt * (k1 - kend));
         const double e2 = fabs(dt * (kbar - ksimp));
@@ -706,7 +692,7 @@ __global__ __launch_bounds__(256, 2) void ens_drag_kernel(const EnsDragTable *__
                 overrun += (k < 0 && k != kDragInvalid);
             } else {
                 invalid += !drag_cell_defined(s.rg, s.rd, s.s0, s.u0);
-                f = exp(-dt * drag_logtrap_rate(c, s.rg, s.rd, s.s0, s.u0, dt, method == DRAG_LOGTRAP3 ? 3 : 2));
+                f = exp_decay(-dt * drag_logtrap_rate(c, s.rg, s.rd, s.s0, s.u0, dt, method == DRAG_LOGTRAP3 ? 3 : 2));
             }
             drag_apply(G, D, 1, s, f);
         }
@@ -787,7 +773,8 @@ __global__ __launch_bounds__(256) void drag_samples_kernel(int64_t n, const doub
         const double tau_in = cells[i * 5 + 4];
         float f[5];
         float t[3];
-        const DragRate r0 = (s.s0 < 1e-9) ? DragRate{0.0, 1.0, 1.0, 0.0} : drag_k_parts(c, s.rg, s.rd, s.s0, s.u0);
+        const DragRate r0 = (s.s0 < 1e-9) ? DragRate{0.0, 1.0, 1.0, 0.0}
+                                               : drag_k_parts(c, drag_pre(c, s.rg, s.rd), s.rg, s.rd, s.s0, s.u0);
         const double dt = (r0.k > 0.0) ? tau_in / r0.k : 0.0;
         if (s.s0 < 1e-9 || !(dt > 0)) {
 #pragma unroll
