@@ -10,12 +10,14 @@
 // 5-slab layout (rho, E, px, py, pz; x fastest), with the reference's periodic
 // wrap along the swept line (cudaFluidStep.cu:1159-1162).
 //
-// Two data-movement schemes, both free of transposes:
+// Three data-movement schemes, all free of transposes through memory:
 //  * X (contiguous) lines: a wave owns whole lines or, for long or few lines,
 //    a part of one. Each lane holds K consecutive cells in registers; the
 //    one-cell neighbours it needs from the adjacent lanes (primitives, left
 //    face, flux) come by cross-lane shuffle. No LDS.
-//  * Y/Z (strided) lines: each lane marches along one column (coalesced over
+//  * Few Y/Z (strided) lines: a block turns 16 columns of up to 64 cells in LDS
+//    and takes them as the X sweep does.
+//  * Other Y/Z lines: each lane marches along one column (coalesced over
 //    x across the wave) keeping a register window of the two-stage stencil.
 //    Columns are split into segments for occupancy. A sweep whose output goes
 //    to a second state array (update_3d pairs such sweeps) may cut them
@@ -233,6 +235,59 @@ static int launch_x(const double *src, double *dst, int64_t pitch, int N, int64_
     return IM_LAUNCHED("sweep_x");
 }
 
+// Parts per column of a tiled Y/Z sweep, 0: the sweep marches. A march of few
+// columns is bound by its serial chain, at least 13 steps of about 1 us however
+// short its segments, and a tile by its waves' issue: about 8 us, and twice as
+// long once each SIMD has 8 waves. So tiles where their waves are few: 16384 of
+// whole columns, or 8192 of parts, which compute their 8 halo cells twice.
+// Device loop (HLLC, van Leer), us per iteration, march -> tile:
+//   whole: 16^3 107 -> 51   32^3 111 -> 59   48^3 133 -> 85   64^3 143 -> 104
+//          200 x 200 x 32 (20000 waves) 282 -> 257   128 x 128 x 64 (16384) 233 -> 227
+//          256 x 256 x 64 (65536) 635 -> 717   512 x 512 x 32 (131072) 1233 -> 1277
+//   parts: 64 x 100 66 -> 45   300^2 81 -> 60   512^2 (5120) 101 -> 89   700^2 (9100) 115 -> 111
+//          80^3 (12800) 174 -> 183   1024^2 (19456) 166 -> 168   128^3 (49152) 345 -> 412
+static int tile_parts(int64_t columns, int N, bool inplace)
+{
+    if (N <= 64) {
+        const int lpw = 64 / N;
+        return (columns + lpw - 1) / lpw <= 16384 ? 1 : 0;
+    }
+    const int parts = (N + 55) / 56;
+    return !inplace && columns * parts <= 8192 ? parts : 0;
+}
+
+bool sweep_cuts(int nx, int ny, int nz, int dir)
+{
+    const int N = (dir == 2) ? ny : nz;
+    return dir != 1 && tile_parts((int64_t)nx * ((dir == 2) ? nz : ny), N, false) != 1;
+}
+
+template <class M, int LIM>
+static int launch_tile(const double *src, double *dst, int64_t pitch, int nx, int ny, int nz, int dir, int parts,
+                       double lambda, const double *lamp, const HydroConsts &hc, int rt, const CflFuse &cf,
+                       hipStream_t s)
+{
+    const int N = (dir == 2) ? ny : nz;
+    const int64_t sstride = (dir == 2) ? (int64_t)nx : (int64_t)nx * ny;
+    const int64_t ostride = (dir == 2) ? (int64_t)nx * ny : (int64_t)nx;
+    const int64_t columns = (int64_t)nx * ((dir == 2) ? nz : ny);
+    const int lpw = parts == 1 ? 64 / N : 1;
+    const int waves = (kTileCols + lpw - 1) / lpw;
+    dim3 grid((unsigned)((columns + kTileCols - 1) / kTileCols), (unsigned)parts), block((unsigned)(64 * waves));
+#define IM_TILE(D, C)                                                                                        \
+    hipLaunchKernelGGL((sweep_tile<M, D, LIM, C>), grid, block, 0, s, src, dst, pitch, nx, sstride, ostride, \
+                       columns, N, parts, lambda, lamp, hc, rt, cf)
+    if (dir == 2) {
+        if (cf.slots) IM_TILE(2, true);
+        else IM_TILE(2, false);
+    } else {
+        if (cf.slots) IM_TILE(3, true);
+        else IM_TILE(3, false);
+    }
+#undef IM_TILE
+    return IM_LAUNCHED("sweep_tile");
+}
+
 template <class M, int LIM>
 static int launch_march(const double *src, double *dst, size_t scratchOff, int64_t pitch, int nx, int ny, int nz,
                         int dir, double lambda, const double *lamp, const HydroConsts &hc, int rt, const CflFuse &cf,
@@ -279,6 +334,8 @@ static int launch_dir(const double *src, double *dst, size_t off, int64_t pitch,
     const int slot = prof_begin(PROF_SWEEP_X + dir - 1, s);
     int rc;
     if (dir == 1) rc = launch_x<M, LIM>(src, dst, pitch, nx, (int64_t)ny * nz, lambda, lamp, hc, rt, cf, s);
+    else if (const int parts = tile_parts((int64_t)nx * ((dir == 2) ? nz : ny), (dir == 2) ? ny : nz, src == dst))
+        rc = launch_tile<M, LIM>(src, dst, pitch, nx, ny, nz, dir, parts, lambda, lamp, hc, rt, cf, s);
     else rc = launch_march<M, LIM>(src, dst, off, pitch, nx, ny, nz, dir, lambda, lamp, hc, rt, cf, s);
     prof_end(slot, s);
     return rc;
@@ -302,6 +359,8 @@ static int launch_method(const double *src, double *dst, size_t off, int64_t pit
     }
 }
 
+// The march's, also where a tiled sweep takes none: the grids that the
+// allocation-free step admits do not depend on that choice.
 int64_t sweep_scratch_bytes(int nx, int ny, int nz, int dir, bool inplace)
 {
     const int N = (dir == 1) ? nx : (dir == 2 ? ny : nz);

@@ -345,6 +345,10 @@ static unsigned paired_dirs(const MGArray *fluid, int method)
     if (d3[1] == 1 && d3[2] == 1) return 0;
     const bool x = d3[0] > 3, y = d3[1] > 3, z = d3[2] > 3;
     const unsigned dirs = (y && z) ? 6u : (x && y) ? 3u : (x && z) ? 5u : 0u;
+    // columns held whole gain nothing
+    bool cuts = false;
+    for (int d = 2; d <= 3; d++) cuts |= (dirs >> (d - 1) & 1) && sweep_cuts(d3[0], d3[1], d3[2], d);
+    if (!cuts) return 0;
     const size_t bytes = pair_bytes(fluid);
     if (!dirs || bytes > kPairBytes) return 0;
     int64_t need = 0;

@@ -83,6 +83,8 @@ bool scratch_available(size_t bytes);
 // Scratch bytes launch_fluid_sweep / launch_xinjin_sweep take for one sweep
 // (the launch shapes of fluid_sweep.hip and xinjin.hip).
 int64_t sweep_scratch_bytes(int nx, int ny, int nz, int dir, bool inplace);
+// Whether a sweep cuts its lines (and gains from a second array).
+bool sweep_cuts(int nx, int ny, int nz, int dir);
 int64_t xinjin_scratch_bytes(int64_t pitch, int nx, int ny, int nz, int dir);
 
 // Validates a 5-array fluid canister (slab views of one 5-slab owner, XYZ

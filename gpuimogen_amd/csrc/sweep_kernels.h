@@ -98,14 +98,14 @@ __device__ __forceinline__ double cfl_of_cell(const CflArgs &a, const V5 &o)
 // Interface fluxes of the cells a lane owns. F[k] is the flux at k+1/2 for
 // k < cnt; Fm is the flux at -1/2 (the left lane's last interface). The
 // method's floors are applied to U in place first.
-template <class M, int K, int LIM>
+template <class M, int K, int LIM, int DIR>
 __device__ __forceinline__ void x_fluxes(const HydroConsts &hc, int rt, V5 (&U)[K], int cnt, int srcL,
                                          int srcR, V5 (&F)[K], V5 &Fm)
 {
     V5 w[K];
 #pragma unroll
     for (int k = 0; k < K; k++) {
-        const double e = M::template floor<1>(hc, U[k]);
+        const double e = M::template floor<DIR>(hc, U[k]);
         w[k] = M::template prims<LIM>(hc, U[k], e);
     }
 
@@ -141,20 +141,20 @@ __device__ __forceinline__ void x_fluxes(const HydroConsts &hc, int rt, V5 (&U)[
 }
 
 // Both stages of the cells a lane owns, Q in, the new state out (in Q).
-template <class M, int K, int LIM>
+template <class M, int K, int LIM, int DIR = 1>
 __device__ __forceinline__ void x_stages(const HydroConsts &hc, int rt, V5 (&Q)[K], int cnt, int srcL, int srcR,
                                          double lambda)
 {
     const double ml = -lambda, mhl = -.5 * lambda;
     V5 F[K], Fm, U1[K];
-    x_fluxes<M, K, LIM>(hc, rt, Q, cnt, srcL, srcR, F, Fm);
+    x_fluxes<M, K, LIM, DIR>(hc, rt, Q, cnt, srcL, srcR, F, Fm);
 #pragma unroll
     for (int k = 0; k < K; k++) {
         const V5 dF = F[k] - (k == 0 ? Fm : F[k > 0 ? k - 1 : 0]);
         U1[k] = axpy5(Q[k], ml, dF);
         if (!M::floors) Q[k] = half_sum<M>(Q[k], U1[k], dF, mhl);
     }
-    x_fluxes<M, K, LIM>(hc, rt, U1, cnt, srcL, srcR, F, Fm);
+    x_fluxes<M, K, LIM, DIR>(hc, rt, U1, cnt, srcL, srcR, F, Fm);
 #pragma unroll
     for (int k = 0; k < K; k++) {
         const V5 dF = F[k] - (k == 0 ? Fm : F[k > 0 ? k - 1 : 0]);
@@ -453,6 +453,81 @@ __global__ __launch_bounds__(256) void sweep_march(const double *src, double *ds
     march_body<M, DIR, LIM, CFL, NT>(src + off, dst + off, pitch, sstride, N, seglen, j0, L, inplace ? 4 : 0, lambda,
                                      hc, rt, defer, gtid, nthr, sring[wib], lane, cf, cmin, nanc);
     if (CFL) cfl_fold(cf, wave, cmin);
+}
+
+// ---------------------------------------------------------------------------
+// Y/Z sweep of few columns: the X scheme on a tile turned in LDS
+// ---------------------------------------------------------------------------
+// A block takes 16 columns (a full cache line of each row) of up to 64 cells,
+// reads them row by row, and its waves take them out of the tile as the X sweep
+// takes its lines: one cell per lane, neighbours by cross-lane shuffle. Rows
+// are 17 doubles apart, so neither way of reading the tile meets a bank twice.
+// Columns of up to 64 cells are held whole (64 / N of them in a wave), in place
+// or not; longer ones go out of place in parts of up to 56 cells, with the 4
+// cells beyond each end as the X sweep's parts (part = blockIdx.y).
+constexpr int kTileCols = 16;
+
+template <class M, int DIR, int LIM, bool CFL>
+__global__ __launch_bounds__(1024) void sweep_tile(const double *src, double *dst, int64_t pitch, int nx,
+                                                   int64_t sstride, int64_t ostride, int64_t columns, int N, int parts,
+                                                   double lambda, const double *__restrict__ lamp, HydroConsts hc,
+                                                   int rt, CflFuse cf)
+{
+    if (lamp) lambda = lamp[0];  // time step kept on the device
+    constexpr int kLd = kTileCols + 1, kSlab = 64 * kLd;
+    __shared__ double tile[5 * kSlab];
+    // rows [0, Wn) of the tile are the column's cells r0 + row (periodic); the
+    // part's outputs are its rows [halo, Wn - halo)
+    const int halo = parts > 1 ? 4 : 0;
+    const int r0 = (int)((int64_t)N * blockIdx.y / parts) - halo;
+    const int Wn = (int)((int64_t)N * (blockIdx.y + 1) / parts) - r0 + halo;
+    const int64_t col0 = (int64_t)blockIdx.x * kTileCols;
+    // this thread's column and first row on the tile's global side
+    const int gc = threadIdx.x % kTileCols, g0 = threadIdx.x / kTileCols, gstep = blockDim.x / kTileCols;
+    const int64_t cid = col0 + gc;
+    const bool gown = cid < columns;
+    const int64_t other = cid / nx;
+    const int64_t goff = (cid - other * nx) + other * ostride;
+    for (int r = g0; r < Wn; r += gstep) {
+        int g = r0 + r;
+        g = (g < 0) ? g + N : ((g >= N) ? g - N : g);
+        if (gown) store_cell<M, DIR>(tile + r * kLd + gc, kSlab, load_cell<M, DIR>(src + goff + g * sstride, pitch));
+    }
+    __syncthreads();
+
+    const int lane = threadIdx.x & 63;
+    const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // in a scalar register
+    const int lpw = 64 / Wn;
+    const int sub = lane / Wn;
+    const int j = lane - sub * Wn;
+    const bool laneUsed = sub < lpw;
+    const int srcL = laneUsed ? sub * Wn + (j == 0 ? Wn - 1 : j - 1) : lane;
+    const int srcR = laneUsed ? sub * Wn + (j == Wn - 1 ? 0 : j + 1) : lane;
+    const int c = wib * lpw + sub;
+    const bool own = laneUsed && c < kTileCols && col0 + c < columns;
+    double *cell = tile + (own ? j * kLd + c : 0);
+    V5 Q[1] = {own ? load_cell<M, DIR>(cell, kSlab) : V5{1.0, 1.0, 0.0, 0.0, 0.0}};
+    x_stages<M, 1, LIM, DIR>(hc, rt, Q, 1, srcL, srcR, lambda);
+    double cmin = kCflNone;
+    if (own) {
+        store_cell<M, DIR>(cell, kSlab, Q[0]);
+        const int g = r0 + j;
+        if (CFL && j >= halo && j < Wn - halo && g >= cf.lo && g < cf.hi) cmin = cfl_of_cell<M, DIR>(cf.a, Q[0]);
+    }
+    __shared__ double least[16];
+    if (CFL) {
+        cmin = wave_min(cmin < kCflNone ? cmin : kCflNone);
+        if (lane == 0) least[wib] = cmin;
+    }
+    __syncthreads();
+    if (CFL && wib == 0) {
+        // one key for the block: 4096 waves of 64^3 cells on the keys took 8 us
+        cmin = wave_min(lane < (int)(blockDim.x >> 6) ? least[lane] : kCflNone);
+        if (lane == 0) fold_min(cf.slots + ((blockIdx.x + blockIdx.y * gridDim.x) & (kCflSlots - 1)), cmin);
+    }
+    for (int r = halo + g0; r < Wn - halo; r += gstep)
+        if (gown)
+            store_cell<M, DIR>(dst + goff + (r0 + r) * sstride, pitch, load_cell<M, DIR>(tile + r * kLd + gc, kSlab));
 }
 
 }  // namespace imogen
