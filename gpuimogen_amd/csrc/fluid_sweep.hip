@@ -183,7 +183,8 @@ static void *sweep_scratch(size_t off, size_t bytes)
 
 template <class M, int LIM>
 static int launch_x(const double *src, double *dst, int64_t pitch, int N, int64_t nlines, double lambda,
-                    const double *lamp, const HydroConsts &hc, int rt, const CflFuse &cf, hipStream_t s)
+                    const double *lamp, const HydroConsts &hc, int rt, const CflFuse &cf, GhostFill gf,
+                    bool *filled, hipStream_t s)
 {
     const XGeom g = x_geom(N, nlines);
     if (g.K == 0) return IM_FAIL(ERROR_NOIMPLEMENT, "X sweep supports lines of at most 1024 cells (got %d)", N);
@@ -191,9 +192,10 @@ static int launch_x(const double *src, double *dst, int64_t pitch, int N, int64_
     if (g.blocks > INT32_MAX) return IM_FAIL(ERROR_INVALID_ARGS, "too many lines for one X launch");
     dim3 grid((unsigned)g.blocks), block((unsigned)g.threads);
     if (g.parts) {
+        if (K > 1 && (gf.lo | gf.hi)) *filled = false;
 #define IM_XP(KK, C)                                                                                          \
     hipLaunchKernelGGL((sweep_xp<M, KK, LIM, C>), grid, block, 0, s, src, dst, pitch, N, g.parts, lambda, \
-                       lamp, hc, rt, cf)
+                       lamp, hc, rt, cf, gf)
 #define IM_XP_CASE(KK)                  \
     case KK:                            \
         if (cf.slots) IM_XP(KK, true);  \
@@ -212,7 +214,7 @@ static int launch_x(const double *src, double *dst, int64_t pitch, int N, int64_
     const bool full = (nl * K == N) && (64 % nl == 0);
 #define IM_X(KK, F, C)                                                                                        \
     hipLaunchKernelGGL((sweep_x<M, KK, LIM, F, C>), grid, block, 0, s, src, dst, pitch, N, nlines, nl, lambda, lamp, \
-                       hc, rt, cf)
+                       hc, rt, cf, gf)
 #define IM_X_CASE(KK)                               \
     case KK:                                        \
         if (full && cf.slots) IM_X(KK, true, true); \
@@ -265,7 +267,7 @@ bool sweep_cuts(int nx, int ny, int nz, int dir)
 template <class M, int LIM>
 static int launch_tile(const double *src, double *dst, int64_t pitch, int nx, int ny, int nz, int dir, int parts,
                        double lambda, const double *lamp, const HydroConsts &hc, int rt, const CflFuse &cf,
-                       hipStream_t s)
+                       GhostFill gf, hipStream_t s)
 {
     const int N = (dir == 2) ? ny : nz;
     const int64_t sstride = (dir == 2) ? (int64_t)nx : (int64_t)nx * ny;
@@ -276,7 +278,7 @@ static int launch_tile(const double *src, double *dst, int64_t pitch, int nx, in
     dim3 grid((unsigned)((columns + kTileCols - 1) / kTileCols), (unsigned)parts), block((unsigned)(64 * waves));
 #define IM_TILE(D, C)                                                                                        \
     hipLaunchKernelGGL((sweep_tile<M, D, LIM, C>), grid, block, 0, s, src, dst, pitch, nx, sstride, ostride, \
-                       columns, N, parts, lambda, lamp, hc, rt, cf)
+                       columns, N, parts, lambda, lamp, hc, rt, cf, gf)
     if (dir == 2) {
         if (cf.slots) IM_TILE(2, true);
         else IM_TILE(2, false);
@@ -291,12 +293,17 @@ static int launch_tile(const double *src, double *dst, int64_t pitch, int nx, in
 template <class M, int LIM>
 static int launch_march(const double *src, double *dst, size_t scratchOff, int64_t pitch, int nx, int ny, int nz,
                         int dir, double lambda, const double *lamp, const HydroConsts &hc, int rt, const CflFuse &cf,
-                        hipStream_t s)
+                        GhostFill gf, bool *filled, hipStream_t s)
 {
     const int64_t sstride = (dir == 2) ? (int64_t)nx : (int64_t)nx * ny;
     const int64_t ostride = (dir == 2) ? (int64_t)nx * ny : (int64_t)nx;
     const MarchGeom g = march_geom(nx, ny, nz, dir, src == dst);
     if (g.blocks > INT32_MAX) return IM_FAIL(ERROR_INVALID_ARGS, "too many columns for one march launch");
+    const int lastlen = g.N - (g.S - 1) * g.seglen;
+    if ((g.seglen < lastlen ? g.seglen : lastlen) < gf.reach()) {
+        if (gf.lo | gf.hi) *filled = false;
+        gf = GhostFill{};
+    }
     dim3 grid((unsigned)g.blocks), block(256);
     double *defer = (double *)sweep_scratch(scratchOff, (size_t)g.nthr * march_slots(src == dst) * sizeof(double));
     if (!defer) return IM_FAIL(ERROR_NOMEM, "no scratch for deferred outputs");
@@ -308,7 +315,7 @@ static int launch_march(const double *src, double *dst, size_t scratchOff, int64
                        pitch * 5 * (int64_t)sizeof(double) > (int64_t)256 << 20;
 #define IM_MARCH(D, C, T)                                                                                      \
     hipLaunchKernelGGL((sweep_march<M, D, LIM, C, T>), grid, block, 0, s, src, dst, pitch, nx, sstride, ostride, \
-                       g.columns, g.N, g.S, g.seglen, lambda, lamp, hc, rt, defer, cf)
+                       g.columns, g.N, g.S, g.seglen, lambda, lamp, hc, rt, defer, cf, gf)
 #define IM_MARCH_NT(D, C)             \
     do {                              \
         if (lines) IM_MARCH(D, C, true);  \
@@ -329,14 +336,15 @@ static int launch_march(const double *src, double *dst, size_t scratchOff, int64
 template <class M, int LIM>
 static int launch_dir(const double *src, double *dst, size_t off, int64_t pitch, int nx, int ny, int nz, int dir,
                       double lambda, const double *lamp, const HydroConsts &hc, int rt, const CflFuse &cf,
-                      hipStream_t s)
+                      GhostFill gf, bool *filled, hipStream_t s)
 {
     const int slot = prof_begin(PROF_SWEEP_X + dir - 1, s);
     int rc;
-    if (dir == 1) rc = launch_x<M, LIM>(src, dst, pitch, nx, (int64_t)ny * nz, lambda, lamp, hc, rt, cf, s);
+    *filled = true;
+    if (dir == 1) rc = launch_x<M, LIM>(src, dst, pitch, nx, (int64_t)ny * nz, lambda, lamp, hc, rt, cf, gf, filled, s);
     else if (const int parts = tile_parts((int64_t)nx * ((dir == 2) ? nz : ny), (dir == 2) ? ny : nz, src == dst))
-        rc = launch_tile<M, LIM>(src, dst, pitch, nx, ny, nz, dir, parts, lambda, lamp, hc, rt, cf, s);
-    else rc = launch_march<M, LIM>(src, dst, off, pitch, nx, ny, nz, dir, lambda, lamp, hc, rt, cf, s);
+        rc = launch_tile<M, LIM>(src, dst, pitch, nx, ny, nz, dir, parts, lambda, lamp, hc, rt, cf, gf, s);
+    else rc = launch_march<M, LIM>(src, dst, off, pitch, nx, ny, nz, dir, lambda, lamp, hc, rt, cf, gf, filled, s);
     prof_end(slot, s);
     return rc;
 }
@@ -344,17 +352,19 @@ static int launch_dir(const double *src, double *dst, size_t off, int64_t pitch,
 template <class M>
 static int launch_method(const double *src, double *dst, size_t off, int64_t pitch, int nx, int ny, int nz, int dir,
                          double lambda, const double *lamp, const HydroConsts &hc, int limiter, const CflFuse &cf,
-                         hipStream_t s)
+                         const GhostFill &gf, bool *filled, hipStream_t s)
 {
     switch (limiter) {
-    case LIMITER_OSPRE: return launch_dir<M, 0>(src, dst, off, pitch, nx, ny, nz, dir, lambda, lamp, hc, 0, cf, s);
-    case LIMITER_VANLEER: return launch_dir<M, 1>(src, dst, off, pitch, nx, ny, nz, dir, lambda, lamp, hc, 1, cf, s);
+    case LIMITER_OSPRE:
+        return launch_dir<M, 0>(src, dst, off, pitch, nx, ny, nz, dir, lambda, lamp, hc, 0, cf, gf, filled, s);
+    case LIMITER_VANLEER:
+        return launch_dir<M, 1>(src, dst, off, pitch, nx, ny, nz, dir, lambda, lamp, hc, 1, cf, gf, filled, s);
     case LIMITER_MINMOD:
     case LIMITER_SUPERBEE:
     case LIMITER_VANALBADA:
     case LIMITER_MC:
     case LIMITER_ZERO:
-        return launch_dir<M, -1>(src, dst, off, pitch, nx, ny, nz, dir, lambda, lamp, hc, limiter, cf, s);
+        return launch_dir<M, -1>(src, dst, off, pitch, nx, ny, nz, dir, lambda, lamp, hc, limiter, cf, gf, filled, s);
     default: return IM_FAIL(ERROR_INVALID_ARGS, "unknown slope limiter %d", limiter);
     }
 }
@@ -371,10 +381,11 @@ int64_t sweep_scratch_bytes(int nx, int ny, int nz, int dir, bool inplace)
 
 int launch_fluid_sweep(const double *src, double *dst, size_t scratchOff, int64_t pitch, int nx, int ny, int nz,
                        int dir, int method, double lambda, double gamma, double rhomin, double ciso, int limiter,
-                       hipStream_t s, const double *lamp, const CflFuse *cfl)
+                       hipStream_t s, const double *lamp, const CflFuse *cfl, const GhostFill &gf, bool *filled)
 {
     if (dir < 1 || dir > 3) return IM_FAIL(ERROR_INVALID_ARGS, "sweep direction %d", dir);
     const int N = (dir == 1) ? nx : (dir == 2 ? ny : nz);
+    *filled = false;
     if (N < 3) return SUCCESSFUL;  // cudaFluidStep.cu:301
     HydroConsts hc;
     hc.gamma = gamma;
@@ -388,9 +399,11 @@ int launch_fluid_sweep(const double *src, double *dst, size_t scratchOff, int64_
     hc.cisosq = ciso * ciso;
     const CflFuse cf = cfl ? *cfl : CflFuse{};
     if (method == METHOD_HLLC)
-        return launch_method<Hllc>(src, dst, scratchOff, pitch, nx, ny, nz, dir, lambda, lamp, hc, limiter, cf, s);
+        return launch_method<Hllc>(src, dst, scratchOff, pitch, nx, ny, nz, dir, lambda, lamp, hc, limiter, cf, gf,
+                                   filled, s);
     if (method == METHOD_HLL)
-        return launch_method<Hll>(src, dst, scratchOff, pitch, nx, ny, nz, dir, lambda, lamp, hc, limiter, cf, s);
+        return launch_method<Hll>(src, dst, scratchOff, pitch, nx, ny, nz, dir, lambda, lamp, hc, limiter, cf, gf,
+                                  filled, s);
     return IM_FAIL(ERROR_INVALID_ARGS, "sweep kernel for method %d", method);
 }
 

@@ -281,11 +281,46 @@ int fluid_boundary(MGArray *fluid, int direction, int xrules, const GeometryPara
     return rc;
 }
 
-// One directional update; to: where the swept state goes (null: in place;
-// HLLC and HLL only), scratchOff: as launch_fluid_sweep.
-static int sweep_1d(MGArray *fluid, double *to, size_t scratchOff, const FluidStepParams &params,
-                    const double *lampBase, const CflFuse *cfl)
+// The ghosts of direction d that its sweep can set: const, mirror or none on
+// either face, alike for all five arrays (the normal momentum's sign apart), of
+// the depth the sweeps know. false: fluid_boundary sets them.
+static bool ghost_fill(const MGArray *fluid, int d, GhostFill *gf)
 {
+    if (!is_xyz(fluid) || fluid->dim[d - 1] < kFillMin) return false;
+    if (fluid->haloSize > 0 && fluid->haloSize != kGhost) return false;
+    for (int i = 0; i < 5; i++) {
+        const ImogenBoundaryData *bd = (const ImogenBoundaryData *)fluid[i].boundaryConditions.externalData;
+        if (bd && bd->statics) return false;
+    }
+    for (int side = 0; side < 2; side++) {
+        int fill = kFillNone;
+        for (int i = 0; i < 5; i++) {
+            int f;
+            switch (fluid[i].boundaryConditions.mode[2 * (d - 1) + side]) {
+            case circular:
+            case stationary: f = kFillNone; break;
+            case extrapConstant: f = kFillConst; break;
+            case mirror:
+                f = kFillMirror;
+                if ((fluid[i].vectorComponent == d) != (i == 1 + d)) return false;
+                break;
+            default: return false;
+            }
+            if (i > 0 && f != fill) return false;
+            fill = f;
+        }
+        (side ? gf->hi : gf->lo) = fill;
+    }
+    return true;
+}
+
+// One directional update; to: where the swept state goes (null: in place;
+// HLLC and HLL only), scratchOff: as launch_fluid_sweep; filled (may be null:
+// the ghosts are left): whether the sweep has set the direction's ghosts.
+static int sweep_1d(MGArray *fluid, double *to, size_t scratchOff, const FluidStepParams &params,
+                    const double *lampBase, const CflFuse *cfl, bool *filled)
+{
+    if (filled) *filled = false;
     double *base;
     int64_t pitch;
     int rc = fluid_view(fluid, &base, &pitch);
@@ -305,10 +340,16 @@ static int sweep_1d(MGArray *fluid, double *to, size_t scratchOff, const FluidSt
     if (!st) return ERROR_CUDA_BLEW_UP;
     switch (params.stepMethod) {
     case METHOD_HLLC:
-    case METHOD_HLL:
-        return launch_fluid_sweep(base, to ? to : base, scratchOff, pitch, fluid->dim[0], fluid->dim[1],
+    case METHOD_HLL: {
+        GhostFill gf;
+        bool did = false;
+        const bool fill = filled && ghost_fill(fluid, dir, &gf);
+        rc = launch_fluid_sweep(base, to ? to : base, scratchOff, pitch, fluid->dim[0], fluid->dim[1],
                                   fluid->dim[2], dir, (int)params.stepMethod, lambda, params.thermoGamma, params.minimumRho,
-                                  params.Cisothermal, params.slopeLimiter, st->stream, lamp, cfl);
+                                  params.Cisothermal, params.slopeLimiter, st->stream, lamp, cfl, fill ? gf : GhostFill{}, &did);
+        if (filled) *filled = fill && did;
+        return rc;
+    }
     case METHOD_XINJIN:
         if (cfl) return IM_FAIL(ERROR_NOIMPLEMENT, "the CFL is not folded into Xin-Jin sweeps");
         return launch_xinjin_sweep(base, pitch, fluid->dim[0], fluid->dim[1], fluid->dim[2], dir, lambda,
@@ -319,7 +360,7 @@ static int sweep_1d(MGArray *fluid, double *to, size_t scratchOff, const FluidSt
 
 int update_1d(MGArray *fluid, const FluidStepParams &params, const double *lampBase, const CflFuse *cfl)
 {
-    return sweep_1d(fluid, nullptr, 0, params, lampBase, cfl);
+    return sweep_1d(fluid, nullptr, 0, params, lampBase, cfl, nullptr);
 }
 
 // Sweeps through a second state array. A sweep that need not leave its input
@@ -430,8 +471,9 @@ int update_3d(MGArray *fluid, const FluidStepParams &fsp, const double *lampBase
     }
     if (fluid->dim[1] == 1 && fluid->dim[2] == 1) {  // flux.cu:57-66
         p.stepDirection = 1;
-        rc = update_1d(fluid, p, lampBase, lastCfl ? &cf : nullptr);
-        if (rc) return rc;
+        bool filled;
+        rc = sweep_1d(fluid, nullptr, 0, p, lampBase, lastCfl ? &cf : nullptr, &filled);
+        if (rc || filled) return rc;
         return fluid_boundary(fluid, 1, 1, &fsp.geometry);
     }
     int sweep = (fsp.stepNumber + 3 * (fsp.stepDirection > 0)) % 6;
@@ -462,9 +504,11 @@ int update_3d(MGArray *fluid, const FluidStepParams &fsp, const double *lampBase
                 to = (at == fluid) ? second : base;
                 next = (at == fluid) ? other : fluid;
             }
-            rc = sweep_1d(at, to, off, p, lampBase, (lastCfl && d == last) ? &cf : nullptr);
+            bool filled;
+            rc = sweep_1d(at, to, off, p, lampBase, (lastCfl && d == last) ? &cf : nullptr, &filled);
             if (rc) return rc;
             at = next;
+            if (filled) continue;
             // the reference sets these boundaries with direction d rotated into
             // memory x (flux.cu:99-107): the x kernels' conventions along d
             rc = fluid_boundary(at, d, 1, &fsp.geometry);

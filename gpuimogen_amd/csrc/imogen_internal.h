@@ -120,6 +120,20 @@ int last_sweep_dir(const MGArray *fluid, int stepNumber, int stepDirection);
 // sweep.
 int cfl_keep_range(MGArray *fluid, int dir, int *lo, int *hi);
 
+// Const and mirror ghosts of depth kGhost, set by the sweep of their direction
+// (sweep_kernels.h). Both faces in one pass need lines of kFillMin cells, so that
+// neither reads what the other writes.
+constexpr int kGhost = 4, kFillMin = 3 * kGhost + 2;
+enum { kFillNone = 0, kFillConst = 1, kFillMirror = 2 };
+struct GhostFill {
+    int lo = kFillNone, hi = kFillNone;
+    // cells from a face in that the segment at the face must hold
+#if defined(__HIPCC__)
+    __host__ __device__
+#endif
+    int reach() const { return (lo == kFillMirror || hi == kFillMirror) ? 2 * kGhost + 1 : kGhost + 1; }
+};
+
 // Launchers (fluid_sweep.hip, xinjin.hip, statics.hip, cfl.hip, drag.hip)
 // method: METHOD_HLLC or METHOD_HLL. rhomin, ciso: HLL floors and isothermal
 // sound speed (-1: adiabatic). lamp: when not null, the kernels read lambda
@@ -129,9 +143,11 @@ int cfl_keep_range(MGArray *fluid, int dir, int *lo, int *hi);
 // src == dst: in place; otherwise the swept state goes to dst, another array
 // of the same pitch, and src stays as it was. scratchOff: bytes at the start of
 // the scratch block the launch leaves alone.
+// gf: ghosts of the swept direction the sweep may set as it stores them; *filled:
+// it has (false: they are still to be set).
 int launch_fluid_sweep(const double *src, double *dst, size_t scratchOff, int64_t pitch, int nx, int ny, int nz,
                        int dir, int method, double lambda, double gamma, double rhomin, double ciso, int limiter,
-                       hipStream_t s, const double *lamp = nullptr, const CflFuse *cfl = nullptr);
+                       hipStream_t s, const double *lamp, const CflFuse *cfl, const GhostFill &gf, bool *filled);
 int launch_xinjin_sweep(double *base, int64_t pitch, int nx, int ny, int nz, int dir, double lambda,
                         double gamma, double rhomin, hipStream_t s, const double *lamp = nullptr);
 // xrules: apply the memory-x kernels' conventions along direction dir (the

@@ -3,6 +3,7 @@
 // (ensemble.hip). See fluid_sweep.hip for the data-movement design.
 #pragma once
 #include "cfl_device.h"
+#include "imogen_internal.h"
 #include "sweep_device.h"
 
 namespace imogen {
@@ -92,6 +93,90 @@ __device__ __forceinline__ double cfl_of_cell(const CflArgs &a, const V5 &o)
 }
 
 // ---------------------------------------------------------------------------
+// ghost cells of the swept direction, set as the sweep stores them
+// ---------------------------------------------------------------------------
+// Const and mirror faces of depth kGhost with the memory-x conventions
+// (cudaStatics.cu:1308-1366), which the fluid step applies along the direction
+// it has just swept: a copy of cell kGhost (N - 1 - kGhost), or the mirror image
+// about it with the normal momentum turned. As launches of their own the two
+// faces cost 4.5 us at 64^3 (a quarter of an iteration), and 30 us along X at
+// 256^3, where they rewrite parts of every row's cache lines.
+// The cell whose value cell g takes; turned: with the normal momentum turned.
+__device__ __forceinline__ int ghost_source(int g, int N, const GhostFill &gf, bool &turned)
+{
+    const int lo = kGhost, hi = N - 1 - kGhost;
+    turned = false;
+    if (gf.lo && g < lo) {
+        turned = gf.lo == kFillMirror;
+        return turned ? 2 * lo - g : lo;
+    }
+    if (gf.hi && g > hi) {
+        turned = gf.hi == kFillMirror;
+        return turned ? 2 * hi - g : hi;
+    }
+    return g;
+}
+
+// Q[i] of a uniform i
+template <int K>
+__device__ __forceinline__ V5 pick5(const V5 (&Q)[K], int i)
+{
+    V5 v = Q[0];
+#pragma unroll
+    for (int k = 1; k < K; k++) v = sel5(k == i, Q[k], v);
+    return v;
+}
+
+// The ghosts among a lane's K cells from the lanes that hold their sources. Slot
+// k is cell w0 + k of its line's (or window's) numbering, whose cell 0 is lane
+// lbase's first; wlo, whi: the innermost cells next to the two faces in that
+// numbering (filled where gf says so), slotHi = whi mod K. All lanes reach it.
+template <int K>
+__device__ __forceinline__ void fill_ghosts(V5 (&Q)[K], int w0, int lbase, int wlo, int whi, int slotHi,
+                                            const GhostFill &gf)
+{
+    if (!(gf.lo | gf.hi)) return;
+    if (K == 1) {
+        int w = w0;
+        bool turned = false;
+        if (gf.lo && w0 < wlo) {
+            turned = gf.lo == kFillMirror;
+            w = turned ? 2 * wlo - w0 : wlo;
+        } else if (gf.hi && w0 > whi) {
+            turned = gf.hi == kFillMirror;
+            w = turned ? 2 * whi - w0 : whi;
+        }
+        V5 v = shfl5(Q[0], lbase + w);
+        v.c = turned ? -v.c : v.c;
+        Q[0] = v;
+        return;
+    }
+    if (gf.lo != kFillMirror && gf.hi != kFillMirror) {
+        // one exchange for both faces: each lane's source is its nearer face's
+        const bool upper = 2 * w0 > wlo + whi;
+        const bool src = w0 <= whi && w0 + K > whi;  // holds the upper face's source
+        const V5 v = shfl5(sel5(src, pick5<K>(Q, slotHi), pick5<K>(Q, wlo % K)), lbase + (upper ? whi : wlo) / K);
+        const bool fill = upper ? gf.hi : gf.lo;
+#pragma unroll
+        for (int k = 0; k < K; k++) Q[k] = sel5(fill && (upper ? w0 + k > whi : w0 + k < wlo), v, Q[k]);
+        return;
+    }
+#pragma unroll
+    for (int side = 0; side < 2; side++) {
+        const int fill = side ? gf.hi : gf.lo, we = side ? whi : wlo, out = side ? 1 : -1;
+        if (!fill) continue;
+#pragma unroll
+        for (int i = 1; i <= kGhost; i++) {
+            const int ws = fill == kFillMirror ? we - out * i : we;
+            V5 v = shfl5(pick5<K>(Q, ws % K), lbase + ws / K);
+            v.c = fill == kFillMirror ? -v.c : v.c;
+#pragma unroll
+            for (int k = 0; k < K; k++) Q[k] = sel5(w0 + k == we + out * i, v, Q[k]);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // X sweep: lanes own K consecutive cells of a line
 // ---------------------------------------------------------------------------
 
@@ -171,7 +256,8 @@ __device__ __forceinline__ void x_stages(const HydroConsts &hc, int rt, V5 (&Q)[
 template <class M, int K, int LIM, bool FULL, bool CFL>
 __global__ __launch_bounds__(256, (K <= 4) ? 2 : 1) void sweep_x(const double *src, double *dst, int64_t pitch, int N,
                                                int64_t nlines, int nl, double lambda,
-                                               const double *__restrict__ lamp, HydroConsts hc, int rt, CflFuse cf)
+                                               const double *__restrict__ lamp, HydroConsts hc, int rt, CflFuse cf,
+                                               GhostFill gf)
 {
     if (lamp) lambda = lamp[0];  // time step kept on the device
     const int lane = threadIdx.x & 63;
@@ -195,6 +281,8 @@ __global__ __launch_bounds__(256, (K <= 4) ? 2 : 1) void sweep_x(const double *s
 #pragma unroll
     for (int k = 0; k < K; k++) Q[k] = (k < cnt) ? load_cell<M, 1>(src + off + k, pitch) : V5{1.0, 1.0, 0.0, 0.0, 0.0};
     x_stages<M, K, LIM>(hc, rt, Q, cnt, srcL, srcR, lambda);
+    fill_ghosts<K>(Q, laneUsed ? x0 : lane, laneUsed ? lbase : 0, kGhost, N - 1 - kGhost,
+                   FULL ? (5 * K - 1 - kGhost) % K : (N - 1 - kGhost) % K, gf);
     double cmin = kCflNone;
 #pragma unroll
     for (int k = 0; k < K; k++) {
@@ -217,11 +305,13 @@ __global__ __launch_bounds__(256, (K <= 4) ? 2 : 1) void sweep_x(const double *s
 // workgroup precedes the barrier while every store follows it, so no wave
 // overwrites a cell another has still to read. valid false: nothing is stored.
 // CFL: cmin takes the minimum CFL limit of the outputs at cells [cf.lo, cf.hi),
-// nanc counts the NaN limits.
+// nanc counts the NaN limits. gf: K = 1 only (with K = 3 the parts of a mirrored
+// 321 x 287 x 305 box took 906 us instead of 793 and its launch of 42, and a
+// periodic 1024 x 1024 plane, which fills nothing, 40 us instead of 33).
 template <class M, int K, int LIM, bool CFL>
 __device__ __forceinline__ void xp_body(const double *src, double *dst, int64_t pitch, int N, int part, int parts,
                                         bool valid, bool inplace, double lambda, const HydroConsts &hc, int rt,
-                                        const CflFuse &cf, double &cmin, unsigned &nanc)
+                                        const CflFuse &cf, const GhostFill &gf, double &cmin, unsigned &nanc)
 {
     const int lane = threadIdx.x & 63;
     const int s0 = (int)((int64_t)N * part / parts);  // first output cell of this part
@@ -240,6 +330,10 @@ __device__ __forceinline__ void xp_body(const double *src, double *dst, int64_t 
     }
     if (inplace) __syncthreads();
     x_stages<M, K, LIM>(hc, rt, Q, K, (lane + 63) & 63, (lane + 1) & 63, lambda);
+    // window cell 4 is the part's first
+    if (K == 1)
+        fill_ghosts<K>(Q, w0, 0, kGhost + 4, N - 1 - kGhost - s0 + 4, 0,
+                       GhostFill{part == 0 ? gf.lo : kFillNone, part == parts - 1 ? gf.hi : kFillNone});
 #pragma unroll
     for (int k = 0; k < K; k++) {
         const int w = w0 + k;
@@ -262,7 +356,7 @@ __device__ __forceinline__ void xp_body(const double *src, double *dst, int64_t 
 template <class M, int K, int LIM, bool CFL>
 __global__ __launch_bounds__(512, 2) void sweep_xp(const double *src, double *dst, int64_t pitch, int N, int parts,
                                                   double lambda, const double *__restrict__ lamp, HydroConsts hc,
-                                                  int rt, CflFuse cf)
+                                                  int rt, CflFuse cf, GhostFill gf)
 {
     if (lamp) lambda = lamp[0];  // time step kept on the device
     const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // in a scalar register
@@ -270,7 +364,7 @@ __global__ __launch_bounds__(512, 2) void sweep_xp(const double *src, double *ds
     double cmin = kCflNone;
     unsigned nanc = 0;  // not reported by the single-array fold
     xp_body<M, K, LIM, CFL>(src + line * (int64_t)N, dst + line * (int64_t)N, pitch, N, wib, parts, true, src == dst,
-                            lambda, hc, rt, cf, cmin, nanc);
+                            lambda, hc, rt, cf, gf, cmin, nanc);
     if (CFL) cfl_fold(cf, (int64_t)blockIdx.x * (blockDim.x >> 6) + wib, cmin);
 }
 
@@ -291,7 +385,7 @@ __device__ __forceinline__ void march_body(const double *col, double *out, int64
                                            int seglen, int j0, int L, int first, double lambda,
                                            const HydroConsts &hc, int rt, double *__restrict__ defer, int64_t gtid,
                                            int64_t nthr, double (*ring)[5][64], int lane, const CflFuse &cf,
-                                           double &cmin, unsigned &nanc)
+                                           const GhostFill &gf, double &cmin, unsigned &nanc)
 {
     // wrapped sweep index of the first load (m = j0 - 4), in [0, N)
     int mw = (j0 - 4) % N;
@@ -410,6 +504,25 @@ __device__ __forceinline__ void march_body(const double *col, double *out, int64
         const V5 o = load_cell<M, DIR, NT>(defer + gtid + (int64_t)oi * 5 * nthr, nthr);
         store_cell<M, DIR, NT>(out + (int64_t)(j0 + oi) * sstride, pitch, o);
     }
+
+    // the faces' ghosts from the cells this lane has stored: a segment at a face
+    // holds the ghosts and their sources (the launcher sees to it)
+    if (gf.lo && j0 == 0 && L > 0) {
+        for (int g = 0; g < kGhost; g++) {
+            bool turned;
+            V5 v = load_cell<M, DIR, NT>(out + (int64_t)ghost_source(g, N, gf, turned) * sstride, pitch);
+            if (turned) v.c = -v.c;
+            store_cell<M, DIR, NT>(out + (int64_t)g * sstride, pitch, v);
+        }
+    }
+    if (gf.hi && j0 + L == N && L > 0) {
+        for (int g = N - kGhost; g < N; g++) {
+            bool turned;
+            V5 v = load_cell<M, DIR, NT>(out + (int64_t)ghost_source(g, N, gf, turned) * sstride, pitch);
+            if (turned) v.c = -v.c;
+            store_cell<M, DIR, NT>(out + (int64_t)g * sstride, pitch, v);
+        }
+    }
 }
 
 // Columns are numbered x + nx * o (o: the other direction), so a wave's
@@ -421,7 +534,8 @@ template <class M, int DIR, int LIM, bool CFL, bool NT>
 __global__ __launch_bounds__(256) void sweep_march(const double *src, double *dst, int64_t pitch, int nx,
                                                    int64_t sstride, int64_t ostride, int64_t columns, int N, int S,
                                                    int seglen, double lambda, const double *__restrict__ lamp,
-                                                   HydroConsts hc, int rt, double *__restrict__ defer, CflFuse cf)
+                                                   HydroConsts hc, int rt, double *__restrict__ defer, CflFuse cf,
+                                                   GhostFill gf)
 {
     if (lamp) lambda = lamp[0];  // time step kept on the device
     const int lane = threadIdx.x & 63;
@@ -451,7 +565,7 @@ __global__ __launch_bounds__(256) void sweep_march(const double *src, double *ds
     double cmin = kCflNone;
     unsigned nanc = 0;  // not reported by the single-array fold
     march_body<M, DIR, LIM, CFL, NT>(src + off, dst + off, pitch, sstride, N, seglen, j0, L, inplace ? 4 : 0, lambda,
-                                     hc, rt, defer, gtid, nthr, sring[wib], lane, cf, cmin, nanc);
+                                     hc, rt, defer, gtid, nthr, sring[wib], lane, cf, gf, cmin, nanc);
     if (CFL) cfl_fold(cf, wave, cmin);
 }
 
@@ -471,7 +585,7 @@ template <class M, int DIR, int LIM, bool CFL>
 __global__ __launch_bounds__(1024) void sweep_tile(const double *src, double *dst, int64_t pitch, int nx,
                                                    int64_t sstride, int64_t ostride, int64_t columns, int N, int parts,
                                                    double lambda, const double *__restrict__ lamp, HydroConsts hc,
-                                                   int rt, CflFuse cf)
+                                                   int rt, CflFuse cf, GhostFill gf)
 {
     if (lamp) lambda = lamp[0];  // time step kept on the device
     constexpr int kLd = kTileCols + 1, kSlab = 64 * kLd;
@@ -525,9 +639,14 @@ __global__ __launch_bounds__(1024) void sweep_tile(const double *src, double *ds
         cmin = wave_min(lane < (int)(blockDim.x >> 6) ? least[lane] : kCflNone);
         if (lane == 0) fold_min(cf.slots + ((blockIdx.x + blockIdx.y * gridDim.x) & (kCflSlots - 1)), cmin);
     }
-    for (int r = halo + g0; r < Wn - halo; r += gstep)
-        if (gown)
-            store_cell<M, DIR>(dst + goff + (r0 + r) * sstride, pitch, load_cell<M, DIR>(tile + r * kLd + gc, kSlab));
+    for (int r = halo + g0; r < Wn - halo; r += gstep) {
+        if (gown) {
+            bool turned;
+            V5 q = load_cell<M, DIR>(tile + (ghost_source(r0 + r, N, gf, turned) - r0) * kLd + gc, kSlab);
+            if (turned) q.c = -q.c;
+            store_cell<M, DIR>(dst + goff + (r0 + r) * sstride, pitch, q);
+        }
+    }
 }
 
 }  // namespace imogen
