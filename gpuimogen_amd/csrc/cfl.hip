@@ -85,9 +85,13 @@ __global__ __launch_bounds__(256) void cfl_pass1(const double *__restrict__ q, i
     }
 }
 
+// out, errOut: pinned host memory, so that the caller has both after one wait
 __global__ __launch_bounds__(256) void cfl_pass2(const double *__restrict__ blockMin, int nblocks,
-                                                 double halve, double *__restrict__ out)
+                                                 double halve, double *__restrict__ out,
+                                                 const unsigned long long *__restrict__ err,
+                                                 unsigned long long *__restrict__ errOut)
 {
+    if (threadIdx.x < ERRW_SLOTS) errOut[threadIdx.x] = err[threadIdx.x];
     double m = 1e38;
     for (int k = threadIdx.x; k < nblocks; k += blockDim.x) m = (blockMin[k] < m) ? blockMin[k] : m;
     m = wave_min(m);
@@ -129,16 +133,19 @@ int launch_cfl_partials(const double *base, int64_t pitch, int64_t n, const doub
     return IM_LAUNCHED("cfl_pass1");
 }
 
-// devOut[0] receives tau; devOut[8..] is used as block scratch (kCflBlocks).
+// st->pinned[0] receives tau and st->errHost the error counters.
 int launch_cfl(const double *base, int64_t pitch, int64_t n, const double *cs, double gamma, int fused,
-               int dim, int xinjin, int halve, double hx, double hy, double hz, double hmin, double *devOut,
-               hipStream_t s)
+               int dim, int xinjin, int halve, double hx, double hy, double hz, double hmin, hipStream_t s)
 {
+    DeviceState *st = state();
     int blocks;
-    int rc = launch_cfl_partials(base, pitch, n, cs, gamma, fused, dim, xinjin, hx, hy, hz, hmin, devOut + 8,
-                                 &blocks, s);
+    int rc = pinned_buffers(st);
     if (rc) return rc;
-    hipLaunchKernelGGL(cfl_pass2, dim3(1), dim3(256), 0, s, devOut + 8, blocks, halve ? 1.0 : 0.0, devOut);
+    rc = launch_cfl_partials(base, pitch, n, cs, gamma, fused, dim, xinjin, hx, hy, hz, hmin, st->devScalars, &blocks,
+                             s);
+    if (rc) return rc;
+    hipLaunchKernelGGL(cfl_pass2, dim3(1), dim3(256), 0, s, st->devScalars, blocks, halve ? 1.0 : 0.0, st->pinned,
+                       st->err, st->errHost);
     return IM_LAUNCHED("cfl_pass2");
 }
 

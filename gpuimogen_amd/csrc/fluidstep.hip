@@ -671,18 +671,12 @@ static int cfl_common(MGArray *fluid, MGArray *csound, GeometryParams *geom, int
     if (!st) return ERROR_CUDA_BLEW_UP;
     const int slot = prof_begin(PROF_CFL, st->stream);
     rc = launch_cfl(base, pitch, fluid->partNumel[0], csound ? csound->devicePtr[0] : nullptr, gamma,
-                    csound ? 0 : 1, dim, xj, halve, geom->h[0], geom->h[1], geom->h[2], hmin, st->devScalars,
-                    st->stream);
+                    csound ? 0 : 1, dim, xj, halve, geom->h[0], geom->h[1], geom->h[2], hmin, st->stream);
     prof_end(slot, st->stream);
     if (rc) return rc;
-    rc = pinned_buffers(st);
-    if (rc) return rc;
-    rc = IM_HIP(hipMemcpyAsync(st->pinned, st->devScalars, sizeof(double), hipMemcpyDeviceToHost, st->stream));
-    if (rc) return rc;
-    rc = IM_HIP(hipStreamSynchronize(st->stream));
-    if (rc) return rc;
-    tstep[0] = st->pinned[0];
-    return take_device_errors(st);
+    rc = take_device_errors(st, true);
+    if (rc != ERROR_CUDA_BLEW_UP) tstep[0] = st->pinned[0];
+    return rc;
 }
 
 int computeLocalCFLTimestep(MGArray *fluid, MGArray *csound, GeometryParams *geom, int method,

@@ -59,8 +59,9 @@ DeviceState *state();
 int pinned_buffers(DeviceState *st);
 // Waits for the stream, reads the device error counters and, when any is
 // set, clears them and returns ERROR_CRASH naming what was counted. Never
-// call it while the stream is being captured.
-int take_device_errors(DeviceState *st);
+// call it while the stream is being captured. reported: the last launch on the
+// stream has left the counters in errHost.
+int take_device_errors(DeviceState *st, bool reported = false);
 
 // Optional per-kernel timing with HIP events on the launch stream
 // (imogen_profile_enable / imogen_profile_read). prof_begin returns a slot
@@ -177,8 +178,7 @@ int launch_static_fade(double *phi, const double *table, int nspec, int64_t blk,
 int launch_soundspeed(const double *base, int64_t pitch, int64_t n, double gamma, double *cs,
                       hipStream_t s);
 int launch_cfl(const double *base, int64_t pitch, int64_t n, const double *cs, double gamma, int fused,
-               int dim, int xinjin, int halve, double hx, double hy, double hz, double hmin, double *devOut,
-               hipStream_t s);
+               int dim, int xinjin, int halve, double hx, double hy, double hz, double hmin, hipStream_t s);
 // The first of launch_cfl's two passes: nblocks (at most kCflBlocks) minima
 // that are still to be reduced and halved.
 constexpr int kCflBlocks = 2048;
