@@ -285,7 +285,7 @@ __global__ __launch_bounds__(256, 2) void ens_sweep_x(const EnsProblem *__restri
         for (int k = 0; k < K; k++)
             Q[k] = (k < cnt) ? load_cell<Hllc, 1>(A.src + off + k, P.pitch) : V5{1.0, 1.0, 0.0, 0.0, 0.0};
         const int first = sub * nl;
-        x_stages<Hllc, K, LIM>(P.hc, rt, Q, cnt, used ? first + (j == 0 ? nl - 1 : j - 1) : lane,
+        x_stages<Hllc, K, LIM, false>(P.hc, rt, Q, cnt, used ? first + (j == 0 ? nl - 1 : j - 1) : lane,
                                used ? first + (j == nl - 1 ? 0 : j + 1) : lane, lambda);
 #pragma unroll
         for (int k = 0; k < K; k++) {

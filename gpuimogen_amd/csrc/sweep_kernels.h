@@ -22,6 +22,37 @@ __device__ __forceinline__ V5 shfl5(const V5 &v, int src)
               shfl_d(v.e, src)};
 }
 
+// v of the lane before (after) in the wave, the first (last) lane's from the
+// other end: one VALU move per word where a shuffle goes through the LDS unit
+// and its address holds registers (sweep_x of 4 cells per lane 226 -> 156; X at
+// 256^3 308 -> 302 us, 1024^2 34.2 -> 32.4).
+template <int CTRL>
+__device__ __forceinline__ double rot_d(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xf, 0xf, false);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+template <int CTRL>
+__device__ __forceinline__ V5 rot5(const V5 &v)
+{
+    return V5{rot_d<CTRL>(v.a), rot_d<CTRL>(v.b), rot_d<CTRL>(v.c), rot_d<CTRL>(v.d), rot_d<CTRL>(v.e)};
+}
+
+// The neighbour lanes' values: ROT: the lines or windows fill the wave, so they
+// are those of the adjacent lanes; otherwise lane src's.
+template <bool ROT>
+__device__ __forceinline__ V5 left5(const V5 &v, int src)
+{
+    return ROT ? rot5<0x13c>(v) : shfl5(v, src);  // wave_ror:1
+}
+template <bool ROT>
+__device__ __forceinline__ V5 right5(const V5 &v, int src)
+{
+    return ROT ? rot5<0x134>(v) : shfl5(v, src);  // wave_rol:1
+}
+
 __device__ __forceinline__ V5 sel5(bool c, const V5 &x, const V5 &y)
 {
     return c ? x : y;
@@ -183,7 +214,7 @@ __device__ __forceinline__ void fill_ghosts(V5 (&Q)[K], int w0, int lbase, int w
 // Interface fluxes of the cells a lane owns. F[k] is the flux at k+1/2 for
 // k < cnt; Fm is the flux at -1/2 (the left lane's last interface). The
 // method's floors are applied to U in place first.
-template <class M, int K, int LIM, int DIR>
+template <class M, int K, int LIM, int DIR, bool ROT>
 __device__ __forceinline__ void x_fluxes(const HydroConsts &hc, int rt, V5 (&U)[K], int cnt, int srcL,
                                          int srcR, V5 (&F)[K], V5 &Fm)
 {
@@ -197,8 +228,8 @@ __device__ __forceinline__ void x_fluxes(const HydroConsts &hc, int rt, V5 (&U)[
     V5 wlast = w[0];
 #pragma unroll
     for (int k = 1; k < K; k++) wlast = sel5(k == cnt - 1, w[k], wlast);
-    const V5 wl = shfl5(wlast, srcL);
-    const V5 wr = shfl5(w[0], srcR);
+    const V5 wl = left5<ROT>(wlast, srcL);
+    const V5 wr = right5<ROT>(w[0], srcR);
 
     // backward differences d[k] = w[k] - w[k-1]; d[cnt] uses the right neighbour
     V5 d[K + 1];
@@ -211,7 +242,7 @@ __device__ __forceinline__ void x_fluxes(const HydroConsts &hc, int rt, V5 (&U)[
 #pragma unroll
     for (int k = 0; k < K; k++) M::template face<LIM>(hc, w[k], d[k], d[k + 1], rt, Lf[k], Rf[k]);
 
-    const V5 LfR = shfl5(Lf[0], srcR);
+    const V5 LfR = right5<ROT>(Lf[0], srcR);
 #pragma unroll
     for (int k = 0; k < K; k++) {
         const V5 right = (k + 1 < K) ? sel5(k + 1 < cnt, Lf[(k + 1 < K) ? k + 1 : 0], LfR) : LfR;
@@ -222,24 +253,24 @@ __device__ __forceinline__ void x_fluxes(const HydroConsts &hc, int rt, V5 (&U)[
     V5 Flast = F[0];
 #pragma unroll
     for (int k = 1; k < K; k++) Flast = sel5(k == cnt - 1, F[k], Flast);
-    Fm = shfl5(Flast, srcL);
+    Fm = left5<ROT>(Flast, srcL);
 }
 
 // Both stages of the cells a lane owns, Q in, the new state out (in Q).
-template <class M, int K, int LIM, int DIR = 1>
+template <class M, int K, int LIM, bool ROT, int DIR = 1>
 __device__ __forceinline__ void x_stages(const HydroConsts &hc, int rt, V5 (&Q)[K], int cnt, int srcL, int srcR,
                                          double lambda)
 {
     const double ml = -lambda, mhl = -.5 * lambda;
     V5 F[K], Fm, U1[K];
-    x_fluxes<M, K, LIM, DIR>(hc, rt, Q, cnt, srcL, srcR, F, Fm);
+    x_fluxes<M, K, LIM, DIR, ROT>(hc, rt, Q, cnt, srcL, srcR, F, Fm);
 #pragma unroll
     for (int k = 0; k < K; k++) {
         const V5 dF = F[k] - (k == 0 ? Fm : F[k > 0 ? k - 1 : 0]);
         U1[k] = axpy5(Q[k], ml, dF);
         if (!M::floors) Q[k] = half_sum<M>(Q[k], U1[k], dF, mhl);
     }
-    x_fluxes<M, K, LIM, DIR>(hc, rt, U1, cnt, srcL, srcR, F, Fm);
+    x_fluxes<M, K, LIM, DIR, ROT>(hc, rt, U1, cnt, srcL, srcR, F, Fm);
 #pragma unroll
     for (int k = 0; k < K; k++) {
         const V5 dF = F[k] - (k == 0 ? Fm : F[k > 0 ? k - 1 : 0]);
@@ -280,7 +311,7 @@ __global__ __launch_bounds__(256, (K <= 4) ? 2 : 1) void sweep_x(const double *s
     V5 Q[K];
 #pragma unroll
     for (int k = 0; k < K; k++) Q[k] = (k < cnt) ? load_cell<M, 1>(src + off + k, pitch) : V5{1.0, 1.0, 0.0, 0.0, 0.0};
-    x_stages<M, K, LIM>(hc, rt, Q, cnt, srcL, srcR, lambda);
+    x_stages<M, K, LIM, (FULL && K > 1)>(hc, rt, Q, cnt, srcL, srcR, lambda);
     fill_ghosts<K>(Q, laneUsed ? x0 : lane, laneUsed ? lbase : 0, kGhost, N - 1 - kGhost,
                    FULL ? (5 * K - 1 - kGhost) % K : (N - 1 - kGhost) % K, gf);
     double cmin = kCflNone;
@@ -329,7 +360,7 @@ __device__ __forceinline__ void xp_body(const double *src, double *dst, int64_t 
         Q[k] = (w0 < Wn) ? load_cell<M, 1>(src + g, pitch) : V5{1.0, 1.0, 0.0, 0.0, 0.0};
     }
     if (inplace) __syncthreads();
-    x_stages<M, K, LIM>(hc, rt, Q, K, (lane + 63) & 63, (lane + 1) & 63, lambda);
+    x_stages<M, K, LIM, true>(hc, rt, Q, K, (lane + 63) & 63, (lane + 1) & 63, lambda);
     // window cell 4 is the part's first
     if (K == 1)
         fill_ghosts<K>(Q, w0, 0, kGhost + 4, N - 1 - kGhost - s0 + 4, 0,
@@ -621,7 +652,7 @@ __global__ __launch_bounds__(1024) void sweep_tile(const double *src, double *ds
     const bool own = laneUsed && c < kTileCols && col0 + c < columns;
     double *cell = tile + (own ? j * kLd + c : 0);
     V5 Q[1] = {own ? load_cell<M, DIR>(cell, kSlab) : V5{1.0, 1.0, 0.0, 0.0, 0.0}};
-    x_stages<M, 1, LIM, DIR>(hc, rt, Q, 1, srcL, srcR, lambda);
+    x_stages<M, 1, LIM, false, DIR>(hc, rt, Q, 1, srcL, srcR, lambda);
     double cmin = kCflNone;
     if (own) {
         store_cell<M, DIR>(cell, kSlab, Q[0]);
