@@ -198,7 +198,7 @@ def run_ensemble(args):
     sweep direction and K class over all problems, each iteration a replayed
     hipGraph. First the hydrodynamics alone, then with dust on the odd problems
     (dust-to-gas 0.5) coupled by the learned drag with exact fallback, both
-    from the same initial states. The march segment counts are autotuned on the
+    from the same initial states. Factors on the march segment counts are tuned on the
     ensemble itself. cell_updates_per_s counts the problems' cells (2 per cell
     per iteration); sweep_hbm_frac is the sweeps' algorithmic bytes (80 B per
     cell and sweep, 4 sweeps per iteration, gas and dust) over the whole
