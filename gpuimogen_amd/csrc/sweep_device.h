@@ -131,10 +131,10 @@ __device__ __forceinline__ double flux_minmod(double a, double b)
     return (fabs(a) > fabs(b)) ? b : a;
 }
 
-// The limited half slope is slope_scale<LIM> * slope_limit<LIM>(a, b).
-// Products of opposite signs are raised to 0 (v_max_f64) in place of a compare
-// and two selects on the result, so a NaN difference gives no slope, as the
-// reference's `r > 0` does.
+// The limited half slope is slope_scale<LIM> * slope_limit<LIM>(a, b). Ospre and
+// van Leer select on a b > 0, as the reference does: a NaN difference gives no
+// slope, so a bad cell spoils its own faces and fluxes and not its neighbours'
+// other faces. (Raising the product to 0 instead left a + b NaN.)
 template <int LIM>
 __device__ __forceinline__ double slope_limit(double a, double b, int rt)
 {
@@ -145,17 +145,15 @@ __device__ __forceinline__ double slope_limit(double a, double b, int rt)
         // |A|, |B| < 1.5e-154, where the numerator has already underflowed to
         // zero and the quotient is +-0; the hardware reciprocal of such a
         // denominator is infinite, so it is raised to the smallest normal.
-        const double r = fmax(a * b, 0.0);
+        const double r = a * b;
         const double s = a + b;
-        return div_fast(((LIM >= 0) ? 1.0 : .75) * r * s, fmax(fma(s, s, -r), 0x1p-1022));
+        const double v = div_fast(((LIM >= 0) ? 1.0 : .75) * r * s, fmax(fma(s, s, -r), 0x1p-1022));
+        return (r > 0) ? v : 0.0;
     }
     case 1: {  // van Leer: A B / (A+B)
-        // A+B = 0 only with A B <= 0: 0 times the infinite reciprocal is NaN,
-        // which the minimum (a number against NaN) turns into |A+B| = 0; it
-        // leaves every other value, at most |A+B|/4 in size, as it is
-        const double r = fmax(a * b, 0.0);
-        const double s = a + b;
-        return fmin(div_fast(r, s), fabs(s));
+        const double r = a * b;
+        const double v = div_fast(r, a + b);
+        return (r > 0) ? v : 0.0;
     }
     case 2: {  // minmod, returned through float as the reference does (:70)
         if (a * b < 0) return 0.0;
