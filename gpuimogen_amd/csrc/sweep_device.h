@@ -116,14 +116,6 @@ __device__ __forceinline__ double sqrt_fast_pos(double x)
     return fma(g, r, g);
 }
 
-// 1/sqrt(|x|) to full precision (third-order step: error ~ e^3)
-__device__ __forceinline__ double rsqrt_abs(double x)
-{
-    const double y = __builtin_amdgcn_rsq(fabs(x));
-    const double e = fma(-(fabs(x) * y), y, 1.0);
-    return fma(y * e, fma(e, 0.375, 0.5), y);
-}
-
 // ---- half-slope limiters (limiter_functions.h) ----------------------------
 __device__ __forceinline__ double flux_minmod(double a, double b)
 {
@@ -230,30 +222,23 @@ __device__ __forceinline__ void faces(const HydroConsts &k, const V5 &w, const V
 }
 
 // Roe weights and sound speeds of an interface from its face densities and
-// pressures. One reciprocal root y = |rhoL rhoR|^-1/2 gives both densities'
-// reciprocals (+-y^2 rhoR, +-y^2 rhoL) and sqrt(rhoR / rhoL) = y |rhoR|, the
-// last only where the densities have one sign (`roe`: the reference's root is
-// NaN otherwise, and the bounds formed of it lose every comparison). SHARED
-// false: a reciprocal per side, for the limiters among which van Albada makes
-// NaN slopes of constant states: a NaN of one side must not reach the other
-// side's sound speed there.
+// pressures. A reciprocal per side: one reciprocal root of the product of the
+// densities would give both with fewer instructions, but a NaN of one side then
+// reaches the other side's sound speed (and the plain flux of a side whose
+// waves all leave the bad cell), and the product leaves the double range for
+// densities below 1.5e-154 or above 1.3e154.
 struct RoeTerms {
     double csql, csqr;  // gamma P / rho
     double Fa, Fb;      // sqrt(rhoR / rhoL), 1 / (1 + Fa)
-    bool roe;
 };
-template <bool SHARED>
 __device__ __forceinline__ RoeTerms roe_terms(const HydroConsts &k, double rl, double rr, double Pl, double Pr)
 {
-    const double d = rl * rr;
-    const double y = rsqrt_abs(d);
-    const double p = copysign(y * y, d);
+    const double il = rcp_fast(rl);
     RoeTerms t;
-    t.csql = fma(k.gamma * Pl, SHARED ? p * rr : rcp_fast(rl), kTinySq);
-    t.csqr = fma(k.gamma * Pr, SHARED ? p * rl : rcp_fast(rr), kTinySq);
-    t.Fa = y * fabs(rr);
+    t.csql = fma(k.gamma * Pl, il, kTinySq);
+    t.csqr = fma(k.gamma * Pr, rcp_fast(rr), kTinySq);
+    t.Fa = sqrt_fast_pos(rr * il);  // NaN where the densities differ in sign, as the reference's
     t.Fb = rcp_fast(1.0 + t.Fa);
-    t.roe = d > 0;
     return t;
 }
 
@@ -268,8 +253,8 @@ __device__ __forceinline__ void einfeldt(const HydroConsts &k, const RoeTerms &t
     const double C = sqrt_fast_pos(fma(x, t.Fb, kTinySq));
     sl = vl - sqrt_fast_pos(t.csql);
     sr = vr + sqrt_fast_pos(t.csqr);
-    sl = (t.roe & (Vroe - C < sl)) ? Vroe - C : sl;
-    sr = (t.roe & (Vroe + C > sr)) ? Vroe + C : sr;
+    sl = (Vroe - C < sl) ? Vroe - C : sl;
+    sr = (Vroe + C > sr) ? Vroe + C : sr;
 }
 
 // HLLC flux through the interface between face state L (right face of cell i)
@@ -281,14 +266,13 @@ __device__ __forceinline__ void einfeldt(const HydroConsts &k, const RoeTerms &t
 // rho beta by rho, so two selects choose between them. With mass flux m the
 // energy flux is m (c^2/(gamma-1) + |v|^2/2 + S_K (S_M - v)) and the
 // tangential ones are v_t m.
-template <int LIM>
 __device__ __forceinline__ V5 hllc_flux(const HydroConsts &k, const V5 &L, const V5 &R)
 {
     // velocity jump squared (cudaFluidStep.cu:1318-1322)
     const double C = L.c - R.c;
     const double D = L.d - R.d;
     const double E = L.e - R.e;
-    const RoeTerms t = roe_terms<(LIM >= 0)>(k, L.a, R.a, L.b, R.b);
+    const RoeTerms t = roe_terms(k, L.a, R.a, L.b, R.b);
     double sl, sr;
     einfeldt(k, t, L.c, R.c, fma(E, E, fma(D, D, C * C)), sl, sr);
 
@@ -353,10 +337,9 @@ struct Hllc {
     {
         faces<LIM>(k, w, dl, dr, rt, L, R);
     }
-    template <int LIM>
     __device__ static __forceinline__ V5 flux(const HydroConsts &k, const V5 &L, const V5 &R)
     {
-        return hllc_flux<LIM>(k, L, R);
+        return hllc_flux(k, L, R);
     }
 };
 
@@ -408,11 +391,10 @@ struct Hll {
         face_pair<LIM>(w.e, dl.e, dr.e, rt, L.e, R.e);
     }
     // L, R = (rho, vN, P, vT1, vT2), the reference's A..E (cudaFluidStep.cu:2124-2196)
-    template <int LIM>
     __device__ static __forceinline__ V5 flux(const HydroConsts &k, const V5 &L, const V5 &R)
     {
         const double Ut = R.b - L.b, St1 = R.d - L.d, St2 = R.e - L.e;
-        const RoeTerms t = roe_terms<(LIM >= 0)>(k, L.a, R.a, L.c, R.c);
+        const RoeTerms t = roe_terms(k, L.a, R.a, L.c, R.c);
         double sl, sr;
         if (k.ciso == -1) {
             einfeldt(k, t, L.b, R.b, fma(St2, St2, fma(St1, St1, Ut * Ut)), sl, sr);

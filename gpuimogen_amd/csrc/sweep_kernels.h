@@ -246,7 +246,7 @@ __device__ __forceinline__ void x_fluxes(const HydroConsts &hc, int rt, V5 (&U)[
 #pragma unroll
     for (int k = 0; k < K; k++) {
         const V5 right = (k + 1 < K) ? sel5(k + 1 < cnt, Lf[(k + 1 < K) ? k + 1 : 0], LfR) : LfR;
-        F[k] = M::template flux<LIM>(hc, Rf[k], right);
+        F[k] = M::flux(hc, Rf[k], right);
         // keep the cells' fluxes apart: interleaved they spill at 4 cells per lane
         if (K >= 4) __builtin_amdgcn_sched_barrier(0);
     }
@@ -453,7 +453,7 @@ __device__ __forceinline__ void march_body(const double *col, double *out, int64
         dn = wn - wp;
         V5 Lc;
         M::template face<LIM>(hc, wp, dp, dn, rt, Lc, Rn);  // faces of cell m-1
-        FAn = M::template flux<LIM>(hc, Rp, Lc);                           // interface (m-2)+1/2
+        FAn = M::flux(hc, Rp, Lc);                           // interface (m-2)+1/2
         const V5 dA = FAn - FAp;
         U1n = axpy5(Qs, ml, dA);
         en = M::template floor<DIR>(hc, U1n);
@@ -473,7 +473,7 @@ __device__ __forceinline__ void march_body(const double *col, double *out, int64
         d1n = w1n - w1p;
         V5 L1c;
         M::template face<LIM>(hc, w1p, d1p, d1n, rt, L1c, R1n);  // faces of cell m-4
-        FBn = M::template flux<LIM>(hc, R1p, L1c);                              // interface (m-5)+1/2
+        FBn = M::flux(hc, R1p, L1c);                              // interface (m-5)+1/2
         const double *r = &ring[(t + 1) & 3][0][lane];  // slot of step t-3
         const V5 S5{r[0], r[64], r[128], r[192], r[256]};
         const V5 o = axpy5(S5, mhl, FBn - FBp);  // cell m-5

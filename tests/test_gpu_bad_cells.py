@@ -56,3 +56,37 @@ def test_nan_cell_spreads_as_in_the_reference(direction, nx, ny, nz, method, lim
     got, ref = sweep_with_bad_cells(q, direction, method, limiter)
     assert np.isnan(ref).any() and np.isfinite(ref).any()
     compare(got, ref, what)
+
+
+@pytest.mark.parametrize("flow", [4.0, -4.0])
+@pytest.mark.parametrize("limiter", sorted(LIMITERS))
+@pytest.mark.parametrize("method", sorted(METHODS))
+@pytest.mark.parametrize("direction,nx,ny,nz", SWEEPS)
+def test_nan_cell_in_supersonic_flow(direction, nx, ny, nz, method, limiter, flow):
+    # where every wave of the good side leaves the bad cell, the interface's flux
+    # is that side's own: the bad side must not reach its sound speed
+    what = f"flow {flow}, sweep {direction} of {nx} x {ny} x {nz}, method {method}, limiter {limiter}"
+    print(what, flush=True)
+    q = state((nz, ny, nx), nx + ny + nz)
+    ke = 0.5 * (q[2:] ** 2).sum(0) / q[0]
+    q[2:] *= 0.3
+    q[1 + direction] += flow * q[0]
+    q[1] += 0.5 * (q[2:] ** 2).sum(0) / q[0] - ke
+    got, ref = sweep_with_bad_cells(q, direction, method, limiter)
+    compare(got, ref, what)
+
+
+@pytest.mark.parametrize("limiter", sorted(LIMITERS))
+@pytest.mark.parametrize("method", sorted(METHODS))
+@pytest.mark.parametrize("direction,nx,ny,nz", SWEEPS)
+def test_densities_whose_product_underflows(direction, nx, ny, nz, method, limiter):
+    # products of two densities underflow in these units; momenta and pressures,
+    # whose squares the formulas take, stay in the double range
+    rho, v = 1e-160, 1e10
+    what = f"density {rho}, sweep {direction} of {nx} x {ny} x {nz}, method {method}, limiter {limiter}"
+    print(what, flush=True)
+    q = state((nz, ny, nx), nx + ny + nz)
+    q *= np.array([rho, rho * v * v, rho * v, rho * v, rho * v]).reshape(5, 1, 1, 1)
+    got, ref = sweep_with_bad_cells(q, direction, method, limiter, bad=False, dt=0.001 / v, rhomin=1e-8 * rho)
+    assert np.isfinite(ref).all()
+    compare(got, ref, what)
