@@ -291,8 +291,9 @@ __device__ __forceinline__ DragRate drag_k_parts(const DragConsts &c, const Drag
 {
     DragRate r;
     r.lT = log_fast(c.alpha * u);
-    r.lRe = pre.ls + log_fast(magdv) + scaled_log(c.viscpow, r.lT);
-    r.Re = exp_fast(r.lRe);
+    const double lTv = scaled_log(c.viscpow, r.lT);
+    r.lRe = pre.ls + log_fast(magdv) + lTv;
+    r.Re = pre.dr * magdv * exp_fast(lTv);
     r.Kn = pre.brg * exp_fast(scaled_log(c.lampow, r.lT));
     const double E = cunningham_exp(r.Kn);
     const double cunningham = 1 + r.Kn * (1.142 + 0.558 * E);
@@ -343,7 +344,7 @@ __device__ __forceinline__ void learned_step(const DragConsts &c, const DragCell
     const bool defined = drag_cell_defined(s.rg, s.rd, s.s0, s.u0);
     const bool moving = defined && s.s0 >= 1e-9;
     DragRate r0 = {0.0, 1.0, 1.0, 0.0};
-    DragPre pre = {0.0, 0.0, 0.0};
+    DragPre pre = {0.0, 0.0, 0.0, 0.0};
     if (moving) {
         pre = drag_pre(c, s.rg, s.rd);
         r0 = drag_k_parts(c, pre, s.rg, s.rd, s.s0, s.u0);
