@@ -166,12 +166,28 @@ __device__ __forceinline__ double drag_rate(const DragConsts &c, const DragPre &
     return div_cr(N * s * pre.C, cunningham);
 }
 
+// drag_rate where T = alpha u may be 0 or infinite (a gas without internal
+// energy: its cells are reported, and updated as the formula falls). log_fast
+// has no such limit, so the powers take theirs here: T^a is 0, 1 or infinite.
+// The adaptive integrator refuses such cells and needs no look.
+__device__ __forceinline__ double drag_rate_any(const DragConsts &c, const DragPre &pre, double s, double ls1, double u)
+{
+    const double T = c.alpha * u, inf = __builtin_inf();
+    if (!(T == 0.0 || T == inf)) return drag_rate(c, pre, s, ls1, u);
+    auto power = [&](double a) { return a == 0.0 ? 1.0 : ((a > 0) == (T == 0.0) ? 0.0 : inf); };
+    const double Re = pre.dr * s * power(c.viscpow);
+    const double Kn = pre.brg * power(c.lampow);
+    const double cunningham = 1 + Kn * (1.142 + 0.558 * exp_decay(-0.999 / Kn));
+    const double E = Re > 0 ? exp_fast(-.319 * log_fast(Re)) : inf;
+    return (3 / Re + .45 * E + .0509 * Re / (8710 + Re)) / cunningham * s * pre.C;
+}
+
 // drag rate k(|dv|, u); no drag below |dv| = 1e-9 (:853-859)
 __device__ __forceinline__ double drag_k(const DragConsts &c, double rhog, double rhod, double magdv, double u)
 {
     if (magdv < 1e-9) return 0.0;
     const DragPre pre = drag_pre(c, rhog, rhod);
-    return drag_rate(c, pre, magdv, pre.ls + log_fast(magdv), u);
+    return drag_rate_any(c, pre, magdv, pre.ls + log_fast(magdv), u);
 }
 
 // |dv| and u_0 of a cell (cukern_prepareForERK_h0, :1883-1908)
@@ -256,9 +272,9 @@ __device__ __forceinline__ double drag_logtrap_rate(const DragConsts &c, double 
         double em1;
         const double e = exp_fast(-t * a, em1);
         const double s = dv0 * e;
-        return s < 1e-9 ? 0.0 : drag_rate(c, pre, s, l0 - t * a, u0 + heat * (em1 * (1.0 + e)));
+        return s < 1e-9 ? 0.0 : drag_rate_any(c, pre, s, l0 - t * a, u0 + heat * (em1 * (1.0 + e)));
     };
-    const double k0 = dv0 < 1e-9 ? 0.0 : drag_rate(c, pre, dv0, l0, u0);
+    const double k0 = dv0 < 1e-9 ? 0.0 : drag_rate_any(c, pre, dv0, l0, u0);
     const double ksum = k0 + end_rate(k0);
     if (order == 3) return 0.16666666666666666667 * ksum + 0.66666666666666666667 * end_rate(.25 * ksum);
     return .5 * ksum;
@@ -363,7 +379,7 @@ __device__ __forceinline__ double drag_exact_ratio(const DragConsts &c, double r
 // core it has no small-|dv| cut-off
 __device__ __forceinline__ double drag_rk_accel(const DragConsts &c, const DragPre &pre, double magdv, double u)
 {
-    return -(drag_rate(c, pre, magdv, pre.ls + log_fast(magdv), u) * magdv);
+    return -(drag_rate_any(c, pre, magdv, pre.ls + log_fast(magdv), u) * magdv);
 }
 
 // |dv| after dt; the stage and accumulator updates of cukern_SolveRK_single /
