@@ -107,7 +107,13 @@ struct XGeom {
 // at most 64 K - 8 cells. Measured (HLLC, van Leer, smooth states, us):
 //  * Lines that fill their lanes (64, 128, 192, 256 cells) stay whole (16384 of
 //    128: 49, K=1 parts 64; 65536 of 256: 347, K=3 parts 477), as do lines of
-//    384 (36864: 341, K=4 parts 375) and of less than 64.
+//    less than 64.
+//  * So do many lines of 384 where six cells a lane stay in registers (`wide`:
+//    HLLC with Ospre or van Leer; 36864 lines: 341, K=4 parts 375). HLL and the
+//    limiters chosen at run time hold more per cell: whole steps of 384 x 384 x
+//    96 cells with whole lines 1307 and 1354, with K=4 parts 1155 and 1129.
+//    Fewer lines go the way of their neighbours (steps of 384 x 200 cells: HLLC
+//    23.1, K=1 parts 17.1; HLL 27.7, 17.7).
 //  * Others of up to 256 cells: K=1 parts, whose lanes need no select at a
 //    line's end and leave room for four waves per SIMD (13560 of 131: 54,
 //    whole 68; 20000 of 150: 77, 92), while the last-level cache holds the
@@ -116,10 +122,13 @@ struct XGeom {
 //  * Longer ones: K=3 (28700 of 321: 250, K=2 263, K=1 283; 1024 of 1024: 34,
 //    K=4 46, whole lines of 16 cells per lane, whose arrays left the
 //    registers, 130), but K=4 where two parts of it replace three (369..496).
+//    Many lines of 497..552 are three parts of K=3 (whole HLLC steps of N x 512 x
+//    64 cells, in place with whole lines of 8 or 9 cells per lane -> as here: 497
+//    1334 -> 1195, 512 1276 -> 1202, 530 2770 -> 1300, 552 2810 -> 1338).
 //  * Too few lines to fill the 1024 SIMDs: smaller K for a shorter chain per
 //    wave (17 lines of 300: K=1 5.3, K=2 5.7, K=3 6.6; 400 x 400: K=1 8.8,
 //    K=2 8.9, K=3 10.8), as far as 8 waves reach.
-static XGeom x_geom(int N, int64_t nlines)
+static XGeom x_geom(int N, int64_t nlines, bool wide)
 {
     XGeom g;
     if (N > 1024) return g;
@@ -127,8 +136,8 @@ static XGeom x_geom(int N, int64_t nlines)
     if (N > 64 && N <= 256) {
         const bool cached = (int64_t)N * nlines * 5 * (int64_t)sizeof(double) <= (int64_t)256 << 20;
         if ((N % 64 != 0 && cached) || nlines * parts(1) <= 1024) g.K = 1;
-    } else if (N > 256 && N != 384) {
-        if (nlines * parts(3) >= 1536) g.K = (N > 368 && N <= 496) ? 4 : 3;
+    } else if (N > 256) {
+        if (nlines * parts(3) >= 1536) g.K = (N == 384 && wide) ? 0 : ((N > 368 && N <= 496) ? 4 : 3);
         else g.K = parts(1) <= 8 ? 1 : (parts(2) <= 8 ? 2 : 3);
     }
     if (g.K) {
@@ -186,7 +195,8 @@ static int launch_x(const double *src, double *dst, int64_t pitch, int N, int64_
                     const double *lamp, const HydroConsts &hc, int rt, const CflFuse &cf, GhostFill gf,
                     bool *filled, hipStream_t s)
 {
-    const XGeom g = x_geom(N, nlines);
+    constexpr bool wide = !M::floors && LIM >= 0;
+    const XGeom g = x_geom(N, nlines, wide);
     if (g.K == 0) return IM_FAIL(ERROR_NOIMPLEMENT, "X sweep supports lines of at most 1024 cells (got %d)", N);
     const int K = g.K, nl = g.nl;
     if (g.blocks > INT32_MAX) return IM_FAIL(ERROR_INVALID_ARGS, "too many lines for one X launch");
@@ -228,8 +238,10 @@ static int launch_x(const double *src, double *dst, int64_t pitch, int N, int64_
         IM_X_CASE(3)
         IM_X_CASE(4)
     case 6:  // 384 cells: every lane full
-        if (cf.slots) IM_X(6, true, true);
-        else IM_X(6, true, false);
+        if constexpr (wide) {
+            if (cf.slots) IM_X(6, true, true);
+            else IM_X(6, true, false);
+        }
         break;
     }
 #undef IM_X_CASE
