@@ -44,6 +44,7 @@ struct DeviceState {
     hipStream_t stream = nullptr;
     void *scratch = nullptr;
     size_t scratchBytes = 0;
+    size_t scratchRefused = SIZE_MAX;  // least size scratch_available could not get (until GPU_ctrl_reset)
     double *fixedScratch = nullptr;  // this device's copy of the fixed scratch array (kFixedScratchBytes)
     int fixedScratchOn = 0;          // scratch_block hands out fixedScratch (never allocates) while set
     double *pinned = nullptr;   // 64 doubles of pinned host memory (pinned_buffers)
@@ -78,8 +79,9 @@ void prof_suspend(int on);
 // allocates.
 void *scratch_block(size_t bytes);
 // Whether scratch_block(bytes) will succeed, for callers that can do with
-// less: the block is grown to that size unless it would take more than half of
-// the free device memory.
+// less: the block is grown to that size unless the stream is being captured or
+// it would take more than half of the free device memory. Where the device has
+// none to give, the old block stays, and that size is refused from then on.
 bool scratch_available(size_t bytes);
 // Scratch bytes launch_fluid_sweep / launch_xinjin_sweep take for one sweep
 // (the launch shapes of fluid_sweep.hip and xinjin.hip).

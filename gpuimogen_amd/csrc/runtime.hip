@@ -108,12 +108,32 @@ int take_device_errors(DeviceState *st, bool reported)
                    c0, c1, c2, c3);
 }
 
+// The scratch block as it is allocated: a quarter above what is asked for.
+static size_t scratch_size(size_t bytes)
+{
+    return bytes + bytes / 4;
+}
+
+// Puts a larger block in the scratch block's place once the stream is done with
+// the old one.
+static int replace_scratch(DeviceState *st, void *block, size_t size)
+{
+    if (st->scratch && (IM_HIP(hipStreamSynchronize(st->stream)) || IM_HIP(hipFree(st->scratch)))) {
+        (void)hipFree(block);
+        return ERROR_CUDA_BLEW_UP;
+    }
+    st->scratch = block;
+    st->scratchBytes = size;
+    return SUCCESSFUL;
+}
+
 bool scratch_available(size_t bytes)
 {
     DeviceState *st = state();
     if (!st) return false;
     if (st->fixedScratchOn) return bytes <= kFixedScratchBytes;
     if (bytes <= st->scratchBytes) return true;
+    if (bytes >= st->scratchRefused) return false;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
         (void)hipGetLastError();
@@ -124,7 +144,17 @@ bool scratch_available(size_t bytes)
         (void)hipGetLastError();
         return false;
     }
-    return bytes + bytes / 4 <= freeB / 2 && scratch_block(bytes);
+    const size_t want = scratch_size(bytes);
+    if (want > freeB / 2) return false;
+    // beside the old block, which stays if this one cannot be had; a size the
+    // device has refused once is not asked for at every step
+    void *block = nullptr;
+    if (hipMalloc(&block, want) != hipSuccess) {
+        (void)hipGetLastError();
+        st->scratchRefused = bytes;
+        return false;
+    }
+    return replace_scratch(st, block, want) == SUCCESSFUL;
 }
 
 void *scratch_block(size_t bytes)
@@ -144,8 +174,11 @@ void *scratch_block(size_t bytes)
         st->scratch = nullptr;
         st->scratchBytes = 0;
     }
-    size_t want = bytes + bytes / 4;
-    if (IM_HIP(hipMalloc(&st->scratch, want))) return nullptr;
+    const size_t want = scratch_size(bytes);
+    if (IM_HIP(hipMalloc(&st->scratch, want))) {
+        st->scratch = nullptr;
+        return nullptr;
+    }
     st->scratchBytes = want;
     return st->scratch;
 }
@@ -683,6 +716,7 @@ int GPU_ctrl_reset(void)
         st->scratch = nullptr;
         st->scratchBytes = 0;
     }
+    st->scratchRefused = SIZE_MAX;
     return rc;
 }
 

@@ -246,7 +246,12 @@ int GPU_ctrl_info(int device, char *text, int len);
 /* gpuclass/flux.h:17, flux.cu:27-155. fluid -> 5 MGArrays (rho E px py pz), the
  * slab views of one 5-slab owner. One `fluidstep`: 3 directional SSP-RK2 sweeps
  * in the order (stepNumber + 3*(stepDirection>0)) % 6, each followed by its
- * boundary conditions. tempStorage may be NULL (scratch is library-cached). */
+ * boundary conditions. tempStorage may be NULL: scratch is the library's, one
+ * block per GPU, kept until GPU_ctrl_reset or the end of the process. An HLLC or
+ * HLL step of a plane or a box takes a second copy of the state in it (40 bytes a
+ * cell, for states of up to 2 GiB) and a quarter more, where at least twice that
+ * is free when it is first asked for; otherwise, and for larger states, it works
+ * in place, with the same results. The device loop's steps do the same. */
 int performFluidUpdate_3D(MGArray *fluid, ParallelTopology *parallelTopo, FluidStepParams fsp,
                           MGArray *tempStorage);
 
@@ -431,7 +436,8 @@ int imogen_mlp_infer_bf16(int64_t batch, const float *x, float *y);
  * CFL time step on the device and applies fluidstep(+1), fluidstep(-1) with
  * batched sweeps, optionally replayed from HIP graphs. Problem p's state is
  * 5 x ny[p] x nx[p] doubles (rho, E, px, py, pz; x fastest), grid spacing
- * hx[p], hy[p]. */
+ * hx[p], hy[p]. Device memory: the states, and as much again for the sweeps, of
+ * which at most 1 GiB (or the largest problem's state, if that is more). */
 typedef struct ImogenEnsemble ImogenEnsemble;
 int imogen_ensemble_create(int nprob, const int *nx, const int *ny, const double *hx, const double *hy,
                            double gamma, int limiter, double cfl, ImogenEnsemble **out);
