@@ -509,34 +509,36 @@ static int segment_cells(const EnsembleImpl *e, const EnsGroup &g)
 
 // Groups of consecutive entries that fit the second pool; every entry's place
 // in it, and the size (doubles) it needs.
-static int64_t make_groups(EnsembleImpl *e)
+static int64_t make_groups(std::vector<EnsProblem> &host, double *pool2, std::vector<EnsGroup> &groups)
 {
-    e->groups.clear();
+    groups.clear();
     int64_t size = 0, at = 0;
-    for (int p = 0; p < e->NE; p++) {
-        const int64_t n = 5 * e->host[p].pitch;
-        if (e->groups.empty() || (at + n) * (int64_t)sizeof(double) > kSecondPool) {
+    for (int p = 0; p < (int)host.size(); p++) {
+        const int64_t n = 5 * host[p].pitch;
+        if (groups.empty() || (at + n) * (int64_t)sizeof(double) > kSecondPool) {
             EnsGroup g{};
             g.e0 = p;
-            e->groups.push_back(g);
+            groups.push_back(g);
             at = 0;
         }
-        e->host[p].q2 = e->pool2 + at;  // rebased once the pool is there
+        host[p].q2 = pool2 + at;
         at += n;
         size = std::max(size, at);
-        e->groups.back().e1 = p + 1;
+        groups.back().e1 = p + 1;
     }
     return size;
 }
 
-// (Re)allocates the second pool for the present entries.
-static int second_pool(EnsembleImpl *e)
+// Allocates the second pool for the entries and gives them their places in it.
+static int second_pool(std::vector<EnsProblem> &host, double **pool2, std::vector<EnsGroup> &groups)
 {
-    if (e->pool2) (void)hipFree(e->pool2);
-    e->pool2 = nullptr;
-    const int64_t size = make_groups(e);
-    if (IM_HIP(hipMalloc(&e->pool2, (size_t)size * sizeof(double)))) return ERROR_CUDA_BLEW_UP;
-    (void)make_groups(e);
+    const int64_t size = make_groups(host, nullptr, groups);
+    *pool2 = nullptr;
+    if (IM_HIP(hipMalloc(pool2, (size_t)size * sizeof(double)))) {
+        *pool2 = nullptr;
+        return ERROR_CUDA_BLEW_UP;
+    }
+    (void)make_groups(host, *pool2, groups);
     return SUCCESSFUL;
 }
 
@@ -786,7 +788,7 @@ int imogen_ensemble_create(int nprob, const int *nx, const int *ny, const double
     int rc = SUCCESSFUL;
     if (IM_HIP(hipMalloc(&e->pool, (size_t)total * sizeof(double)))) rc = ERROR_CUDA_BLEW_UP;
     for (int p = 0; p < nprob && !rc; p++) e->host[p].q = e->pool + off[p];
-    if (!rc) rc = second_pool(e);
+    if (!rc) rc = second_pool(e->host, &e->pool2, e->groups);
     if (!rc && IM_HIP(hipMalloc(&e->dprobs, nprob * sizeof(EnsProblem)))) rc = ERROR_CUDA_BLEW_UP;
     if (!rc && IM_HIP(hipMemcpy(e->dprobs, e->host.data(), nprob * sizeof(EnsProblem), hipMemcpyHostToDevice)))
         rc = ERROR_CUDA_BLEW_UP;
@@ -869,7 +871,8 @@ int imogen_ensemble_set_dust(ImogenEnsemble *E, const int *hasDust, double dustG
         }
     if (dusty.empty()) return SUCCESSFUL;
     const int NE = e->P + (int)dusty.size();
-    double *dpool = nullptr, *lam = nullptr, *part = nullptr;
+    double *dpool = nullptr, *pool2 = nullptr, *lam = nullptr, *part = nullptr;
+    std::vector<EnsGroup> groups;
     EnsProblem *dprobs = nullptr;
     EnsDragTable *tab = nullptr;
     EnsDragItem *items = nullptr;
@@ -894,6 +897,7 @@ int imogen_ensemble_set_dust(ImogenEnsemble *E, const int *hasDust, double dustG
         htab.push_back(EnsDragTable{host[p].q, D.q, D.pitch, n, p, 0});
         for (int64_t b = 0; b < n; b += 64) hitems.push_back(EnsDragItem{(int)k, 0, b});
     }
+    if (!rc) rc = second_pool(host, &pool2, groups);
     if (!rc) rc = IM_HIP(hipMalloc(&dprobs, NE * sizeof(EnsProblem)));
     if (!rc) rc = IM_HIP(hipMemcpy(dprobs, host.data(), NE * sizeof(EnsProblem), hipMemcpyHostToDevice));
     if (!rc) rc = IM_HIP(hipMalloc(&lam, 2 * NE * sizeof(double)));
@@ -905,15 +909,17 @@ int imogen_ensemble_set_dust(ImogenEnsemble *E, const int *hasDust, double dustG
     if (!rc) rc = IM_HIP(hipMalloc(&queue, (size_t)cells * 2 * sizeof(int64_t)));  // queue + second-call list
     if (!rc) rc = IM_HIP(hipMalloc(&qcount, 3 * sizeof(unsigned long long)));
     if (rc) {
-        void *bufs[] = {dpool, dprobs, lam, part, tab, items, queue, qcount};
+        void *bufs[] = {dpool, pool2, dprobs, lam, part, tab, items, queue, qcount};
         for (void *b : bufs)
             if (b) (void)hipFree(b);
         return ERROR_CUDA_BLEW_UP;
     }
-    void *old[] = {e->dprobs, e->lam, e->cflPart};
+    void *old[] = {e->pool2, e->dprobs, e->lam, e->cflPart};
     for (void *b : old)
         if (b) (void)hipFree(b);
     e->host = host;
+    e->pool2 = pool2;
+    e->groups = groups;
     e->NE = NE;
     e->Pd = (int)dusty.size();
     e->dpool = dpool;
@@ -929,8 +935,7 @@ int imogen_ensemble_set_dust(ImogenEnsemble *E, const int *hasDust, double dustG
     e->dc = drag_consts(gas, dust);
     e->dragMethod = dragMethod;
     e->modelGen = learned_model_generation();
-    rc = second_pool(e);
-    return rc ? rc : build_work(e);
+    return build_work(e);
 }
 
 static int dust_entry(EnsembleImpl *e, int p)
@@ -979,7 +984,6 @@ int imogen_ensemble_run(ImogenEnsemble *E, int firstIteration, int iterations, i
     }
     if (!E) return IM_FAIL(ERROR_NULL_POINTER, "null ensemble");
     EnsembleImpl *e = &E->impl;
-    if (!e->pool2) return IM_FAIL(ERROR_NOMEM, "the ensemble has no second pool (adding its dust failed)");
     DeviceState *st = state();
     if (!st) return ERROR_CUDA_BLEW_UP;
     for (int k = 0; k < iterations; k++) {
@@ -1023,7 +1027,6 @@ int imogen_ensemble_autotune(ImogenEnsemble *E, int trials, int *chosen)
 {
     if (!E) return IM_FAIL(ERROR_NULL_POINTER, "null ensemble");
     EnsembleImpl *e = &E->impl;
-    if (!e->pool2) return IM_FAIL(ERROR_NOMEM, "the ensemble has no second pool (adding its dust failed)");
     DeviceState *st = state();
     if (!st) return ERROR_CUDA_BLEW_UP;
     if (trials < 1) trials = 1;
