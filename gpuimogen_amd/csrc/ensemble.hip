@@ -264,7 +264,7 @@ __global__ __launch_bounds__(256, 2) void ens_sweep_x(const EnsProblem *__restri
     unsigned nan = 0;
     if (it.c) {
         const int64_t row = (int64_t)it.a * N;
-        xp_body<Hllc, K, LIM, CFL>(A.src + row, A.dst + row, P.pitch, N, it.b, it.c, true, false, lambda, P.hc, rt,
+        xp_body<Hllc, K, LIM, CFL>(A.src + row, A.dst + row, P.pitch, N, it.b, it.c, false, lambda, P.hc, rt,
                                    cf, GhostFill{}, cmin, nan);
     } else if (K <= 4) {
         const int lane = threadIdx.x & 63;

@@ -334,14 +334,14 @@ __global__ __launch_bounds__(256, (K <= 4) ? 2 : 1) void sweep_x(const double *s
 // so it forms its outputs alone; the window's outer cells only feed discarded
 // values. inplace: the waves of a line share a workgroup and every load of the
 // workgroup precedes the barrier while every store follows it, so no wave
-// overwrites a cell another has still to read. valid false: nothing is stored.
+// overwrites a cell another has still to read.
 // CFL: cmin takes the minimum CFL limit of the outputs at cells [cf.lo, cf.hi),
 // nanc counts the NaN limits. gf: K = 1 only (with K = 3 the parts of a mirrored
 // 321 x 287 x 305 box took 906 us instead of 793 and its launch of 42, and a
 // periodic 1024 x 1024 plane, which fills nothing, 40 us instead of 33).
 template <class M, int K, int LIM, bool CFL>
 __device__ __forceinline__ void xp_body(const double *src, double *dst, int64_t pitch, int N, int part, int parts,
-                                        bool valid, bool inplace, double lambda, const HydroConsts &hc, int rt,
+                                        bool inplace, double lambda, const HydroConsts &hc, int rt,
                                         const CflFuse &cf, const GhostFill &gf, double &cmin, unsigned &nanc)
 {
     const int lane = threadIdx.x & 63;
@@ -368,7 +368,7 @@ __device__ __forceinline__ void xp_body(const double *src, double *dst, int64_t 
 #pragma unroll
     for (int k = 0; k < K; k++) {
         const int w = w0 + k;
-        if (valid && w >= 4 && w < Wn - 4) {
+        if (w >= 4 && w < Wn - 4) {
             const int x = s0 + w - 4;
             const V5 &o = Q[k];
             store_cell<M, 1>(dst + x, pitch, o);
@@ -394,7 +394,7 @@ __global__ __launch_bounds__(512, 2) void sweep_xp(const double *src, double *ds
     const int64_t line = blockIdx.x;
     double cmin = kCflNone;
     unsigned nanc = 0;  // not reported by the single-array fold
-    xp_body<M, K, LIM, CFL>(src + line * (int64_t)N, dst + line * (int64_t)N, pitch, N, wib, parts, true, src == dst,
+    xp_body<M, K, LIM, CFL>(src + line * (int64_t)N, dst + line * (int64_t)N, pitch, N, wib, parts, src == dst,
                             lambda, hc, rt, cf, gf, cmin, nanc);
     if (CFL) cfl_fold(cf, (int64_t)blockIdx.x * (blockDim.x >> 6) + wib, cmin);
 }
