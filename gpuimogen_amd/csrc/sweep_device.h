@@ -116,6 +116,17 @@ __device__ __forceinline__ double sqrt_fast_pos(double x)
     return fma(g, r, g);
 }
 
+// sqrt(x), x > 0, as a product g t: a sum v +- g t is then one FMA
+struct Root {
+    double g, t;
+};
+__device__ __forceinline__ Root root_fast(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    const double g = x * y;
+    return Root{g, fma(.5, fma(-g, y, 1.0), 1.0)};
+}
+
 // ---- half-slope limiters (limiter_functions.h) ----------------------------
 __device__ __forceinline__ double flux_minmod(double a, double b)
 {
@@ -133,14 +144,14 @@ __device__ __forceinline__ double slope_limit(double a, double b, int rt)
     const int which = (LIM >= 0) ? LIM : rt;
     switch (which) {
     case 0: {  // Ospre: .75 A B (A+B) / (A^2 + AB + B^2)
-        // With A B > 0 the denominator falls below the normal range only for
-        // |A|, |B| < 1.5e-154, where the numerator has already underflowed to
-        // zero and the quotient is +-0; the hardware reciprocal of such a
-        // denominator is infinite, so it is raised to the smallest normal.
+        // Where A B is positive but below the normal range, the numerator
+        // underflows and the slope is 0 (the hardware reciprocal of so small a
+        // denominator would be infinite); otherwise the denominator is at least
+        // 3 A B, a normal.
         const double r = a * b;
         const double s = a + b;
-        const double v = div_fast(((LIM >= 0) ? 1.0 : .75) * r * s, fmax(fma(s, s, -r), 0x1p-1022));
-        return (r > 0) ? v : 0.0;
+        const double v = div_fast(((LIM >= 0) ? 1.0 : .75) * r * s, fma(s, s, -r));
+        return (r >= 0x1p-1022) ? v : 0.0;
     }
     case 1: {  // van Leer: A B / (A+B)
         const double r = a * b;
@@ -250,11 +261,12 @@ __device__ __forceinline__ void einfeldt(const HydroConsts &k, const RoeTerms &t
 {
     const double Vroe = fma(t.Fa, vr, vl) * t.Fb;
     const double x = fma(k.hgm1 * dvsq, t.Fa * t.Fb, fma(t.Fa, t.csqr, t.csql));
-    const double C = sqrt_fast_pos(fma(x, t.Fb, kTinySq));
-    sl = vl - sqrt_fast_pos(t.csql);
-    sr = vr + sqrt_fast_pos(t.csqr);
-    sl = (Vroe - C < sl) ? Vroe - C : sl;
-    sr = (Vroe + C > sr) ? Vroe + C : sr;
+    const Root C = root_fast(fma(x, t.Fb, kTinySq)), cl = root_fast(t.csql), cr = root_fast(t.csqr);
+    const double sroe = fma(-C.g, C.t, Vroe), rroe = fma(C.g, C.t, Vroe);
+    sl = fma(-cl.g, cl.t, vl);
+    sr = fma(cr.g, cr.t, vr);
+    sl = (sroe < sl) ? sroe : sl;
+    sr = (rroe > sr) ? rroe : sr;
 }
 
 // HLLC flux through the interface between face state L (right face of cell i)

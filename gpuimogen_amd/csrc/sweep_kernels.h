@@ -437,8 +437,8 @@ __device__ __forceinline__ void march_body(const double *col, double *out, int64
     V5 w1A = one, w1B = one, d1A = zero, d1B = zero, R1A = one, R1B = one, FBA = zero, FBB = zero;
 
     // Stage B runs one step behind stage A (it consumes the previous step's
-    // U1), so the two long dependency chains of a step are independent and
-    // interleave. (U1+Q)/2 of a cell is needed three steps after it is formed:
+    // U1), so the two long dependency chains of a step are independent.
+    // (U1+Q)/2 of a cell is needed three steps after it is formed:
     // it waits in a 4-slot ring in LDS, private to the lane.
 
     auto step = [&](int t, V5 &Qcur, V5 &Qs, const V5 &U1p, V5 &U1n, const double &ep, double &en,
@@ -468,7 +468,12 @@ __device__ __forceinline__ void march_body(const double *col, double *out, int64
         }
         Qs = Qcur;
 
-        // stage B at cell m-5, from the previous step's U1 (cell m-3)
+        // stage B at cell m-5, from the previous step's U1 (cell m-3). Its code
+        // stays behind stage A's: scheduled into one another the two hold more
+        // than two waves' registers (the ensembles' march spilled 16 of them:
+        // 60 problems of 64..512 cells 664 us an iteration, 604 so; 200^3 step
+        // with van Leer 580, 571).
+        __builtin_amdgcn_sched_barrier(0);
         w1n = M::template prims<LIM>(hc, U1p, ep);
         d1n = w1n - w1p;
         V5 L1c;
