@@ -437,7 +437,7 @@ int imogen_mlp_infer_bf16(int64_t batch, const float *x, float *y);
  * batched sweeps, optionally replayed from HIP graphs. Problem p's state is
  * 5 x ny[p] x nx[p] doubles (rho, E, px, py, pz; x fastest), grid spacing
  * hx[p], hy[p]. Device memory: the states, and as much again for the sweeps, of
- * which at most 1 GiB (or the largest problem's state, if that is more). */
+ * which at most 2 GiB (or the largest problem's state, if that is more). */
 typedef struct ImogenEnsemble ImogenEnsemble;
 int imogen_ensemble_create(int nprob, const int *nx, const int *ny, const double *hx, const double *hy,
                            double gamma, int limiter, double cfl, ImogenEnsemble **out);
