@@ -7,7 +7,8 @@
 // limiters (gpuclass/limiter_functions.h:50-117), Einfeldt speed bounds
 // (:1728-1799), the HLLC contact speed and four-way flux selection
 // (:1357-1431), the HLL flux (:2124-2196) and the HLL density/energy floors.
-// Divisions and square roots use refined hardware estimates (within 1-2 ulp).
+// Divisions and square roots use refined hardware estimates: 1-2 ulp for the
+// densities' reciprocals and HLL's quotients, 3e-15 and 5e-15 elsewhere.
 // The data movement around these functions (which lane owns which cell, how
 // neighbours are exchanged) is this library's own.
 #pragma once

@@ -24,8 +24,8 @@ __device__ __forceinline__ V5 shfl5(const V5 &v, int src)
 
 // v of the lane before (after) in the wave, the first (last) lane's from the
 // other end: one VALU move per word where a shuffle goes through the LDS unit
-// and its address holds registers (sweep_x of 4 cells per lane 226 -> 156; X at
-// 256^3 308 -> 302 us, 1024^2 34.2 -> 32.4).
+// and its address holds registers (sweep_x of 4 cells per lane 226 -> 156 by
+// this alone; X at 256^3 308 -> 302 us, 1024^2 34.2 -> 32.4).
 template <int CTRL>
 __device__ __forceinline__ double rot_d(double v)
 {
